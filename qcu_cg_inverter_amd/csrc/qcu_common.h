@@ -176,4 +176,50 @@ inline Walk make_walk(const Geom& g, int ty, int tz, int tt) {
   return w;
 }
 
+// Order in which a launch takes the 64-site storage chunks of a half lattice.  tt = 0:
+// storage order.  Otherwise the t-slices are taken tt at a time, t fastest: a chunk's t
+// neighbours are then one step away and its z neighbours tt planes, instead of a whole
+// t-slice.  Needs t-slices of whole chunks (slice chunks each) and tt dividing Lt.
+struct ChunkOrder {
+  unsigned n;  // chunks
+  int tt;
+  unsigned slice;
+  FastDiv dtt, dslice;
+  __host__ __device__ inline unsigned chunk(unsigned u) const {
+    if (tt == 0) return u;
+    const unsigned p = dtt.div(u), t_in = u - p * (unsigned)tt;
+    const unsigned tile = dslice.div(p);
+    return (tile * (unsigned)tt + t_in) * slice + (p - tile * slice);
+  }
+};
+inline ChunkOrder make_chunk_order(const Geom& g, int tt) {
+  ChunkOrder o;
+  o.n = (unsigned)((g.vh + 63) / 64);
+  o.tt = 0;
+  o.slice = 0;
+  if (tt > 1 && g.st % 64 == 0 && g.L[3] % tt == 0) {
+    o.tt = tt;
+    o.slice = (unsigned)(g.st / 64);
+    o.dtt = FastDiv((uint32_t)tt);
+    o.dslice = FastDiv(o.slice);
+  }
+  return o;
+}
+
+// One launch on the caller's interface fields (k_hop_split.inc): half spinors in[r] ->
+// out[r] of one parity, or, with parity -1, full spinors on both parities, where an
+// epilogue's x is the other half of `in` and the clover clov0 / clov1 by parity.
+struct IfaceArgs {
+  const void* gauge;
+  const void* clov0;
+  const void* clov1;
+  double tbc, coef;
+  int parity;
+  FastDiv drhs;       // by the number of right-hand sides
+  ChunkOrder order;
+  Geom geo;
+  const void* in[kMaxRhs];
+  void* out[kMaxRhs];
+};
+
 }  // namespace qcu

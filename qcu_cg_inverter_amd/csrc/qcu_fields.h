@@ -240,6 +240,33 @@ __device__ __forceinline__ uint4 pack8(const float f[8]) {
   return uint4{w[0], w[1], w[2], w[3]};
 }
 
+// The norm m of a site, its largest |real|, and the factors that bring its reals to
+// [-1, 1].  1 / m overflows float for m below 2^-128 (denormal norms): such a site is
+// scaled by 2^64 first, exactly; other sites see s = 1.
+struct F16Scale {
+  float m, s, inv;
+  __device__ __forceinline__ explicit F16Scale(float norm) : m(norm) {
+    s = m < 0x1p-100f ? 0x1p64f : 1.0f;
+    inv = m > 0.f ? 1.0f / (m * s) : 0.f;
+  }
+  __device__ __forceinline__ F16Scale(const cx<float>* v, int n) : F16Scale(largest(v, n)) {}
+  static __device__ __forceinline__ float largest(const cx<float>* v, int n) {
+    float m = 0.f;
+#pragma unroll
+    for (int c = 0; c < n; ++c) m = fmaxf(m, fmaxf(fabsf(v[c].re), fabsf(v[c].im)));
+    return m;
+  }
+  // z / m as a half pair (re low, im high), each product rounded once, straight to half.
+  // Written out because the compiler picks this form or a rounding to float first by
+  // context, and every kernel that stores or imitates a stored site has to agree.
+  __device__ __forceinline__ unsigned pair(cx<float> z) const {
+    unsigned r;
+    asm("v_fma_mixlo_f16 %0, %1, %3, 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0"
+        : "=&v"(r) : "v"(z.re * s), "v"(z.im * s), "v"(inv));
+    return r;
+  }
+};
+
 // half precision with one float scale per site: value = half * norm,
 // norm = max |real component| of the site
 template <>
@@ -291,25 +318,13 @@ struct SpinorIO<F16> {
   }
   template <int NTS = 0>
   static __device__ __forceinline__ void store(void* base, long vh, long i, const cx<T> v[12]) {
-    float m = 0.f;
-#pragma unroll
-    for (int c = 0; c < 12; ++c) m = fmaxf(m, fmaxf(fabsf(v[c].re), fabsf(v[c].im)));
-    // 1 / m overflows float for m below 2^-128 (denormal norms): such a site is scaled
-    // by 2^64 first, exactly, so its halves stay in [-1, 1]; other sites see s = 1
-    const float s = m < 0x1p-100f ? 0x1p64f : 1.0f;
-    const float inv = m > 0.f ? 1.0f / (m * s) : 0.f;
+    const F16Scale sc(v, 12);
     uint4* b = site_block<3>(static_cast<uint4*>(base), i);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      float f[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f[2 * j] = (v[4 * k + j].re * s) * inv;
-        f[2 * j + 1] = (v[4 * k + j].im * s) * inv;
-      }
-      stp<NTS>(b + k * kSiteBlock, pack8(f));
-    }
-    stp<NTS>(reinterpret_cast<float*>(static_cast<uint4*>(base) + 3 * padded_sites(vh)) + i, m);
+    for (int k = 0; k < 3; ++k)
+      stp<NTS>(b + k * kSiteBlock,
+               uint4{sc.pair(v[4 * k]), sc.pair(v[4 * k + 1]), sc.pair(v[4 * k + 2]), sc.pair(v[4 * k + 3])});
+    stp<NTS>(reinterpret_cast<float*>(static_cast<uint4*>(base) + 3 * padded_sites(vh)) + i, sc.m);
   }
 };
 

@@ -164,6 +164,18 @@ void hop(GaugeField& g, int prec, int recon, int epi, int parity, int dagger, do
 void hop_v(GaugeField& g, int prec, int recon, int epi, int parity, int dagger, double tbc, Vec in, Vec out, Vec x,
            const void* const* clovs, const double* coefs, int nrhs, double* partials, hipStream_t st);
 
+// the hop on the caller's interface buffers (api.cpp)
+struct IfaceHop {
+  const void* links;          // packed field of (prec, recon)
+  int prec, recon, epi;
+  int parity;                 // -1: both parities of full spinors
+  int dagger;
+  double tbc, coef;
+  const void* clov[2];        // per parity, for the clover epilogues
+};
+// false, with nothing launched, when an output overlaps an input or another output
+bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, const void* const* in, hipStream_t st);
+
 // solver entry (solver.cpp)
 void solve_batch(GaugeField& g, const qcuOperator& op, const qcuSolveParams& sp, int nrhs, void* const* x,
                  const void* const* b, qcuSolveStats* stats);

@@ -21,11 +21,13 @@ __host__ __device__ inline long n_partials(long vh) { return (vh + 15) / 16; }
 // right-hand sides per wave (1, 2 or 4), rpt per thread (1..4)
 void launch_hop(int prec, int recon, int epi, const HopArgs& a, int block, int rb, int rpt, hipStream_t st);
 
-// the hop on the interface layouts (complex128 half spinors [Vh][4][3], gauge
-// [4][2][Vh][3][3] of which rows 0-1 are read): out = coef * D^s_{p,1-p} in, FP64,
-// straight from and to the caller's buffers (k_hop_iface.hip)
-void launch_hop_iface(const void* in, void* out, const void* gauge_aos, const Geom& g, int parity, int dagger,
-                      double tbc, double coef, hipStream_t st);
+// the hop straight from and to the caller's interface fields (complex128 [Vh][4][3], or
+// full spinors), computed in `prec` (k_hop_split.inc); FP32 and FP16 take the plain
+// epilogue.  No out buffer may overlap an in buffer or another out buffer.
+void launch_hop_iface(int prec, int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st);
+// out(parity) = D in, FP64, periodic, with links from the caller's own gauge
+// [4][2][Vh][3][3], of which rows 0-1 are read; no overlap
+void launch_dslash(const void* in, void* out, const void* gauge, const Geom& g, int parity, hipStream_t st);
 
 // --------------------------------------------------------------- layout -----
 // interface spinor (complex128 [Vh][4][3]) <-> internal layout of `prec`

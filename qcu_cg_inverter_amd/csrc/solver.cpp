@@ -208,6 +208,12 @@ void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void*
   QREQ(kind >= QCU_COMP_AINV_D && kind <= QCU_COMP_NORMAL, "qcuApplyComposite: unknown kind");
   OpView o = make_view(g, op, F64);
   const long vh = g.geo.vh;
+  if (kind == QCU_COMP_AINV_D) {
+    IfaceHop p = {g.get(F64, op.recon), F64, op.recon, o.clover ? EPI_CLOV : EPI_PLAIN, -1, dagger ? 1 : 0, o.tbc(),
+                  op.kappa, {nullptr, nullptr}};
+    for (int q = 0; q < 2 && o.clover; ++q) p.clov[q] = o.cf->ainv(F64, q);
+    if (hop_iface(g.geo, p, 1, &out, &in, stream())) return;
+  }
   const size_t fb = spinor_bytes(F64, vh);
   Vec vi[2] = {vec(ctx().buf("cp_i0", fb)->p), vec(ctx().buf("cp_i1", fb)->p)};
   Vec vo[2] = {vec(ctx().buf("cp_o0", fb)->p), vec(ctx().buf("cp_o1", fb)->p)};
@@ -242,6 +248,11 @@ void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void*
 void apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger) {
   OpView o = make_view(g, op, F64);
   long vh = g.geo.vh;
+  IfaceHop p = {g.get(F64, op.recon), F64, op.recon, o.clover ? EPI_CLOV_XPAY : EPI_XPAY, -1, dagger, o.tbc(),
+                -op.kappa, {nullptr, nullptr}};
+  for (int q = 0; q < 2 && o.clover; ++q) p.clov[q] = o.cf->a(F64, q);
+  if (hop_iface(g.geo, p, 1, &out, &in, stream())) return;
+  // in and out overlap: staged in internal fields
   Vec ie = vec(ctx().buf("m_ie", spinor_bytes(F64, vh))->p);
   Vec io = vec(ctx().buf("m_io", spinor_bytes(F64, vh))->p);
   Vec oe = vec(ctx().buf("m_oe", spinor_bytes(F64, vh))->p);

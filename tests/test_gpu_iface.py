@@ -1,0 +1,70 @@
+"""Hops and operators straight from and to the caller's interface buffers
+(hop_split_kernel) against the path through internal fields, which a call whose output
+overlaps its input still takes, and against the oracle.  Half volumes off the 64-site
+chunk (8, 24 and 240 sites), of whole chunks, and t extents on and off the chunk order's
+tiles; right-hand sides from one to the most a launch takes."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+LATS = [(2, 2, 2, 2), (6, 2, 2, 2), (4, 6, 2, 10), (8, 8, 4, 16), (8, 4, 8, 12)]
+
+
+@pytest.fixture(scope="module")
+def q():
+    import qcu_cg_inverter_amd as q
+
+    q.init(0)
+    return q
+
+
+def ptrs(bufs):
+    return (ctypes.c_void_p * len(bufs))(*[b.ptr for b in bufs])
+
+
+@pytest.mark.parametrize("L", LATS)
+@pytest.mark.parametrize("prec,tol", [(0, 1e-14), (1, 1e-6), (2, 3e-3)])
+def test_hop_bits_equal_staged(q, L, prec, tol):
+    g = q.Gauge.random(L, seed=41, eps=0.3)
+    gref = g.to_numpy()
+    vh = q.half_volume(L)
+    for recon, nrhs, parity, dag, tb in ((12, 1, 0, 0, 1), (18, 1, 1, 1, -1), (12, 16, 1, 1, -1), (18, 3, 0, 0, -1)):
+        vs = [orc.source_gauss(L, 70 + r)[1 - parity] for r in range(nrhs)]
+        ins = [q.DeviceBuffer.from_numpy(v) for v in vs]
+        outs = [q.DeviceBuffer(vh * 192) for _ in range(nrhs)]
+        q.check(q.lib().qcuHopBatch(g.handle, nrhs, ptrs(outs), ptrs(ins), parity, dag, tb, recon, prec))
+        direct = [o.to_numpy((vh, 4, 3)) for o in outs]
+        q.check(q.lib().qcuHopBatch(g.handle, nrhs, ptrs(ins), ptrs(ins), parity, dag, tb, recon, prec))
+        for r in range(nrhs):
+            assert np.array_equal(direct[r], ins[r].to_numpy((vh, 4, 3))), (recon, nrhs, r)
+        ref = orc.hop(vs[-1], gref, L, parity, s=-1 if dag else 1, tbc=float(tb), recon=recon)
+        assert np.linalg.norm(direct[-1] - ref) <= tol * np.linalg.norm(ref), (recon, nrhs)
+
+
+@pytest.mark.parametrize("L", LATS)
+@pytest.mark.parametrize("csw", [0.0, 1.0])
+def test_full_operator_bits_equal_staged(q, L, csw):
+    g = q.Gauge.random(L, seed=42, eps=0.25)
+    gref = g.to_numpy()
+    vh = q.half_volume(L)
+    v = orc.source_gauss(L, 8)
+    A = orc.clover_fields(gref, L, 0.122, csw, recon=18)[0] if csw else None
+    for recon, dag, tb in ((12, 0, -1), (18, 1, 1)):
+        op = q.Operator(0.122, csw, tb, recon)
+        a, o = q.DeviceBuffer.from_numpy(v), q.DeviceBuffer(2 * vh * 192)
+        q.check(q.lib().qcuApplyM(g.handle, ctypes.byref(op), o.ptr, a.ptr, dag))
+        direct = o.to_numpy((2, vh, 4, 3))
+        q.check(q.lib().qcuApplyM(g.handle, ctypes.byref(op), a.ptr, a.ptr, dag))
+        assert np.array_equal(direct, a.to_numpy((2, vh, 4, 3))), (recon, dag)
+        ref = orc.full_op(v, gref, L, 0.122, A=A, s=-1 if dag else 1, tbc=float(tb), recon=recon)
+        assert np.linalg.norm(direct - ref) <= 1e-14 * np.linalg.norm(ref), (recon, dag)
+        a = q.DeviceBuffer.from_numpy(v)
+        q.check(q.lib().qcuApplyComposite(g.handle, ctypes.byref(op), q.COMP_AINV_D, o.ptr, a.ptr, dag))
+        direct = o.to_numpy((2, vh, 4, 3))
+        q.check(q.lib().qcuApplyComposite(g.handle, ctypes.byref(op), q.COMP_AINV_D, a.ptr, a.ptr, dag))
+        assert np.array_equal(direct, a.to_numpy((2, vh, 4, 3))), (recon, dag)
