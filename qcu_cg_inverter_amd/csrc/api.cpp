@@ -217,6 +217,38 @@ std::string tune_key(int prec, int recon, long vh, int nrhs, int epi) {
   else snprintf(b, sizeof b, "hop:%d:%d:%ld:%d:e%d", prec, recon, vh, nrhs, epi);
   return b;
 }
+// the largest divisor of Lt up to an eighth of it (rounded up)
+static int eighth_of_t(const Geom& geo) {
+  int tt = (geo.L[3] + 7) / 8;
+  while (geo.L[3] % tt) --tt;
+  return tt;
+}
+
+// Whether a hop on internal fields takes the leg-split kernel (k_hop_split.inc) when no
+// shape was tuned or pinned for it: while the launch's links and spinors come from the
+// Infinity Cache, the split's four waves per chunk keep more of that latency in flight;
+// past it the two kernels wait for the same HBM bytes, and the LDS kernel's one read of
+// the links per batch wins.  Per launch, hop_kernel / hop_lds_kernel against this one
+// (us): 8^4 FP64 9.2 / 5.1, FP32 6.9 / 4.2, 12-RHS FP32 14.2 / 6.0; 16^3x32 FP64 recon-18
+// 20.2 / 17.3, FP32 10.9 / 7.4, FP16 9.4 / 6.4, 12-RHS FP32 55.5 / 45.5; 24^3x48 FP32
+// 43.6 / 29.2 (190 MB); above the line: FP32 4 RHS (382 MB) 111 / 118, 32^3x64 (600 MB)
+// 113 / 127, FP64 recon-18 on 24^4 4 RHS (445 MB) 133 / 140.  FP64 recon-12 gains up to
+// 509 MB (24^3x48 95 / 75, 2 RHS 142 / 127) and is even at 1.2 GB.  FP16 spends its time
+// on unpacking and rebuilding the links, which the LDS kernel does once per batch: 24^3x48
+// 27 / 18.5, 4 RHS 63 / 59, but 16^3x32 12 RHS 31.6 / 36.
+static bool split_pays(int prec, int recon, long vh, int nrhs) {
+  const size_t bytes = gauge_bytes(prec, recon, vh) + 2 * (size_t)nrhs * spinor_bytes(prec, vh);
+  if (bytes > ((size_t)(prec == F64 && recon == 12 ? 550 : 320) << 20)) return false;
+  return prec != F16 || nrhs <= 4 || (vh + 63) / 64 * nrhs <= 6144;
+}
+// t-slices its chunks are taken at a time (ChunkOrder): an eighth of Lt, one tile per XCD
+// (16^3x32 FP64 4 RHS 40.4 -> 35.6 us, 24^3x48 FP32 33.4 -> 29.2), or storage order past
+// the Infinity Cache (24^3x48 FP64 recon-12 75 us, 85 in tiles)
+static int split_slices(const Geom& geo, size_t bytes) {
+  if (bytes > ((size_t)256 << 20)) return 1;
+  return eighth_of_t(geo);
+}
+
 // the shape tuned for this epilogue, else the one tuned for the plain epilogue, else
 // the default
 Tune tuned_hop(int prec, int recon, long vh, int nrhs, int epi) {
@@ -225,6 +257,7 @@ Tune tuned_hop(int prec, int recon, long vh, int nrhs, int epi) {
   it = ctx().tune.find(tune_key(prec, recon, vh, nrhs, EPI_PLAIN));
   if (it != ctx().tune.end()) return it->second;
   Tune t;
+  t.split = split_pays(prec, recon, vh, nrhs);
   if (nrhs > 1) {  // every right-hand side in one block per 64-site chunk, its links
     // staged in LDS once (hop_lds_kernel; on 32^3x64 with 12 right-hand sides 22-29 %
     // faster than the best shape sharing link loads within a wave), 4 waves per block,
@@ -240,6 +273,26 @@ Tune tuned_hop(int prec, int recon, long vh, int nrhs, int epi) {
 void set_tuned_hop(int prec, int recon, long vh, int nrhs, const Tune& t) {
   for (int e = EPI_PLAIN; e <= EPI_CLOV_XPAY; ++e) ctx().tune.erase(tune_key(prec, recon, vh, nrhs, e));
   ctx().tune[tune_key(prec, recon, vh, nrhs, EPI_PLAIN)] = t;
+}
+
+void launch_shape(int prec, int recon, int epi, HopArgs& a, const Tune& t, hipStream_t st) {
+  if (t.split) {
+    HopSplit s;
+    s.h = a;
+    s.drhs = FastDiv((uint32_t)a.nrhs);
+    s.order = make_chunk_order(a.geo, split_slices(a.geo, gauge_bytes(prec, recon, a.geo.vh) +
+                                                             2 * (size_t)a.nrhs * spinor_bytes(prec, a.geo.vh)));
+    launch_hop_split(prec, recon, epi, s, st);
+    return;
+  }
+  a.xcd_remap = t.xcd;
+  a.gmajor = t.gm;
+  a.rpw = t.rpw;
+  a.spt = t.spt;
+  a.cached = t.cached;
+  a.lds = t.lds;
+  a.walk = make_walk(a.geo, t.ty, t.tz < 0 ? a.geo.L[2] : t.tz, t.tt);
+  launch_hop(prec, recon, epi, a, t.block, t.rb, t.rpt, st);
 }
 
 void hop(GaugeField& g, int prec, int recon, int epi, int parity, int dagger, double tbc, Vec in, Vec out, Vec x,
@@ -278,15 +331,8 @@ void hop_v(GaugeField& g, int prec, int recon, int epi, int parity, int dagger, 
   a.dagger = dagger;
   a.tbc = tbc;
   a.nrhs = nrhs;
-  Tune t = tuned_hop(prec, recon, g.geo.vh, nrhs, epi);
-  a.xcd_remap = t.xcd;
-  a.gmajor = t.gm;
-  a.rpw = t.rpw;
-  a.spt = t.spt;
-  a.cached = t.cached;
-  a.lds = t.lds;
-  a.walk = make_walk(g.geo, t.ty, t.tz < 0 ? g.geo.L[2] : t.tz, t.tt);
-  launch_hop(prec, recon, epi, a, t.block, t.rb, t.rpt, st);
+  const Tune t = tuned_hop(prec, recon, g.geo.vh, nrhs, epi);
+  launch_shape(prec, recon, epi, a, t, st);
 }
 
 // t-slices the chunks of an interface launch are taken at a time (ChunkOrder): an eighth
@@ -297,9 +343,7 @@ void hop_v(GaugeField& g, int prec, int recon, int epi, int parity, int dagger, 
 // operator 812 / 675; but one FP64 half spinor 84.7 / 91.7 and 264.6 / 269.6 us.
 static int iface_slices(const Geom& geo, const IfaceHop& p, int nrhs) {
   if (p.prec == F64 && nrhs == 1 && p.parity >= 0) return 1;
-  int tt = (geo.L[3] + 7) / 8;
-  while (geo.L[3] % tt) --tt;
-  return tt;
+  return eighth_of_t(geo);
 }
 
 bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, const void* const* in, hipStream_t st) {

@@ -16,6 +16,10 @@ void launch_iface_f64(int, int, int, const IfaceArgs&, hipStream_t);
 void launch_iface_f32(int, int, const IfaceArgs&, hipStream_t);
 void launch_iface_f16(int, int, const IfaceArgs&, hipStream_t);
 
+void launch_split_f64(int, int, const HopSplit&, hipStream_t);
+void launch_split_f32(int, int, const HopSplit&, hipStream_t);
+void launch_split_f16(int, int, const HopSplit&, hipStream_t);
+
 void launch_hop(int prec, int recon, int epi, const HopArgs& a, int block, int rb, int rpt, hipStream_t st) {
   typedef void (*Fn)(int, int, const HopArgs&, int, int, hipStream_t);
   static const Fn table[3][4] = {
@@ -31,5 +35,11 @@ void launch_hop_iface(int prec, int recon, int epi, int dagger, const IfaceArgs&
   if (prec == F64) launch_iface_f64(recon, epi, dagger, a, st);
   else if (prec == F32) launch_iface_f32(recon, dagger, a, st);
   else launch_iface_f16(recon, dagger, a, st);
+}
+
+void launch_hop_split(int prec, int recon, int epi, const HopSplit& a, hipStream_t st) {
+  if (prec == F64) launch_split_f64(recon, epi, a, st);
+  else if (prec == F32) launch_split_f32(recon, epi, a, st);
+  else launch_split_f16(recon, epi, a, st);
 }
 }  // namespace qcu

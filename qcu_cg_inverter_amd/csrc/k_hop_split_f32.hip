@@ -8,4 +8,9 @@ void launch_iface_f32(int recon, int dagger, const IfaceArgs& a, hipStream_t st)
   else launch_iface<F32, 18, EPI_PLAIN>(a, dagger, st);
 }
 
+void launch_split_f32(int recon, int epi, const HopSplit& a, hipStream_t st) {
+  if (recon == 12) launch_split_epi<F32, 12>(epi, a, st);
+  else launch_split_epi<F32, 18>(epi, a, st);
+}
+
 }  // namespace qcu

@@ -30,4 +30,9 @@ void launch_dslash(const void* in, void* out, const void* gauge, const Geom& g, 
                      static_cast<const double2*>(gauge), g, parity);
 }
 
+void launch_split_f64(int recon, int epi, const HopSplit& a, hipStream_t st) {
+  if (recon == 12) launch_split_epi<F64, 12>(epi, a, st);
+  else launch_split_epi<F64, 18>(epi, a, st);
+}
+
 }  // namespace qcu

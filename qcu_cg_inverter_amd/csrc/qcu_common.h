@@ -206,6 +206,14 @@ inline ChunkOrder make_chunk_order(const Geom& g, int tt) {
   return o;
 }
 
+// One launch of the leg-split kernel on internal fields (k_hop_split.inc); h's launch
+// shape does not apply.
+struct HopSplit {
+  HopArgs h;
+  FastDiv drhs;
+  ChunkOrder order;
+};
+
 // One launch on the caller's interface fields (k_hop_split.inc): half spinors in[r] ->
 // out[r] of one parity, or, with parity -1, full spinors on both parities, where an
 // epilogue's x is the other half of `in` and the clover clov0 / clov1 by parity.

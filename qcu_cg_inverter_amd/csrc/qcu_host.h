@@ -113,6 +113,7 @@ struct Tune {
   int cached = 0;
   int lds = 0;  // 1: every right-hand side in one block per 64-site chunk, its links staged in LDS;
                 // 2: a clover shared by every right-hand side staged too
+  int split = 0;  // 1: the leg-split kernel; the rest does not apply
 };
 
 struct Context {
@@ -145,6 +146,8 @@ std::unique_ptr<GaugeField> make_gauge_from_aos(const void* aos_device, const in
 std::unique_ptr<GaugeField> make_gauge_random(const int L[4], uint64_t seed, double eps);
 
 Tune tuned_hop(int prec, int recon, long vh, int nrhs, int epi = EPI_PLAIN);
+// one hop launch with shape t (a's shape fields are set from it)
+void launch_shape(int prec, int recon, int epi, HopArgs& a, const Tune& t, hipStream_t st);
 std::string tune_key(int prec, int recon, long vh, int nrhs, int epi);
 void set_tuned_hop(int prec, int recon, long vh, int nrhs, const Tune& t);
 // autotuner (tune.cpp)

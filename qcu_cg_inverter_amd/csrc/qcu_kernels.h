@@ -21,6 +21,9 @@ __host__ __device__ inline long n_partials(long vh) { return (vh + 15) / 16; }
 // right-hand sides per wave (1, 2 or 4), rpt per thread (1..4)
 void launch_hop(int prec, int recon, int epi, const HopArgs& a, int block, int rb, int rpt, hipStream_t st);
 
+// the hop on internal fields with each chunk's legs split over four waves
+void launch_hop_split(int prec, int recon, int epi, const HopSplit& a, hipStream_t st);
+
 // the hop straight from and to the caller's interface fields (complex128 [Vh][4][3], or
 // full spinors), computed in `prec` (k_hop_split.inc); FP32 and FP16 take the plain
 // epilogue.  No out buffer may overlap an in buffer or another out buffer.
