@@ -71,11 +71,12 @@ void DevBuf::release() {
   p = nullptr;
   n = 0;
 }
-void DevBuf::alloc(size_t bytes) {
+void* DevBuf::alloc(size_t bytes) {
   release();
-  if (bytes == 0) return;
+  if (bytes == 0) return nullptr;
   QHIP(hipMalloc(&p, bytes));
   n = bytes;
+  return p;
 }
 void DevBuf::ensure(size_t bytes) {
   if (bytes > n) alloc(bytes);
@@ -140,43 +141,40 @@ const void* GaugeField::get(int prec, int recon) {
   return b.p;
 }
 
-CloverField* GaugeField::clover(double ck, int prec, bool full_inverse) {
+CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
   auto it = clovers.find(ck);
   CloverField* cf;
   if (it == clovers.end()) {
     std::unique_ptr<CloverField> c(new CloverField);
     c->ck = ck;
     c->vh = geo.vh;
+    c->bad.alloc(sizeof(int));
+    QHIP(hipMemsetAsync(c->bad.p, 0, sizeof(int), stream()));
     cf = c.get();
     clovers[ck] = std::move(c);
   } else {
     cf = it->second.get();
   }
   const size_t half64 = clover_bytes(F64, geo.vh) / 2;
-  // FP64 parts: A on both parities, A^-1 on the odd one, A^-1 on the even one if asked
-  const bool need_a = !cf->A[F64][0].p, need_ie = full_inverse && !cf->Ainv[F64][0].p;
-  if (need_a || need_ie) {
-    const void* g18 = get(F64, 18);
-    DevBuf* G = ctx().buf("clover_G", (size_t)6 * 9 * 16 * geo.vh);
-    DevBuf* nb = ctx().buf("clover_nbad", sizeof(int));
-    QHIP(hipMemsetAsync(nb->p, 0, sizeof(int), stream()));
-    for (int p = 0; p < 2; ++p) {
-      const bool want_a = need_a, want_i = p == 1 ? need_a : (need_ie || (need_a && full_inverse));
-      if (!want_a && !want_i) continue;
-      if (want_a) cf->A[F64][p].alloc(half64);
-      if (want_i) cf->Ainv[F64][p].alloc(half64);
-      launch_clover_leaves(g18, G->p, geo, p, stream());
-      launch_clover_assemble(G->p, want_a ? cf->A[F64][p].p : nullptr, want_i ? cf->Ainv[F64][p].p : nullptr,
-                             geo.vh, ck, static_cast<int*>(nb->p), stream());
-    }
+  CloverBuild b;
+  bool need[2];
+  for (int p = 0; p < 2; ++p) {
+    const bool inv = parts == CLOVER_ALL || (parts == CLOVER_SOLVE && p == 1);
+    b.A[p] = cf->A[F64][p].p ? nullptr : cf->A[F64][p].alloc(half64);
+    b.Ainv[p] = !inv || cf->Ainv[F64][p].p ? nullptr : cf->Ainv[F64][p].alloc(half64);
+    need[p] = b.A[p] || b.Ainv[p];
+  }
+  if (need[0] || need[1]) {
+    b.gauge = get(F64, 18);
+    b.nbad = static_cast<int*>(cf->bad.p);
+    b.ck = ck;
+    b.only = need[0] && need[1] ? -1 : need[1];
+    b.geo = geo;
+    launch_clover_build(18, b, stream());
     QHIP(hipGetLastError());
-    int nbad = 0;
-    QHIP(hipMemcpyAsync(&nbad, nb->p, sizeof(int), hipMemcpyDeviceToHost, stream()));
-    QHIP(hipStreamSynchronize(stream()));
-    cf->nbad += nbad;
   }
   // inner-precision parts: A_ee and A^-1_oo
-  if (prec != F64 && !cf->A[prec][0].p) {
+  if (parts != CLOVER_A && prec != F64 && !cf->A[prec][0].p) {
     const size_t half = clover_bytes(prec, geo.vh) / 2;
     cf->A[prec][0].alloc(half);
     cf->Ainv[prec][1].alloc(half);
@@ -767,15 +765,17 @@ int qcuCloverExport(qcuGauge h, const qcuOperator* op, void* A, void* Ainv, int*
     ensure_init();
     QREQ(h && op, "qcuCloverExport: NULL argument");
     GaugeField& g = *reinterpret_cast<GaugeField*>(h);
-    CloverField* cf = g.clover(op->kappa * op->csw, F64, true);
+    CloverField* cf = g.clover(op->kappa * op->csw, F64, CLOVER_ALL);
     size_t half = (size_t)g.geo.vh * 72 * 16;
     for (int p = 0; p < 2; ++p) {
       if (A) launch_clover_unpack(cf->a(F64, p), static_cast<char*>(A) + p * half, g.geo.vh, stream());
       if (Ainv) launch_clover_unpack(cf->ainv(F64, p), static_cast<char*>(Ainv) + p * half, g.geo.vh, stream());
     }
     QHIP(hipGetLastError());
+    int nbad = 0;
+    QHIP(hipMemcpyAsync(&nbad, cf->bad.p, sizeof(int), hipMemcpyDeviceToHost, stream()));
     QHIP(hipStreamSynchronize(stream()));
-    if (nfallback) *nfallback = cf->nbad;
+    if (nfallback) *nfallback = nbad;
   });
 }
 

@@ -18,151 +18,194 @@ typedef cx<double> zd;
 
 static inline unsigned nblk(long n, int b) { return (unsigned)((n + b - 1) / b); }
 
-__device__ __forceinline__ void load_link_at(const double2* g, const Geom& geo, int x, int y, int z, int t, int mu,
-                                             zd u[9]) {
-  x = x < 0 ? x + geo.L[0] : (x >= geo.L[0] ? x - geo.L[0] : x);
-  y = y < 0 ? y + geo.L[1] : (y >= geo.L[1] ? y - geo.L[1] : y);
-  z = z < 0 ? z + geo.L[2] : (z >= geo.L[2] ? z - geo.L[2] : z);
-  t = t < 0 ? t + geo.L[3] : (t >= geo.L[3] ? t - geo.L[3] : t);
-  int par = (x + y + z + t) & 1;
-  long idx = t * geo.st + z * geo.sz + y * geo.sy + (x >> 1);
-  const double2* b = link_word<F64, 18>(g, geo.vh, mu * 2 + par, idx);
-  const long ws = link_stride<F64, 18>(geo.vh);
+// U_dir at site c + dm e_mu + dn e_nu (dm, dn in -1, 0, 1)
+template <int R>
+__device__ __forceinline__ void load_link_at(const void* g, const Geom& geo, const int c[4], int mu, int nu, int dm,
+                                             int dn, int dir, zd u[9]) {
+  int x[4];
+  int par = 0;
 #pragma unroll
-  for (int e = 0; e < 9; ++e) {
-    double2 q = b[e * ws];
-    u[e] = {q.x, q.y};
+  for (int k = 0; k < 4; ++k) {
+    int v = c[k] + (k == mu ? dm : 0) + (k == nu ? dn : 0);
+    v = v < 0 ? v + geo.L[k] : (v >= geo.L[k] ? v - geo.L[k] : v);
+    x[k] = v;
+    par ^= v & 1;
   }
+  const long idx = x[3] * geo.st + x[2] * geo.sz + x[1] * geo.sy + (x[0] >> 1);
+  LinkIO<F64, R>::template load<0>(g, geo.vh, dir, par, idx, u);
 }
 
-__device__ __forceinline__ void m3mul(zd r[9], const zd a[9], const zd b[9]) {
+// r = a b and a b^dag; r must not alias a or b
+__device__ __forceinline__ void mul_nn(zd r[9], const zd a[9], const zd b[9]) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) r[i * 3 + j] = a[i * 3] * b[j] + a[i * 3 + 1] * b[3 + j] + a[i * 3 + 2] * b[6 + j];
+    for (int j = 0; j < 3; ++j)
+      r[i * 3 + j] = cmad(a[i * 3 + 2], b[6 + j], cmad(a[i * 3 + 1], b[3 + j], a[i * 3] * b[j]));
 }
-__device__ __forceinline__ void m3dag(zd r[9], const zd a[9]) {
+__device__ __forceinline__ void mul_nd(zd r[9], const zd a[9], const zd b[9]) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) r[i * 3 + j] = conj(a[j * 3 + i]);
+    for (int j = 0; j < 3; ++j)
+      r[i * 3 + j] = cmadc(b[j * 3 + 2], a[i * 3 + 2], cmadc(b[j * 3 + 1], a[i * 3 + 1], mulc(a[i * 3], b[j * 3])));
+}
+// r -= a^dag b and r += a b
+__device__ __forceinline__ void sub_dn(zd r[9], const zd a[9], const zd b[9]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      r[i * 3 + j] =
+          r[i * 3 + j] - cmadc(a[6 + i], b[6 + j], cmadc(a[3 + i], b[3 + j], mulc(b[j], a[i])));
+}
+__device__ __forceinline__ void add_nn(zd r[9], const zd a[9], const zd b[9]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      r[i * 3 + j] =
+          r[i * 3 + j] + cmad(a[i * 3 + 2], b[6 + j], cmad(a[i * 3 + 1], b[3 + j], a[i * 3] * b[j]));
 }
 
-// thread per (site, plane): G = Q - Q^dag written to G[(pl * 9 + e) * vh + site]
-__global__ void clover_leaves_kernel(const double2* gauge, double2* G, Geom geo, int parity) {
-  long site = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int pl = blockIdx.y;
-  if (site >= geo.vh) return;
-  const int pmu[6] = {0, 0, 0, 1, 1, 2}, pnu[6] = {1, 2, 3, 2, 3, 3};
-  int mu = pmu[pl], nu = pnu[pl];
-  long r = site;
-  int xh = (int)(r % geo.lxh); r /= geo.lxh;
-  int y = (int)(r % geo.L[1]); r /= geo.L[1];
-  int z = (int)(r % geo.L[2]); r /= geo.L[2];
-  int t = (int)r;
-  int x = 2 * xh + ((parity + y + z + t) & 1);
-  int c[4] = {x, y, z, t};
-  auto at = [&](int dm, int dn, int dir, zd u[9]) {
-    int d[4] = {c[0], c[1], c[2], c[3]};
-    d[mu] += dm;
-    d[nu] += dn;
-    load_link_at(gauge, geo, d[0], d[1], d[2], d[3], dir, u);
-  };
-  zd a[9], b[9], t1[9], t2[9], q[9];
-  // F1 = U_mu(x) U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag
-  at(0, 0, mu, a); at(1, 0, nu, b); m3mul(t1, a, b);
-  at(0, 1, mu, a); m3dag(b, a); m3mul(t2, t1, b);
-  at(0, 0, nu, a); m3dag(b, a); m3mul(q, t2, b);
-  // F2 = U_nu(x) U_mu(x-mu+nu)^dag U_nu(x-mu)^dag U_mu(x-mu)
-  at(0, 0, nu, a); at(-1, 1, mu, t2); m3dag(b, t2); m3mul(t1, a, b);
-  at(-1, 0, nu, a); m3dag(b, a); m3mul(t2, t1, b);
-  at(-1, 0, mu, a); m3mul(t1, t2, a);
+// G = Q - Q^dag of plane (mu, nu) at site c, Q the sum of the four leaves
+//   U_mu(x) S1, S1 = U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag
+//   S2 U_mu(x-mu), S2 = U_nu(x) U_mu(x-mu+nu)^dag U_nu(x-mu)^dag
+//   U_mu(x-mu)^dag S3, S3 = U_nu(x-mu-nu)^dag U_mu(x-mu-nu) U_nu(x-nu)
+//   S4 U_mu(x)^dag, S4 = U_nu(x-nu)^dag U_mu(x-nu) U_nu(x-nu+mu)
+// as D - D^dag with D = U_mu(x) (S1 - S4^dag) + (S2 - S3^dag) U_mu(x-mu): ten matrix
+// products and twelve links.  G is anti-Hermitian: out holds the imaginary diagonal, then
+// the entries (1,0) (2,0) (2,1) below it.
+template <int R>
+__device__ __forceinline__ void plane_field(const void* gauge, const Geom& geo, const int c[4], int mu, int nu,
+                                            double out[9]) {
+  auto at = [&](int dm, int dn, int dir, zd u[9]) { load_link_at<R>(gauge, geo, c, mu, nu, dm, dn, dir, u); };
+  zd a[9], b[9], t[9], d[9], r[9];  // at most four of them live
+  at(0, 0, nu, a); at(0, 1, mu, b); mul_nn(t, a, b);     // U_nu(x) U_mu(x+nu)
+  at(1, 0, nu, b); mul_nd(d, b, t);                      // S1
+  at(0, -1, mu, a); at(1, -1, nu, b); mul_nn(t, a, b);   // U_mu(x-nu) U_nu(x-nu+mu)
+  at(0, -1, nu, a); sub_dn(d, t, a);                     // S1 - S4^dag
+  at(0, 0, mu, a); mul_nn(r, a, d);
+  at(-1, 0, nu, a); at(-1, 1, mu, b); mul_nn(t, a, b);   // U_nu(x-mu) U_mu(x-mu+nu)
+  at(0, 0, nu, a); mul_nd(d, a, t);                      // S2
+  at(-1, -1, mu, a); at(0, -1, nu, b); mul_nn(t, a, b);  // U_mu(x-mu-nu) U_nu(x-nu)
+  at(-1, -1, nu, a); sub_dn(d, t, a);                    // S2 - S3^dag
+  at(-1, 0, mu, a); add_nn(r, d, a);
 #pragma unroll
-  for (int k = 0; k < 9; ++k) q[k] = q[k] + t1[k];
-  // F3 = U_mu(x-mu)^dag U_nu(x-mu-nu)^dag U_mu(x-mu-nu) U_nu(x-nu)
-  at(-1, 0, mu, b); m3dag(a, b); at(-1, -1, nu, t2); m3dag(b, t2); m3mul(t1, a, b);
-  at(-1, -1, mu, a); m3mul(t2, t1, a);
-  at(0, -1, nu, a); m3mul(t1, t2, a);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) q[k] = q[k] + t1[k];
-  // F4 = U_nu(x-nu)^dag U_mu(x-nu) U_nu(x-nu+mu) U_mu(x)^dag
-  at(0, -1, nu, b); m3dag(a, b); at(0, -1, mu, b); m3mul(t1, a, b);
-  at(1, -1, nu, a); m3mul(t2, t1, a);
-  at(0, 0, mu, a); m3dag(b, a); m3mul(t1, t2, b);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) q[k] = q[k] + t1[k];
-  m3dag(b, q);
-  double2* o = G + (long)pl * 9 * geo.vh + site;
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    zd v = q[k] - b[k];
-    o[k * geo.vh] = double2{v.re, v.im};
-  }
+  for (int k = 0; k < 3; ++k) out[k] = r[4 * k].im + r[4 * k].im;
+  const zd g10 = r[3] - conj(r[1]), g20 = r[6] - conj(r[2]), g21 = r[7] - conj(r[5]);
+  out[3] = g10.re; out[4] = g10.im; out[5] = g20.re; out[6] = g20.im; out[7] = g21.re; out[8] = g21.im;
 }
 
-// g_mu g_nu entries per plane: (row spin, col spin, phase i^k), the reference's table
-__device__ constexpr int CL_COL[6][4] = {{0, 1, 2, 3}, {1, 0, 3, 2}, {1, 0, 3, 2}, {1, 0, 3, 2}, {1, 0, 3, 2}, {0, 1, 2, 3}};
+// g_mu g_nu entries per plane: phase i^k by row spin; planes 0 and 5 couple a spin to
+// itself, the others the two spins of a chiral block (the reference's table)
 __device__ constexpr int CL_PH[6][4] = {{3, 1, 3, 1}, {2, 0, 2, 0}, {1, 1, 3, 3}, {3, 3, 3, 3}, {2, 0, 0, 2}, {1, 3, 3, 1}};
 
-// Cholesky inverse of a Hermitian 6x6 (full storage m[36]); false if not
-// positive definite
-__device__ bool chol_inv6(const zd m[36], zd inv[36]) {
-  zd l[36];
-  double dinv[6];
+// a packed Hermitian 6x6 block: real diagonal d, entry (i, j) below it at
+// l[i (i - 1) / 2 + j]
+struct Block6 {
+  double d[6];
+  zd l[15];
+  __device__ __forceinline__ zd& at(int i, int j) { return l[i * (i - 1) / 2 + j]; }
+};
+
+// plane fields of one site in LDS, [plane][9 reals][64 lanes]
+typedef double PlaneLds[6][9][64];
+__device__ __forceinline__ zd plane_entry(const PlaneLds& G, int pl, int lane, int i, int j) {
+  if (i == j) return {0.0, G[pl][i][lane]};
+  const int k = 3 + 2 * (i + j - 1);
+  const double re = G[pl][k][lane], im = G[pl][k + 1][lane];
+  return i > j ? zd{re, im} : zd{-re, im};
+}
+
+// chiral block B of 1 + ck T
+template <int B>
+__device__ __forceinline__ void assemble_block(const PlaneLds& G, int lane, double ck, Block6& m) {
 #pragma unroll
-  for (int k = 0; k < 36; ++k) l[k] = {0.0, 0.0};
+  for (int s = 0; s < 2; ++s) {
+    constexpr int planes[2] = {0, 5};
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j <= i; ++j) {
+        zd v = {0.0, 0.0};
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          v = v + -0.125 * iph(plane_entry(G, planes[p], lane, i, j), CL_PH[planes[p]][2 * B + s]);
+        if (i == j) m.d[3 * s + i] = 1.0 + ck * v.re;
+        else m.at(3 * s + i, 3 * s + j) = ck * v;
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      zd v = {0.0, 0.0};
+#pragma unroll
+      for (int pl = 1; pl < 5; ++pl) v = v + -0.125 * iph(plane_entry(G, pl, lane, i, j), CL_PH[pl][2 * B + 1]);
+      m.at(3 + i, j) = ck * v;
+    }
+}
+
+// Inverse of a Hermitian 6x6 in place by Cholesky, W = L^-1, W^dag W; every step
+// overwrites only entries no later step reads, so the block never leaves 72 registers.
+// false, with the block spoilt, if it is not positive definite.
+__device__ __forceinline__ bool chol_inv6(Block6& m) {
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
-    double d = m[j * 6 + j].re;
+    double d = m.d[j];
 #pragma unroll
-    for (int k = 0; k < j; ++k) d -= norm2(l[j * 6 + k]);
+    for (int k = 0; k < j; ++k) d -= norm2(m.at(j, k));
     if (!(d > 0.0)) return false;
-    double lj = sqrt(d);
-    l[j * 6 + j] = {lj, 0.0};
-    dinv[j] = 1.0 / lj;
+    m.d[j] = 1.0 / sqrt(d);  // 1 / l_jj from here on
 #pragma unroll
     for (int i = j + 1; i < 6; ++i) {
-      zd s = m[i * 6 + j];
+      zd s = m.at(i, j);
 #pragma unroll
-      for (int k = 0; k < j; ++k) s = s - mulc(l[i * 6 + k], l[j * 6 + k]);
-      l[i * 6 + j] = dinv[j] * s;
-    }
-  }
-  zd w[36];
-#pragma unroll
-  for (int k = 0; k < 36; ++k) w[k] = {0.0, 0.0};
-#pragma unroll
-  for (int j = 0; j < 6; ++j) {
-    w[j * 6 + j] = {dinv[j], 0.0};
-#pragma unroll
-    for (int i = j + 1; i < 6; ++i) {
-      zd s = {0.0, 0.0};
-#pragma unroll
-      for (int k = j; k < i; ++k) s = s + l[i * 6 + k] * w[k * 6 + j];
-      w[i * 6 + j] = (-dinv[i]) * s;
+      for (int k = 0; k < j; ++k) s = s - mulc(m.at(i, k), m.at(j, k));
+      m.at(i, j) = m.d[j] * s;
     }
   }
 #pragma unroll
-  for (int i = 0; i < 6; ++i)
+  for (int j = 0; j < 6; ++j)
 #pragma unroll
-    for (int j = 0; j <= i; ++j) {
-      zd s = {0.0, 0.0};
+    for (int i = j + 1; i < 6; ++i) {
+      zd s = m.d[j] * m.at(i, j);
 #pragma unroll
-      for (int k = i; k < 6; ++k) s = s + conj(w[k * 6 + i]) * w[k * 6 + j];
-      inv[i * 6 + j] = s;
-      inv[j * 6 + i] = conj(s);
+      for (int k = j + 1; k < i; ++k) s = s + m.at(i, k) * m.at(k, j);
+      m.at(i, j) = (-m.d[i]) * s;
     }
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+#pragma unroll
+    for (int j = 0; j < i; ++j) {
+      zd s = m.d[i] * m.at(i, j);
+#pragma unroll
+      for (int k = i + 1; k < 6; ++k) s = s + mulc(m.at(k, j), m.at(k, i));
+      m.at(i, j) = s;
+    }
+    double s = m.d[i] * m.d[i];
+#pragma unroll
+    for (int k = i + 1; k < 6; ++k) s += norm2(m.at(k, i));
+    m.d[i] = s;
+  }
   return true;
 }
 
 // Gauss-Jordan with partial pivoting (any nonsingular 6x6)
-__device__ void gj_inv6(const zd m[36], zd inv[36]) {
+// of the packed block, for the rare blocks that are not positive definite; out of line, so
+// its arrays stay out of the common path's registers
+__device__ __attribute__((noinline)) void gj_inv6(Block6& m) {
+  zd inv[36];
   zd a[36];
-#pragma unroll
-  for (int k = 0; k < 36; ++k) {
-    a[k] = m[k];
-    inv[k] = {(k % 7 == 0) ? 1.0 : 0.0, 0.0};
+  for (int i = 0; i < 6; ++i) {
+    a[i * 7] = {m.d[i], 0.0};
+    for (int j = 0; j < i; ++j) {
+      a[i * 6 + j] = m.at(i, j);
+      a[j * 6 + i] = conj(m.at(i, j));
+    }
   }
+  for (int k = 0; k < 36; ++k) inv[k] = {(k % 7 == 0) ? 1.0 : 0.0, 0.0};
   for (int c = 0; c < 6; ++c) {
     int piv = c;
     double best = norm2(a[c * 6 + c]);
@@ -192,65 +235,74 @@ __device__ void gj_inv6(const zd m[36], zd inv[36]) {
       }
     }
   }
+  for (int i = 0; i < 6; ++i) {
+    m.d[i] = inv[i * 7].re;
+    for (int j = 0; j < i; ++j) m.at(i, j) = inv[i * 6 + j];
+  }
 }
 
-__device__ __forceinline__ void pack_block(const zd m[36], double2* out, long vh, long site, int b) {
-  double r[36];
-  for (int i = 0; i < 6; ++i) r[i] = m[i * 7].re;
-  int k = 6;
-  for (int i = 1; i < 6; ++i)
-    for (int j = 0; j < i; ++j) {
-      r[k] = m[i * 6 + j].re;
-      r[k + 1] = m[i * 6 + j].im;
-      k += 2;
-    }
-  double2* o = site_block<36>(out, site) + b * 18 * kSiteBlock;
+__device__ __forceinline__ void pack_block(const Block6& m, void* out, long site, int b) {
+  double2* o = site_block<36>(static_cast<double2*>(out), site) + b * 18 * kSiteBlock;
 #pragma unroll
-  for (int q = 0; q < 18; ++q) o[q * kSiteBlock] = double2{r[2 * q], r[2 * q + 1]};
+  for (int q = 0; q < 3; ++q) o[q * kSiteBlock] = double2{m.d[2 * q], m.d[2 * q + 1]};
+#pragma unroll
+  for (int q = 0; q < 15; ++q) o[(3 + q) * kSiteBlock] = double2{m.l[q].re, m.l[q].im};
 }
 
-// thread per (site, chiral block b)
-__global__ void clover_assemble_kernel(const double2* G, double2* A, double2* Ainv, long vh, double ck, int* nbad) {
-  long site = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int b = blockIdx.y;
-  if (site >= vh) return;
-  zd m[36];
-#pragma unroll
-  for (int k = 0; k < 36; ++k) m[k] = {0.0, 0.0};
-  for (int pl = 0; pl < 6; ++pl) {
-    zd g[9];
-    const double2* gp = G + (long)pl * 9 * vh + site;
-#pragma unroll
-    for (int e = 0; e < 9; ++e) {
-      double2 q = gp[e * vh];
-      g[e] = {q.x, q.y};
-    }
-#pragma unroll
-    for (int e = 2 * b; e < 2 * b + 2; ++e) {  // entries whose row spin lies in block b
-      int rs = e, cs = CL_COL[pl][e];
-      zd ph = iph(zd{-0.125, 0.0}, CL_PH[pl][e]);
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          int row = (rs & 1) * 3 + i, col = (cs & 1) * 3 + j;
-          m[row * 6 + col] = m[row * 6 + col] + ph * g[i * 3 + j];
-        }
-    }
+template <int B>
+__device__ __forceinline__ void build_block(const PlaneLds& G, int lane, bool live, const CloverBuild& a, int parity,
+                                            long site) {
+  Block6 m;
+  assemble_block<B>(G, lane, a.ck, m);
+  if (a.A[parity] && live) pack_block(m, a.A[parity], site, B);
+  if (!a.Ainv[parity]) return;
+  if (!chol_inv6(m)) {
+    Block6 f;  // of its own: its address leaves the function, m's registers must not
+    assemble_block<B>(G, lane, a.ck, f);
+    gj_inv6(f);
+    m = f;
+    if (live) atomicAdd(a.nbad, 1);
+  }
+  if (live) pack_block(m, a.Ainv[parity], site, B);
+}
+
+// A block of six waves per (64-site chunk, parity), the two parities of a chunk side by
+// side: wave pl multiplies out the leaves of plane pl for the 64 sites and leaves G in
+// LDS; then waves 0 and 1 assemble chiral blocks 0 and 1, write A and invert them in
+// place.  G never goes to memory and a block lives in 72 registers: the two kernels this
+// replaces wrote and read 864 B of G a site and kept four full 6x6 complex arrays, mostly
+// in scratch.  The leaves bound it (12 links of 144 B and 1,080 FP64 instructions a site
+// and plane, one block of 256-register waves per CU).  16^3x32: A of both parities 92 us,
+// with the odd inverse 117 (1,030 before); 24^3x48: 520 and 660 us (3,100 before).  Three
+// waves a SIMD (168 registers) spill: 125 and 720 us for A.
+template <int R>
+__global__ void __launch_bounds__(384, 2) clover_build_kernel(const CloverBuild a) {
+  __shared__ PlaneLds G;
+  const Geom& geo = a.geo;
+  const int lane = threadIdx.x & 63;
+  const int pl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned u = remap_block(blockIdx.x, gridDim.x, 1);
+  const int parity = a.only < 0 ? (int)(u & 1u) : a.only;
+  const long l = (long)(a.only < 0 ? u >> 1 : u) * 64 + lane;
+  const bool live = l < geo.vh;
+  const long site = live ? l : geo.vh - 1;
+  const uint32_t q1 = geo.dx.div((uint32_t)site), q2 = geo.dy.div(q1), q3 = geo.dz.div(q2);
+  const int y = (int)(q1 - q2 * geo.dy.d), z = (int)(q2 - q3 * geo.dz.d), t = (int)q3;
+  const int c[4] = {2 * (int)((uint32_t)site - q1 * geo.dx.d) + ((parity + y + z + t) & 1), y, z, t};
+  double g[9];
+  switch (pl) {
+    case 0: plane_field<R>(a.gauge, geo, c, 0, 1, g); break;
+    case 1: plane_field<R>(a.gauge, geo, c, 0, 2, g); break;
+    case 2: plane_field<R>(a.gauge, geo, c, 0, 3, g); break;
+    case 3: plane_field<R>(a.gauge, geo, c, 1, 2, g); break;
+    case 4: plane_field<R>(a.gauge, geo, c, 1, 3, g); break;
+    default: plane_field<R>(a.gauge, geo, c, 2, 3, g); break;
   }
 #pragma unroll
-  for (int k = 0; k < 36; ++k) m[k] = ck * m[k];
-#pragma unroll
-  for (int i = 0; i < 6; ++i) m[i * 7].re += 1.0;
-  if (A) pack_block(m, A, vh, site, b);
-  if (Ainv) {  // the even-odd solve needs the inverse on one parity only
-    zd inv[36];
-    if (!chol_inv6(m, inv)) {
-      gj_inv6(m, inv);
-      atomicAdd(nbad, 1);
-    }
-    pack_block(inv, Ainv, vh, site, b);
-  }
+  for (int k = 0; k < 9; ++k) G[pl][k][lane] = g[k];
+  __syncthreads();
+  if (pl == 0) build_block<0>(G, lane, live, a, parity, site);
+  else if (pl == 1) build_block<1>(G, lane, live, a, parity, site);
 }
 
 // packed F64 -> F32 (18 float4 words per site) / F16 (9 uint4 words); one parity
@@ -304,13 +356,10 @@ __global__ void clover_unpack_kernel(const double2* src, double2* out, long vh) 
   }
 }
 
-void launch_clover_leaves(const void* gauge, void* G, const Geom& g, int parity, hipStream_t st) {
-  hipLaunchKernelGGL(clover_leaves_kernel, dim3(nblk(g.vh, 128), 6), dim3(128), 0, st,
-                     static_cast<const double2*>(gauge), static_cast<double2*>(G), g, parity);
-}
-void launch_clover_assemble(const void* G, void* A, void* Ainv, long vh, double ck, int* nbad, hipStream_t st) {
-  hipLaunchKernelGGL(clover_assemble_kernel, dim3(nblk(vh, 64), 2), dim3(64), 0, st, static_cast<const double2*>(G),
-                     static_cast<double2*>(A), static_cast<double2*>(Ainv), vh, ck, nbad);
+void launch_clover_build(int recon, const CloverBuild& a, hipStream_t st) {
+  const dim3 grid((a.only < 0 ? 2 : 1) * nblk(a.geo.vh, 64)), block(384);
+  if (recon == 12) hipLaunchKernelGGL(clover_build_kernel<12>, grid, block, 0, st, a);
+  else hipLaunchKernelGGL(clover_build_kernel<18>, grid, block, 0, st, a);
 }
 void launch_clover_convert(int prec, const void* src, void* dst, long vh, hipStream_t st) {
   if (prec == F32)

@@ -43,19 +43,22 @@ struct DevBuf {
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf();
-  void alloc(size_t bytes);
+  void* alloc(size_t bytes);
   void ensure(size_t bytes);
   void release();
   char* c() const { return static_cast<char*>(p); }
 };
 
-// A = 1 + ck T and A^-1, packed, per precision and parity, built on demand.  The
-// even-odd solve reads A on both parities and A^-1 on the odd one in FP64, and A_ee and
-// A^-1_oo in its inner precision; A^-1_ee (export, full-lattice compositions) is built
-// only when asked for.  Low precisions are converted from FP64.
+// Parts of a clover field a caller needs.  The full operator reads A alone; the even-odd
+// solve reads A on both parities and A^-1 on the odd one in FP64, and A_ee and A^-1_oo in
+// its inner precision; the export and the compositions with A^-1 also read A^-1_ee.
+enum CloverParts : int { CLOVER_A = 0, CLOVER_SOLVE = 1, CLOVER_ALL = 2 };
+
+// A = 1 + ck T and A^-1, packed, per precision and parity, built on demand.  Low
+// precisions are converted from FP64.
 struct CloverField {
   double ck = 0.0;
-  int nbad = 0;  // blocks inverted by the pivoted fallback, over the parities inverted so far
+  DevBuf bad;  // int: blocks inverted by the pivoted fallback, over the parities inverted so far
   long vh = 0;
   // serving slots (of every server) solving with this field; a server frees the field
   // only when this reaches zero, so servers that share a gauge never free a field
@@ -85,8 +88,8 @@ struct GaugeField {
   DevBuf packed[3][2];  // [precision][recon == 12]
   std::map<double, std::unique_ptr<CloverField>> clovers;
   const void* get(int prec, int recon);
-  // the solve's parts in F64 and prec; full_inverse adds A^-1_ee (FP64)
-  CloverField* clover(double ck, int prec, bool full_inverse = false);
+  // with `parts` in F64 and, for the solve's parts, in prec (built on the context stream)
+  CloverField* clover(double ck, int prec, CloverParts parts = CLOVER_SOLVE);
   size_t bytes() const;
 };
 

@@ -43,14 +43,14 @@ static void check_op(const qcuOperator& op) {
   QREQ(op.t_boundary == 1 || op.t_boundary == -1, "t_boundary must be +1 or -1");
 }
 
-static OpView make_view(GaugeField& g, const qcuOperator& op, int prec) {
+static OpView make_view(GaugeField& g, const qcuOperator& op, int prec, CloverParts parts) {
   check_op(op);
   OpView o;
   o.g = &g;
   o.op = op;
   o.clover = op.csw != 0.0;
   o.cf = nullptr;
-  if (o.clover) o.cf = g.clover(op.kappa * op.csw, prec, true);
+  if (o.clover) o.cf = g.clover(op.kappa * op.csw, prec, parts);
   g.get(prec, op.recon);
   g.get(F64, op.recon);
   return o;
@@ -175,7 +175,7 @@ void solve_batch(GaugeField& g, const qcuOperator& op, const qcuSolveParams& spi
 }
 
 void apply_mhat_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger, int prec) {
-  OpView o = make_view(g, op, prec);
+  OpView o = make_view(g, op, prec, CLOVER_SOLVE);
   long vh = g.geo.vh;
   Vec a = vec(ctx().buf("mh_a", spinor_bytes(prec, vh))->p);
   Vec b = vec(ctx().buf("mh_b", spinor_bytes(prec, vh))->p);
@@ -206,7 +206,7 @@ static void one_minus_ainv_d(OpView& o, int dag, const Vec in[2], const Vec out[
 
 void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger) {
   QREQ(kind >= QCU_COMP_AINV_D && kind <= QCU_COMP_NORMAL, "qcuApplyComposite: unknown kind");
-  OpView o = make_view(g, op, F64);
+  OpView o = make_view(g, op, F64, kind == QCU_COMP_A ? CLOVER_A : CLOVER_ALL);
   const long vh = g.geo.vh;
   if (kind == QCU_COMP_AINV_D) {
     IfaceHop p = {g.get(F64, op.recon), F64, op.recon, o.clover ? EPI_CLOV : EPI_PLAIN, -1, dagger ? 1 : 0, o.tbc(),
@@ -246,7 +246,7 @@ void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void*
 }
 
 void apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger) {
-  OpView o = make_view(g, op, F64);
+  OpView o = make_view(g, op, F64, CLOVER_A);
   long vh = g.geo.vh;
   IfaceHop p = {g.get(F64, op.recon), F64, op.recon, o.clover ? EPI_CLOV_XPAY : EPI_XPAY, -1, dagger, o.tbc(),
                 -op.kappa, {nullptr, nullptr}};

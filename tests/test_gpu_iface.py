@@ -101,3 +101,28 @@ def test_split_kernel_bits_equal_pinned_shape(q, L, prec):
             assert np.array_equal(a, c), (recon, csw)
         assert np.array_equal(want[1], got[1]) and want[2:] == got[2:], (recon, csw, want[2:], got[2:])
         assert want[3] <= 1e-9
+
+
+@pytest.mark.parametrize("L", LATS)
+@pytest.mark.parametrize("ck", [0.122, 1.0])
+def test_clover_built_in_parts(q, L, ck):
+    """A, the odd inverse and the even inverse built one after another, as the full
+    operator, the Schur operator and the export ask for them, have the bits of one build
+    for the export, and the oracle's values; blocks that are not positive definite (they
+    occur at ck = 1) are counted once each."""
+    vh = q.half_volume(L)
+    g = q.Gauge.random(L, seed=44, eps=0.45)
+    gref = g.to_numpy()
+    op = q.Operator(ck, 1.0, 1, 18)
+    v = orc.source_gauss(L, 9)
+    q.apply_m(g, op, v)
+    q.apply_mhat(g, op, v[0])
+    A, Ainv, nf = g.clover(ck, 1.0)
+    A1, Ainv1, nf1 = q.Gauge.from_numpy(gref, L).clover(ck, 1.0)
+    assert np.array_equal(A, A1) and np.array_equal(Ainv, Ainv1) and nf == nf1
+    Aref = orc.clover_A(orc.clover_T(gref, L, recon=18), ck)
+    inv_ref, nbad = orc.clover_invert(Aref, chol=True)
+    assert nf == nbad
+    assert np.abs(A - Aref).max() < 1e-14 * max(1.0, np.abs(Aref).max())
+    cond = np.linalg.cond(Aref.reshape(-1, 6, 6)).max()
+    assert np.abs(Ainv - inv_ref).max() < 1e-14 * cond * max(1.0, np.abs(inv_ref).max())
