@@ -128,13 +128,47 @@ size_t GaugeField::bytes() const {
   for (auto& kv : clovers)
     for (int p = 0; p < 3; ++p)
       for (int q = 0; q < 2; ++q) s += kv.second->A[p][q].n + kv.second->Ainv[p][q].n;
+  for (auto& b : spare) s += b.n;
   return s;
+}
+
+void* GaugeField::take(DevBuf& b, size_t bytes) {
+  for (auto it = spare.begin(); it != spare.end(); ++it)
+    if (it->n == bytes) {
+      b.swap(*it);
+      spare.erase(it);
+      return b.p;
+    }
+  try {
+    return b.alloc(bytes);
+  } catch (const Error& e) {
+    if (e.code != QCU_ERROR_OUT_OF_MEMORY || spare.empty()) throw;
+  }
+  spare.clear();
+  return b.alloc(bytes);
+}
+
+void GaugeField::forget_links() {
+  auto keep = [&](DevBuf& b) {
+    if (!b.p) return;
+    spare.emplace_back();
+    spare.back().swap(b);
+  };
+  for (auto& a : packed)
+    for (auto& b : a) keep(b);
+  for (auto& kv : clovers)
+    for (int p = 0; p < 3; ++p)
+      for (int q = 0; q < 2; ++q) {
+        keep(kv.second->A[p][q]);
+        keep(kv.second->Ainv[p][q]);
+      }
+  clovers.clear();
 }
 
 const void* GaugeField::get(int prec, int recon) {
   DevBuf& b = packed[prec][recon == 12 ? 1 : 0];
   if (!b.p) {
-    b.alloc(gauge_bytes(prec, recon, geo.vh));
+    take(b, gauge_bytes(prec, recon, geo.vh));
     launch_gauge_pack(prec, recon, aos.p, b.p, geo.vh, stream());
     QHIP(hipGetLastError());
   }
@@ -160,8 +194,8 @@ CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
   bool need[2];
   for (int p = 0; p < 2; ++p) {
     const bool inv = parts == CLOVER_ALL || (parts == CLOVER_SOLVE && p == 1);
-    b.A[p] = cf->A[F64][p].p ? nullptr : cf->A[F64][p].alloc(half64);
-    b.Ainv[p] = !inv || cf->Ainv[F64][p].p ? nullptr : cf->Ainv[F64][p].alloc(half64);
+    b.A[p] = cf->A[F64][p].p ? nullptr : take(cf->A[F64][p], half64);
+    b.Ainv[p] = !inv || cf->Ainv[F64][p].p ? nullptr : take(cf->Ainv[F64][p], half64);
     need[p] = b.A[p] || b.Ainv[p];
   }
   if (need[0] || need[1]) {
@@ -176,8 +210,8 @@ CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
   // inner-precision parts: A_ee and A^-1_oo
   if (parts != CLOVER_A && prec != F64 && !cf->A[prec][0].p) {
     const size_t half = clover_bytes(prec, geo.vh) / 2;
-    cf->A[prec][0].alloc(half);
-    cf->Ainv[prec][1].alloc(half);
+    take(cf->A[prec][0], half);
+    take(cf->Ainv[prec][1], half);
     launch_clover_convert(prec, cf->a(F64, 0), cf->A[prec][0].p, geo.vh, stream());
     launch_clover_convert(prec, cf->ainv(F64, 1), cf->Ainv[prec][1].p, geo.vh, stream());
     QHIP(hipGetLastError());
@@ -413,17 +447,14 @@ static uint64_t* fingerprint_host() {
 // remake the drop-in copy from the caller's gauge, whose fingerprint is fp
 static void dropin_rebuild(void* gauge, const QcuParam* param, bool same_geom, uint64_t fp) {
   Context::Dropin& d = ctx().dropin;
-  if (d.g) {
-    QHIP(hipStreamSynchronize(stream()));
-    drop_cached_batches(d.g.get());
-  }
-  if (same_geom) {  // reuse the allocation: new links, no packed copies, no clover
+  if (d.g) QHIP(hipStreamSynchronize(stream()));
+  if (same_geom) {  // new links, no packed copies, no clover, in the old allocations
     GaugeField& g = *d.g;
-    for (auto& a : g.packed)
-      for (auto& b : a) b.release();
-    g.clovers.clear();
+    unbind_cached_batches(&g);
+    g.forget_links();
     QHIP(hipMemcpyAsync(g.aos.p, gauge, g.aos.n, hipMemcpyDeviceToDevice, stream()));
   } else {
+    if (d.g) drop_cached_batches(d.g.get());
     d.g.reset();
     d.g = make_gauge_from_aos(gauge, param->lattice_size);
   }

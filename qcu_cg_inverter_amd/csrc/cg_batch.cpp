@@ -17,7 +17,7 @@ size_t CgBatch::bytes_for(long vh, int prec, int cap) {
 
 CgBatch::CgBatch(GaugeField& g, int prec, int recon, int t_boundary, bool clover, int capacity,
                  const qcuSolveParams& sp, hipStream_t st)
-    : g_(g), prec_(prec), xprec_(iterate_precision(prec)), recon_(recon), tbc_(t_boundary), clover_(clover),
+    : g_(&g), prec_(prec), xprec_(iterate_precision(prec)), recon_(recon), tbc_(t_boundary), clover_(clover),
       cap_(capacity), sp_(sp), st_(st) {
   QREQ(capacity >= 1 && capacity <= kMaxRhs, "batch capacity must be 1..16");
   QREQ(prec >= 0 && prec <= 2, "bad precision");
@@ -61,11 +61,18 @@ CgBatch::CgBatch(GaugeField& g, int prec, int recon, int t_boundary, bool clover
   scal_.alloc(sizeof(CgScal) * cap_);
   dsc_ = static_cast<CgScal*>(scal_.p);
   QHIP(hipHostMalloc((void**)&hsc_, sizeof(CgScal) * cap_, 0));
-  g.get(prec, recon);
-  g.get(F64, recon);
-  QHIP(hipStreamSynchronize(ctx().stream));  // packed fields were made on the context stream
+  rebind(g);
   const char* e = getenv("QCU_DEBUG");
   debug_ = e && e[0] && e[0] != '0';
+}
+
+void CgBatch::rebind(GaugeField& g) {
+  if (n_ != 0 || g.geo.vh != vh_) throw Error(QCU_ERROR_STATE, "internal: batch cannot change its gauge");
+  g_ = &g;
+  clear_graphs();  // they hold the old gauge's fields
+  g.get(prec_, recon_);
+  g.get(F64, recon_);
+  QHIP(hipStreamSynchronize(ctx().stream));  // packed fields were made on the context stream
 }
 
 CgBatch::~CgBatch() {
@@ -119,9 +126,9 @@ void CgBatch::mhat(int prec, int dag, Vec in, Vec out, Vec tmp, int r0, int n, d
     k1[j] = 1.0;
     k2[j] = -sl.spec.kappa * sl.spec.kappa;
   }
-  hop_v(g_, prec, recon_, clover_ ? EPI_CLOV : EPI_PLAIN, 1, dag, (double)tbc_, at(in, r0), at(tmp, r0), vec(nullptr),
+  hop_v(*g_, prec, recon_, clover_ ? EPI_CLOV : EPI_PLAIN, 1, dag, (double)tbc_, at(in, r0), at(tmp, r0), vec(nullptr),
         c1, k1, n, nullptr, st_);
-  hop_v(g_, prec, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 0, dag, (double)tbc_, at(tmp, r0), at(out, r0),
+  hop_v(*g_, prec, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 0, dag, (double)tbc_, at(tmp, r0), at(out, r0),
         at(in, r0), c2, k2, n, partials ? partials + (long)r0 * nw_ : nullptr, st_);
 }
 
@@ -140,8 +147,8 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
     sl.updates = 0;
     sl.cf = nullptr;
     if (clover_) {
-      sl.cf = g_.clover(sl.spec.kappa * sl.spec.csw, F64);
-      if (prec_ != F64) g_.clover(sl.spec.kappa * sl.spec.csw, prec_);
+      sl.cf = g_->clover(sl.spec.kappa * sl.spec.csw, F64);
+      if (prec_ != F64) g_->clover(sl.spec.kappa * sl.spec.csw, prec_);
     }
     if (sl.spec.max_iter <= 0) sl.spec.max_iter = (int)std::min<long>(20 * vh_, 1000000);
     slots_.push_back(sl);
@@ -182,7 +189,7 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
       lo = hi + 1;
     }
   }
-  hop_v(g_, F64, recon_, EPI_XPAY, 0, 0, (double)tbc_, at(t64_, r0), at(bh_, r0), at(shi_, r0), none, kap, m,
+  hop_v(*g_, F64, recon_, EPI_XPAY, 0, 0, (double)tbc_, at(t64_, r0), at(bh_, r0), at(shi_, r0), none, kap, m,
         nullptr, st_);
   launch_zero(F64, at(xe_, r0), vh_, m, st_);
   for (int r = r0; r <= r1; ++r)
@@ -409,21 +416,21 @@ void CgBatch::finish_run(int lo, int hi, std::vector<double>& nr) {
                            1, st_);
   // x_o = A_oo^-1 (b_o + kappa D_oe x_e)
   if (clover_) {
-    hop_v(g_, F64, recon_, EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), tmp, bq, none, kap, m, nullptr, st_);
+    hop_v(*g_, F64, recon_, EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), tmp, bq, none, kap, m, nullptr, st_);
     for (int r = lo; r <= hi; ++r)
       launch_clover_apply(F64, slots_[r].cf->ainv(F64, 1), at(bh_, r), at(shi_, r), vh_, 1, st_);
   } else {
-    hop_v(g_, F64, recon_, EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), xo, bq, none, kap, m, nullptr, st_);
+    hop_v(*g_, F64, recon_, EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), xo, bq, none, kap, m, nullptr, st_);
   }
   // r = b - M x with M = A - kappa D, odd then even parity
   std::vector<double> ro(m), re(m);
-  hop_v(g_, F64, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), tmp, xo,
+  hop_v(*g_, F64, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), tmp, xo,
         clover_ ? a_o : none, mkap, m, nullptr, st_);
   launch_axpby(F64, 1.0, bq, -1.0, tmp, vh_, m, st_);
   norm2_run(bh_, lo, hi, ro.data());
   for (int r = lo; r <= hi; ++r)  // b_e
     launch_spinor_from_aos(F64, source_aos(slots_[r]), 0, at(t64_, r), vh_, 1, st_);
-  hop_v(g_, F64, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 0, 0, (double)tbc_, xo, tmp, at(xe_, lo),
+  hop_v(*g_, F64, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 0, 0, (double)tbc_, xo, tmp, at(xe_, lo),
         clover_ ? a_e : none, mkap, m, nullptr, st_);
   launch_axpby(F64, 1.0, bq, -1.0, tmp, vh_, m, st_);
   for (int r = lo; r <= hi; ++r) {

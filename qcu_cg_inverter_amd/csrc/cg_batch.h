@@ -47,11 +47,13 @@ class CgBatch {
   CgBatch& operator=(const CgBatch&) = delete;
 
   static size_t bytes_for(long vh, int prec, int capacity);
-  size_t bytes() const { return bytes_for(g_.geo.vh, prec_, cap_); }
+  size_t bytes() const { return bytes_for(vh_, prec_, cap_); }
   int capacity() const { return cap_; }
   int active() const { return n_; }
   int free_slots() const { return cap_ - n_; }
-  GaugeField& gauge() { return g_; }
+  GaugeField& gauge() { return *g_; }
+  // the same workspace for another gauge on the same lattice (no active slots)
+  void rebind(GaugeField& g);
   bool clover() const { return clover_; }
   int precision() const { return prec_; }
 
@@ -93,7 +95,7 @@ class CgBatch {
   double norm2_slot(Vec v, int r);
   void clear_graphs();
 
-  GaugeField& g_;
+  GaugeField* g_;
   int prec_, xprec_, recon_, tbc_;
   bool clover_;
   int cap_, n_ = 0;

@@ -1,6 +1,7 @@
 // qcu_host.h -- host-side runtime of libqcu.so: context, resident fields, errors.
 #pragma once
 
+#include <list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -46,6 +47,10 @@ struct DevBuf {
   void* alloc(size_t bytes);
   void ensure(size_t bytes);
   void release();
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+  }
   char* c() const { return static_cast<char*>(p); }
 };
 
@@ -87,6 +92,14 @@ struct GaugeField {
   DevBuf aos;
   DevBuf packed[3][2];  // [precision][recon == 12]
   std::map<double, std::unique_ptr<CloverField>> clovers;
+  // Allocations of the fields dropped by forget_links, for the next ones of their size: a
+  // drop-in gauge that changes remakes the same fields, and freeing and allocating one of
+  // 76 MB takes 265 us, several times what its kernel takes.  At most what this gauge
+  // held before; freed with it.
+  std::list<DevBuf> spare;
+  void* take(DevBuf& b, size_t bytes);  // b (empty) gets a spare of that size, or a new allocation
+  // drop every packed and clover field, keeping the allocations; the context stream is idle
+  void forget_links();
   const void* get(int prec, int recon);
   // with `parts` in F64 and, for the solve's parts, in prec (built on the context stream)
   CloverField* clover(double ck, int prec, CloverParts parts = CLOVER_SOLVE);
@@ -188,6 +201,8 @@ void solve_batch(GaugeField& g, const qcuOperator& op, const qcuSolveParams& sp,
 void apply_mhat_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger, int prec);
 // forget solver state that refers to gauge g (all gauges if null)
 void drop_cached_batches(GaugeField* g);
+// the fields of g changed: the next solve takes them up again, in the same workspace
+void unbind_cached_batches(GaugeField* g);
 void apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger);
 void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger);
 

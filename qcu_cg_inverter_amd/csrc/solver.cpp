@@ -78,10 +78,12 @@ static void full_op_parity(OpView& o, int p, int dag, Vec in_p, Vec in_q, Vec ou
     hop(*o.g, F64, o.op.recon, EPI_XPAY, p, dag, o.tbc(), in_q, out, in_p, nullptr, -o.op.kappa, 1, nullptr, st);
 }
 
-// A batch object kept between calls so repeated solves of the same shape reuse
-// their device buffers and captured graphs' allocations.
+// A batch object kept between calls, so repeated solves of the same shape reuse its device
+// buffers, also for another gauge of the same lattice (a 16^3x32 batch is seven
+// allocations, about 1 ms to free and make again).  Dropped with the gauge it last served.
 struct CachedBatch {
   GaugeField* g = nullptr;
+  int L[4] = {0, 0, 0, 0};
   int prec = -1, recon = 0, tbc = 0, clover = -1, cap = 0, chunk = 0, graph = -1;
   double delta = 0.0;
   std::unique_ptr<CgBatch> batch;
@@ -95,14 +97,19 @@ void drop_cached_batches(GaugeField* g) {
   }
 }
 
+void unbind_cached_batches(GaugeField* g) {
+  if (g_cached.g == g) g_cached.g = nullptr;
+}
+
 static CgBatch& batch_for(GaugeField& g, int prec, const qcuOperator& op, int nrhs, const qcuSolveParams& sp) {
   CachedBatch& c = g_cached;
   const int clov = op.csw != 0.0;
-  if (!c.batch || c.g != &g || c.prec != prec || c.recon != op.recon || c.tbc != op.t_boundary || c.clover != clov ||
-      c.cap != nrhs || c.chunk != sp.chunk || c.graph != sp.graph || c.delta != sp.delta) {
-    c.batch.reset();
+  if (!c.batch || memcmp(c.L, g.L, sizeof c.L) != 0 || c.prec != prec || c.recon != op.recon ||
+      c.tbc != op.t_boundary || c.clover != clov || c.cap != nrhs || c.chunk != sp.chunk || c.graph != sp.graph ||
+      c.delta != sp.delta) {
+    drop_cached_batches(nullptr);
     c.batch.reset(new CgBatch(g, prec, op.recon, op.t_boundary, clov != 0, nrhs, sp, stream()));
-    c.g = &g;
+    memcpy(c.L, g.L, sizeof c.L);
     c.prec = prec;
     c.recon = op.recon;
     c.tbc = op.t_boundary;
@@ -111,7 +118,11 @@ static CgBatch& batch_for(GaugeField& g, int prec, const qcuOperator& op, int nr
     c.chunk = sp.chunk;
     c.graph = sp.graph;
     c.delta = sp.delta;
+  } else if (c.g != &g) {
+    c.g = nullptr;  // a rebind that throws is tried again by the next solve
+    c.batch->rebind(g);
   }
+  c.g = &g;
   return *c.batch;
 }
 

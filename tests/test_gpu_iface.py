@@ -126,3 +126,28 @@ def test_clover_built_in_parts(q, L, ck):
     assert np.abs(A - Aref).max() < 1e-14 * max(1.0, np.abs(Aref).max())
     cond = np.linalg.cond(Aref.reshape(-1, 6, 6)).max()
     assert np.abs(Ainv - inv_ref).max() < 1e-14 * cond * max(1.0, np.abs(inv_ref).max())
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_solves_alternate_gauges(q, prec):
+    """Solves that go back and forth between gauges, one of another lattice with the same
+    half volume, share a workspace where the lattice is the same; each gives the bits of
+    a solve on a gauge of its own, also after the other gauge is gone."""
+    b = {L: orc.source_gauss(L, 12) for L in ((8, 4, 8, 8), (4, 8, 8, 8))}
+    sp = q.default_solve_params(tol=1e-10, precision=prec)
+    op = q.Operator(0.12, 1.0, -1, 12)
+
+    def make(k):
+        L = (4, 8, 8, 8) if k == 2 else (8, 4, 8, 8)
+        return q.Gauge.random(L, seed=50 + k, eps=0.2)
+
+    alone = {}
+    for k in range(3):
+        g = make(k)
+        alone[k] = q.solve(g, op, b[g.L], sp)[0]
+        g.destroy()
+    gs = [make(k) for k in range(3)]
+    for k in (0, 1, 0, 2, 1, 0):
+        assert np.array_equal(q.solve(gs[k], op, b[gs[k].L], sp)[0], alone[k]), k
+    gs[1].destroy()
+    assert np.array_equal(q.solve(gs[0], op, b[gs[0].L], sp)[0], alone[0])
