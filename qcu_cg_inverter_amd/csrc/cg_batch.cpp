@@ -228,17 +228,21 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
 void CgBatch::launch_chunk() {
   const int n = n_;
   if (n == 0) return;
-  auto iteration = [&]() {
+  // few partials: the vector kernels take the scalar steps, six launches an iteration
+  // instead of nine; the last iteration's |s|^2 is looked at by the one-block kernel
+  const bool in_step = cg_step_chains(nw_, n) != 0;
+  auto iteration = [&](int i) {
     mhat(prec_, 1, S_, R_, TO_, 0, n, part_rr_);
-    launch_cg_beta(part_rr_, nw_, dsc_, n, st_);
-    launch_cg_xpay(prec_, xprec_, R_, P_, X_, dsc_, vh_, n, st_);
+    if (!in_step) launch_cg_beta(part_rr_, nw_, dsc_, n, st_);
+    launch_cg_xpay(prec_, xprec_, R_, P_, X_, dsc_, in_step ? part_rr_ : nullptr, i > 0 ? part_ss_ : nullptr, nw_,
+                   vh_, n, st_);
     mhat(prec_, 0, P_, T_, TO_, 0, n, part_tt_);
-    launch_cg_alpha(part_tt_, nw_, dsc_, n, st_);
-    launch_cg_update(prec_, T_, S_, dsc_, part_ss_, vh_, n, st_);
-    launch_cg_ss(part_ss_, nw_, dsc_, n, st_);
+    if (!in_step) launch_cg_alpha(part_tt_, nw_, dsc_, n, st_);
+    launch_cg_update(prec_, T_, S_, dsc_, in_step ? part_tt_ : nullptr, nw_, part_ss_, vh_, n, st_);
+    if (!in_step || i == sp_.chunk - 1) launch_cg_ss(part_ss_, nw_, dsc_, n, st_);
   };
   if (!sp_.graph) {
-    for (int i = 0; i < sp_.chunk; ++i) iteration();
+    for (int i = 0; i < sp_.chunk; ++i) iteration(i);
     QHIP(hipGetLastError());
     return;
   }
@@ -246,7 +250,7 @@ void CgBatch::launch_chunk() {
   auto& gr = graphs_[n];
   if (!gr.second) {
     QHIP(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < sp_.chunk; ++i) iteration();
+    for (int i = 0; i < sp_.chunk; ++i) iteration(i);
     QHIP(hipStreamEndCapture(st_, &gr.first));
     QHIP(hipGraphInstantiate(&gr.second, gr.first, nullptr, nullptr, 0));
   }

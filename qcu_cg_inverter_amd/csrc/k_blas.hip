@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(kSumThreads) cg_alpha_kernel(const double* par
     } else {
       s.alpha = s.gamma / tt;
     }
+    s.gamma_old = s.gamma;  // for a later chunk whose vector kernels take the steps
   }
 }
 
@@ -174,113 +175,223 @@ __global__ void __launch_bounds__(kSumThreads) cg_ss_kernel(const double* part, 
   }
 }
 
+// The sum of a right-hand side's nw partials, by every block that needs it (256 threads, nw
+// <= 1024 K), with the bits of block_sum_partials: thread u stands for its threads u + 256
+// q, whose chains beyond K are empty, and the sixteen wave sums are added in its order.
+constexpr int kStepThreads = 256;
+template <int K>
+__device__ __forceinline__ double step_sum(const double* part, long nw, double* red) {
+  double v[kSumThreads / kStepThreads];
+#pragma unroll
+  for (int q = 0; q < kSumThreads / kStepThreads; ++q) {
+    double c[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const long j = (long)threadIdx.x + q * kStepThreads + (long)k * kSumThreads;
+      c[k] = j < nw ? part[j] : 0.0;
+    }
+#pragma unroll
+    for (int h = K / 2; h >= 1; h >>= 1)
+#pragma unroll
+      for (int k = 0; k < h; ++k) c[k] += c[k + h];
+    v[q] = c[0];
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+    for (int q = 0; q < kSumThreads / kStepThreads; ++q) v[q] += __shfl_xor(v[q], off, 64);
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < kSumThreads / kStepThreads; ++q) red[(threadIdx.x >> 6) + q * (kStepThreads / 64)] = v[q];
+  }
+  __syncthreads();
+  double sum = 0.0;
+#pragma unroll
+  for (int k = 0; k < kSumThreads / 64; ++k) sum += red[k];
+  return sum;
+}
+
+// The beta step by every block of the p update: the sums of |r|^2 and, when the previous
+// iteration's |s|^2 is still to be looked at (part_ss), of that; block 0 writes what the
+// later steps read.  Nothing another block reads here is written here.
+template <int K>
+__device__ __forceinline__ double beta_step(CgScal& s, const double* part_rr, const double* part_ss, long nw,
+                                            double (*red)[kSumThreads / 64]) {
+  const double rr = step_sum<K>(part_rr, nw, red[0]);
+  int conv = s.converged;
+  double ss = 0.0;
+  if (part_ss) {
+    ss = step_sum<K>(part_ss, nw, red[1]);
+    conv = conv || ss <= s.target2;
+  }
+  const double beta = s.first || conv || !(s.gamma_old > 0.0) ? 0.0 : rr / s.gamma_old;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (part_ss && !s.converged) {
+      s.ss = ss;
+      s.iter += 1;
+    }
+    s.conv_now = conv;
+    s.beta = beta;
+    s.gamma = rr;
+  }
+  return beta;
+}
+
+// the alpha step by every block of the s update, likewise
+template <int K>
+__device__ __forceinline__ double alpha_step(CgScal& s, const double* part_tt, long nw, double* red) {
+  const double tt = step_sum<K>(part_tt, nw, red);
+  const double g = s.gamma;
+  const bool conv = s.conv_now, bad = !conv && (!(tt > 0.0) || g != g || tt != tt || tt > 1.0e300);
+  const double alpha = conv || bad ? 0.0 : g / tt;  // breakdown freezes, as in cg_alpha_kernel
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    s.tt = tt;
+    s.alpha = alpha;
+    if (bad) s.breakdown = 1;
+    s.converged = conv;
+    s.gamma_old = g;
+    s.first = 0;
+  }
+  return alpha;
+}
+
 // x += alpha_k p_k of the previous iteration (still pending: alpha is that iteration's,
 // p not yet overwritten), then p = r + beta p.  Folding the iterate update in here
 // saves one read of p per iteration against doing it in the s update; the host
-// applies a pending update itself (cg_xflush) before it reads x.
-template <int P, int PX>
-__global__ void cg_xpay_kernel(Vec r, Vec p, Vec x, const CgScal* sc, long vh, int nts) {
+// applies a pending update itself (cg_xflush) before it reads x.  K > 0: the blocks take
+// the beta step themselves (beta_step), while their first fields load.
+template <int P, int PX, int K>
+__global__ void __launch_bounds__(256) cg_xpay_kernel(Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr,
+                                                      const double* part_ss, long nw, long vh, int nts) {
   using T = typename Real<P>::T;
   using TX = typename Real<PX>::T;
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int k = blockIdx.y;
-  if (i >= vh || !sc[k].active) return;
+  __shared__ double red[K ? 2 : 1][kSumThreads / 64];
+  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = blockIdx.y;
+  if (!sc[k].active) return;
+  if (K == 0 && i0 >= vh) return;
+  const bool live = i0 < vh;
+  const long i = live ? i0 : vh - 1;
   const double alpha = sc[k].alpha;
-  const T beta = T(sc[k].beta);
   char* pp = static_cast<char*>(p.p) + k * p.stride;
   char* xp = static_cast<char*>(x.p) + k * x.stride;
   const char* rp = static_cast<const char*>(r.p) + k * r.stride;
-  if (P == F64 && PX == F64) {
+  if constexpr (P == F64 && PX == F64) {
     // FP64 in halves of 6 components (p, r and x at once would spill)
+    cx<double> pv[6], rv[6], xv[6];
+    double beta = K ? 1.0 : sc[k].beta;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      cx<double> pv[6], rv[6];
-      if (alpha != 0.0 || beta != T(0)) SpinorIO<F64>::load_half<1>(pp, vh, i, h, pv);
+      if (alpha != 0.0 || beta != 0.0) SpinorIO<F64>::load_half<1>(pp, vh, i, h, pv);
+      if (alpha != 0.0) SpinorIO<F64>::load_half<1>(xp, vh, i, h, xv);
+      SpinorIO<F64>::load_half<1>(rp, vh, i, h, rv);
+      if constexpr (K > 0)
+        if (h == 0) beta = beta_step<K>(sc[k], part_rr + k * nw, part_ss ? part_ss + k * nw : nullptr, nw, red);
       if (alpha != 0.0) {
-        cx<double> xv[6];
-        SpinorIO<F64>::load_half<1>(xp, vh, i, h, xv);
 #pragma unroll
         for (int c = 0; c < 6; ++c) xv[c] = {xv[c].re + alpha * pv[c].re, xv[c].im + alpha * pv[c].im};
-        if (nts) SpinorIO<F64>::store_half<1>(xp, vh, i, h, xv);
-        else SpinorIO<F64>::store_half<0>(xp, vh, i, h, xv);
+        if (live) {
+          if (nts) SpinorIO<F64>::store_half<1>(xp, vh, i, h, xv);
+          else SpinorIO<F64>::store_half<0>(xp, vh, i, h, xv);
+        }
       }
-      SpinorIO<F64>::load_half<1>(rp, vh, i, h, rv);
-      if (beta != T(0)) {
+      if (beta != 0.0) {
 #pragma unroll
-        for (int c = 0; c < 6; ++c) rv[c] = rv[c] + (double)beta * pv[c];
+        for (int c = 0; c < 6; ++c) rv[c] = rv[c] + beta * pv[c];
       }
-      if (nts) SpinorIO<F64>::store_half<1>(pp, vh, i, h, rv);
-      else SpinorIO<F64>::store_half<0>(pp, vh, i, h, rv);
+      if (live) {
+        if (nts) SpinorIO<F64>::store_half<1>(pp, vh, i, h, rv);
+        else SpinorIO<F64>::store_half<0>(pp, vh, i, h, rv);
+      }
     }
-    return;
-  }
-  cx<T> pv[12];
-  if (alpha != 0.0 || beta != T(0)) SpinorIO<P>::load(pp, vh, i, pv);
-  if (alpha != 0.0) {
-    const TX ax = TX(alpha);
-    cx<TX> xv[12];
-    SpinorIO<PX>::load(xp, vh, i, xv);
-#pragma unroll
-    for (int c = 0; c < 12; ++c) xv[c] = {xv[c].re + ax * TX(pv[c].re), xv[c].im + ax * TX(pv[c].im)};
-    if (nts) SpinorIO<PX>::template store<1>(xp, vh, i, xv);
-    else SpinorIO<PX>::template store<0>(xp, vh, i, xv);
-  }
-  cx<T> rv[12];
-  SpinorIO<P>::load(rp, vh, i, rv);
-  if (beta == T(0)) {
-    // restart (first iteration, after a restart, or converged): p = r
-#pragma unroll
-    for (int c = 0; c < 12; ++c) pv[c] = rv[c];
   } else {
+    cx<T> pv[12], rv[12];
+    cx<TX> xv[12];
+    T beta = K ? T(1) : T(sc[k].beta);
+    if (alpha != 0.0 || beta != T(0)) SpinorIO<P>::load(pp, vh, i, pv);
+    if constexpr (K > 0) {
+      if (alpha != 0.0) SpinorIO<PX>::load(xp, vh, i, xv);
+      SpinorIO<P>::load(rp, vh, i, rv);
+      beta = T(beta_step<K>(sc[k], part_rr + k * nw, part_ss ? part_ss + k * nw : nullptr, nw, red));
+    }
+    if (alpha != 0.0) {
+      const TX ax = TX(alpha);
+      if (K == 0) SpinorIO<PX>::load(xp, vh, i, xv);
 #pragma unroll
-    for (int c = 0; c < 12; ++c) pv[c] = rv[c] + beta * pv[c];
+      for (int c = 0; c < 12; ++c) xv[c] = {xv[c].re + ax * TX(pv[c].re), xv[c].im + ax * TX(pv[c].im)};
+      if (live) {
+        if (nts) SpinorIO<PX>::template store<1>(xp, vh, i, xv);
+        else SpinorIO<PX>::template store<0>(xp, vh, i, xv);
+      }
+    }
+    if (K == 0) SpinorIO<P>::load(rp, vh, i, rv);
+    if (beta == T(0)) {
+      // restart (first iteration, after a restart, or converged): p = r
+#pragma unroll
+      for (int c = 0; c < 12; ++c) pv[c] = rv[c];
+    } else {
+#pragma unroll
+      for (int c = 0; c < 12; ++c) pv[c] = rv[c] + beta * pv[c];
+    }
+    if (live) {
+      if (nts) SpinorIO<P>::template store<1>(pp, vh, i, pv);
+      else SpinorIO<P>::template store<0>(pp, vh, i, pv);
+    }
   }
-  if (nts) SpinorIO<P>::template store<1>(pp, vh, i, pv);
-  else SpinorIO<P>::template store<0>(pp, vh, i, pv);
 }
 
-// s -= alpha t, with the 16-site partials of |s|^2
-template <int P>
-__global__ void cg_update_kernel(Vec t, Vec s, const CgScal* sc, double* part, long vh, int nts) {
+// s -= alpha t, with the 16-site partials of |s|^2.  K > 0: the blocks take the alpha step
+// themselves (alpha_step), while their fields load.
+template <int P, int K>
+__global__ void __launch_bounds__(256) cg_update_kernel(Vec t, Vec s, CgScal* sc, const double* part_tt, long nw,
+                                                        double* part, long vh, int nts) {
   using T = typename Real<P>::T;
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int k = blockIdx.y;
+  __shared__ double red[kSumThreads / 64];
+  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = blockIdx.y;
   if (!sc[k].active) return;
-  double acc = 0.0;
-  if (i < vh) {
-    const T a = T(sc[k].alpha);
-    char* sp = static_cast<char*>(s.p) + k * s.stride;
-    const char* tp = static_cast<const char*>(t.p) + k * t.stride;
-    T n = T(0);
-    if (P == F64) {
+  const bool live = i0 < vh;
+  const long i = live ? i0 : vh - 1;
+  char* sp = static_cast<char*>(s.p) + k * s.stride;
+  const char* tp = static_cast<const char*>(t.p) + k * t.stride;
+  T n = T(0);
+  if constexpr (P == F64) {
+    double a = K ? 0.0 : sc[k].alpha;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        cx<double> tv[6], sv[6];
-        SpinorIO<F64>::load_half<1>(tp, vh, i, h, tv);
-        SpinorIO<F64>::load_half<1>(sp, vh, i, h, sv);
+    for (int h = 0; h < 2; ++h) {
+      cx<double> tv[6], sv[6];
+      SpinorIO<F64>::load_half<1>(tp, vh, i, h, tv);
+      SpinorIO<F64>::load_half<1>(sp, vh, i, h, sv);
+      if constexpr (K > 0)
+        if (h == 0) a = alpha_step<K>(sc[k], part_tt + k * nw, nw, red);
 #pragma unroll
-        for (int c = 0; c < 6; ++c) {
-          sv[c] = sv[c] - (double)a * tv[c];
-          n += T(norm2(sv[c]));
-        }
-        if (nts) SpinorIO<F64>::store_half<1>(sp, vh, i, h, sv);
-        else SpinorIO<F64>::store_half<0>(sp, vh, i, h, sv);
-      }
-    } else {
-      cx<T> tv[12], sv[12];
-      SpinorIO<P>::load(tp, vh, i, tv);
-      SpinorIO<P>::load(sp, vh, i, sv);
-#pragma unroll
-      for (int c = 0; c < 12; ++c) {
+      for (int c = 0; c < 6; ++c) {
         sv[c] = sv[c] - a * tv[c];
         n += norm2(sv[c]);
       }
+      if (live) {
+        if (nts) SpinorIO<F64>::store_half<1>(sp, vh, i, h, sv);
+        else SpinorIO<F64>::store_half<0>(sp, vh, i, h, sv);
+      }
+    }
+  } else {
+    cx<T> tv[12], sv[12];
+    SpinorIO<P>::load(tp, vh, i, tv);
+    SpinorIO<P>::load(sp, vh, i, sv);
+    T a;
+    if constexpr (K > 0) a = T(alpha_step<K>(sc[k], part_tt + k * nw, nw, red));
+    else a = T(sc[k].alpha);
+#pragma unroll
+    for (int c = 0; c < 12; ++c) {
+      sv[c] = sv[c] - a * tv[c];
+      n += norm2(sv[c]);
+    }
+    if (live) {
       if (nts) SpinorIO<P>::template store<1>(sp, vh, i, sv);
       else SpinorIO<P>::template store<0>(sp, vh, i, sv);
     }
-    acc = (double)n;
   }
-  put_partial(part, vh, k, i, acc);
+  put_partial(part, vh, k, i0, live ? (double)n : 0.0);
 }
 
 // x += alpha p for one slot: a pending iterate update applied by the host
@@ -346,14 +457,31 @@ void launch_cg_alpha(const double* part, long nw, CgScal* sc, int nrhs, hipStrea
 void launch_cg_ss(const double* part, long nw, CgScal* sc, int nrhs, hipStream_t st) {
   hipLaunchKernelGGL(cg_ss_kernel, dim3(nrhs), dim3(kSumThreads), 0, st, part, nw, sc);
 }
-void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, const CgScal* sc, long vh, int nrhs, hipStream_t st) {
-  dim3 g(nblk(vh, 256), nrhs), b(256);
-  const int n = nt_store(prec, vh, nrhs);  // p decides for x as well
-  if (prec == F64) hipLaunchKernelGGL((cg_xpay_kernel<F64, F64>), g, b, 0, st, r, p, x, sc, vh, n);
-  else if (prec == F32 && xprec == F64) hipLaunchKernelGGL((cg_xpay_kernel<F32, F64>), g, b, 0, st, r, p, x, sc, vh, n);
-  else if (prec == F32) hipLaunchKernelGGL((cg_xpay_kernel<F32, F32>), g, b, 0, st, r, p, x, sc, vh, n);
-  else if (xprec == F64) hipLaunchKernelGGL((cg_xpay_kernel<F16, F64>), g, b, 0, st, r, p, x, sc, vh, n);
-  else hipLaunchKernelGGL((cg_xpay_kernel<F16, F32>), g, b, 0, st, r, p, x, sc, vh, n);
+// Every block sums all the partials, which costs nrhs nw^2 reads and saves two one-block
+// launches and most of a third, about 13 us an iteration of one right-hand side.  Solves
+// with the steps apart and in the vector kernels (ms): 8^4 FP32 2.61 / 2.27, 16^3x32 FP64
+// 10.87 / 10.26, FP32 6.74 / 5.98, 6 RHS 19.6 / 18.7; 16^3x64 (nw 8192) FP32 11.8 / 11.0 but
+// 6 RHS, at nrhs nw^2 = 4e8, 42.6 / 43.2.
+int cg_step_chains(long nw, int nrhs) {
+  if (nw > 8 * kSumThreads || nrhs * nw * nw > 250000000) return 0;
+  return nw <= 4 * kSumThreads ? 4 : 8;
+}
+
+template <int P, int PX>
+static void xpay(Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr, const double* part_ss, long nw, long vh,
+                 int nrhs, hipStream_t st) {
+  const dim3 g(nblk(vh, 256), nrhs), b(256);
+  const int n = nt_store(P, vh, nrhs);  // p decides for x as well
+  const int k = part_rr ? cg_step_chains(nw, nrhs) : 0;
+  if (k == 4) hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 4>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
+  else if (k) hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 8>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
+  else hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 0>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
+}
+void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr,
+                    const double* part_ss, long nw, long vh, int nrhs, hipStream_t st) {
+  if (prec == F64) xpay<F64, F64>(r, p, x, sc, part_rr, part_ss, nw, vh, nrhs, st);
+  else if (prec == F32) xpay<F32, F32>(r, p, x, sc, part_rr, part_ss, nw, vh, nrhs, st);
+  else xpay<F16, F32>(r, p, x, sc, part_rr, part_ss, nw, vh, nrhs, st);
 }
 void launch_cg_xflush(int prec, int xprec, Vec x, Vec p, double alpha, long vh, hipStream_t st) {
   dim3 g(nblk(vh, 256)), b(256);
@@ -363,9 +491,21 @@ void launch_cg_xflush(int prec, int xprec, Vec x, Vec p, double alpha, long vh, 
   else if (xprec == F64) hipLaunchKernelGGL((cg_xflush_kernel<F16, F64>), g, b, 0, st, x, p, alpha, vh);
   else hipLaunchKernelGGL((cg_xflush_kernel<F16, F32>), g, b, 0, st, x, p, alpha, vh);
 }
-void launch_cg_update(int prec, Vec t, Vec s, const CgScal* sc, double* part, long vh, int nrhs, hipStream_t st) {
-  QCU_PSW(prec, cg_update_kernel, dim3(nblk(vh, 256), nrhs), dim3(256), 0, st, t, s, sc, part, vh,
-          nt_store(prec, vh, nrhs));
+template <int P>
+static void update(Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part, long vh, int nrhs,
+                   hipStream_t st) {
+  const dim3 g(nblk(vh, 256), nrhs), b(256);
+  const int n = nt_store(P, vh, nrhs);
+  const int k = part_tt ? cg_step_chains(nw, nrhs) : 0;
+  if (k == 4) hipLaunchKernelGGL((cg_update_kernel<P, 4>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
+  else if (k) hipLaunchKernelGGL((cg_update_kernel<P, 8>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
+  else hipLaunchKernelGGL((cg_update_kernel<P, 0>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
+}
+void launch_cg_update(int prec, Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part_ss, long vh,
+                      int nrhs, hipStream_t st) {
+  if (prec == F64) update<F64>(t, s, sc, part_tt, nw, part_ss, vh, nrhs, st);
+  else if (prec == F32) update<F32>(t, s, sc, part_tt, nw, part_ss, vh, nrhs, st);
+  else update<F16>(t, s, sc, part_tt, nw, part_ss, vh, nrhs, st);
 }
 
 }  // namespace qcu

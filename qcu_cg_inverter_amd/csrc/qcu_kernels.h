@@ -56,7 +56,9 @@ void launch_spinor_convert(int pin, Vec in, int pout, Vec out, long vh, int nrhs
 // per-right-hand-side CG scalars kept in device memory
 struct CgScal {
   double alpha, beta, gamma, tt, ss, target2, ss_ref;
-  int first, converged, active, breakdown, iter, pad;
+  double gamma_old;  // |r|^2 of the iteration before, where the vector kernels take the steps
+  int first, converged, active, breakdown, iter;
+  int conv_now;      // converged, as the beta step of the iteration saw it
 };
 
 void launch_zero(int prec, Vec v, long vh, int nrhs, hipStream_t st);
@@ -75,11 +77,17 @@ void launch_clover_apply(int prec, const void* clov, Vec in, Vec out, long vh, i
 void launch_cg_beta(const double* part_rr, long nw, CgScal* sc, int nrhs, hipStream_t st);
 void launch_cg_alpha(const double* part_tt, long nw, CgScal* sc, int nrhs, hipStream_t st);
 void launch_cg_ss(const double* part_ss, long nw, CgScal* sc, int nrhs, hipStream_t st);
+// nonzero: nrhs right-hand sides of nw partials take their scalar steps inside the vector
+// kernels below (pass the partials); 0: by the one-block kernels above, before them
+int cg_step_chains(long nw, int nrhs);
 // x += alpha p with the alpha and p of the previous iteration (pending until here), then
-// p = r + beta p
-void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, const CgScal* sc, long vh, int nrhs, hipStream_t st);
-// s -= alpha t ; partials of |s|^2
-void launch_cg_update(int prec, Vec t, Vec s, const CgScal* sc, double* part_ss, long vh, int nrhs, hipStream_t st);
+// p = r + beta p.  With part_rr (|r|^2) the blocks take the beta step themselves, and with
+// part_ss they also look at the |s|^2 that the previous iteration left.
+void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr,
+                    const double* part_ss, long nw, long vh, int nrhs, hipStream_t st);
+// s -= alpha t ; partials of |s|^2.  With part_tt (|t|^2) the blocks take the alpha step.
+void launch_cg_update(int prec, Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part_ss, long vh,
+                      int nrhs, hipStream_t st);
 // x += alpha p for one right-hand side (a pending iterate update, applied by the host)
 void launch_cg_xflush(int prec, int xprec, Vec x, Vec p, double alpha, long vh, hipStream_t st);
 

@@ -151,3 +151,26 @@ def test_solves_alternate_gauges(q, prec):
         assert np.array_equal(q.solve(gs[k], op, b[gs[k].L], sp)[0], alone[k]), k
     gs[1].destroy()
     assert np.array_equal(q.solve(gs[0], op, b[gs[0].L], sp)[0], alone[0])
+
+
+def test_scalar_steps_change_kernels_mid_solve(q):
+    """Sixteen right-hand sides on 16^3x32, checked after every iteration: 16 and 15 take
+    their scalar steps in one-block kernels, 14 and fewer in the vector kernels.  Point
+    and Gaussian sources converge at different iterations, so the solve goes from one to
+    the other; each right-hand side keeps the bits and iterations of its solve alone."""
+    L = (16, 16, 16, 32)
+    g = q.Gauge.random(L, seed=45, eps=0.2)
+    op = q.Operator(0.115, 0.0, -1, 12)
+    sp = q.default_solve_params(tol=1e-8, precision=1, chunk=1)
+    bs = [q.source_point_device(L, (r, 1, 2, 2 * r), r % 4, r % 3) if r % 3 == 0 else q.source_gaussian_device(L, 60 + r)
+          for r in range(16)]
+    vh = q.half_volume(L)
+    xs = [q.DeviceBuffer(2 * vh * 192) for _ in bs]
+    sts = q.solve_batch_device(g, op, xs, bs, sp)
+    its = [s.iterations for s in sts]
+    assert len(set(its)) >= 2, its
+    xa = q.DeviceBuffer(2 * vh * 192)
+    for r in range(16):
+        sa = q.solve_batch_device(g, op, [xa], [bs[r]], sp)[0]
+        assert sa.converged and sa.iterations == its[r], (r, its)
+        assert np.array_equal(xa.to_numpy((2, vh, 4, 3)), xs[r].to_numpy((2, vh, 4, 3))), r
