@@ -168,8 +168,10 @@ void GaugeField::forget_links() {
 const void* GaugeField::get(int prec, int recon) {
   DevBuf& b = packed[prec][recon == 12 ? 1 : 0];
   if (!b.p) {
+    if (!aos.p && (prec == F64 || recon != 12)) throw Error(QCU_ERROR_STATE, "internal: drop-in links are recon-12");
     take(b, gauge_bytes(prec, recon, geo.vh));
-    launch_gauge_pack(prec, recon, aos.p, b.p, geo.vh, stream());
+    if (aos.p) launch_gauge_pack(prec, recon, aos.p, b.p, geo.vh, stream());
+    else launch_gauge_repack(prec, packed[F64][1].p, b.p, geo.vh, stream());
     QHIP(hipGetLastError());
   }
   return b.p;
@@ -182,8 +184,6 @@ CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
     std::unique_ptr<CloverField> c(new CloverField);
     c->ck = ck;
     c->vh = geo.vh;
-    c->bad.alloc(sizeof(int));
-    QHIP(hipMemsetAsync(c->bad.p, 0, sizeof(int), stream()));
     cf = c.get();
     clovers[ck] = std::move(c);
   } else {
@@ -197,14 +197,19 @@ CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
     b.A[p] = cf->A[F64][p].p ? nullptr : take(cf->A[F64][p], half64);
     b.Ainv[p] = !inv || cf->Ainv[F64][p].p ? nullptr : take(cf->Ainv[F64][p], half64);
     need[p] = b.A[p] || b.Ainv[p];
+    if (b.Ainv[p] && !cf->bad.p) {
+      cf->bad.alloc(sizeof(int));
+      QHIP(hipMemsetAsync(cf->bad.p, 0, sizeof(int), stream()));
+    }
   }
   if (need[0] || need[1]) {
-    b.gauge = get(F64, 18);
+    const int recon = aos.p ? 18 : 12;
+    b.gauge = get(F64, recon);
     b.nbad = static_cast<int*>(cf->bad.p);
     b.ck = ck;
     b.only = need[0] && need[1] ? -1 : need[1];
     b.geo = geo;
-    launch_clover_build(18, b, stream());
+    launch_clover_build(recon, b, stream());
     QHIP(hipGetLastError());
   }
   // inner-precision parts: A_ee and A^-1_oo
@@ -219,12 +224,12 @@ CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
   return cf;
 }
 
-static std::unique_ptr<GaugeField> new_gauge(const int L[4]) {
+static std::unique_ptr<GaugeField> new_gauge(const int L[4], bool keep_aos = true) {
   validate_lattice(L);
   std::unique_ptr<GaugeField> g(new GaugeField);
   for (int i = 0; i < 4; ++i) g->L[i] = L[i];
   g->geo = make_geom(L);
-  g->aos.alloc((size_t)8 * g->geo.vh * 9 * 16);
+  if (keep_aos) g->aos.alloc((size_t)8 * g->geo.vh * 9 * 16);
   return g;
 }
 
@@ -415,17 +420,6 @@ using namespace qcu;
 // =================================================================== qcu.h ===
 static QcuParam g_param;
 
-// fingerprint of the caller's interface gauge (launch_fingerprint), on the host
-static uint64_t gauge_fingerprint(const void* aos, long vh) {
-  DevBuf* s = ctx().buf("fingerprint", sizeof(uint64_t) * (kFingerprintBlocks + 1));
-  launch_fingerprint(aos, (size_t)8 * vh * 9 * 16, static_cast<uint64_t*>(s->p), stream());
-  QHIP(hipGetLastError());
-  uint64_t h = 0;
-  QHIP(hipMemcpyAsync(&h, s->p, sizeof h, hipMemcpyDeviceToHost, stream()));
-  QHIP(hipStreamSynchronize(stream()));
-  return h;
-}
-
 // 1: the drop-in calls trust that a gauge pointer they have seen still holds the same
 // links (the copy is remade only by initGridSize / loadQcuGauge or a new pointer)
 static bool dropin_trust_pointer() {
@@ -437,31 +431,46 @@ static void require_aligned(const void* p, const char* what) {
   QREQ((reinterpret_cast<uintptr_t>(p) & 15) == 0, std::string(what) + " must be 16-byte aligned (complex128)");
 }
 
-// pinned host word the fingerprint of a deferred check lands in
-static uint64_t* fingerprint_host() {
-  static uint64_t* h = nullptr;
-  if (!h) QHIP(hipHostMalloc(reinterpret_cast<void**>(&h), sizeof(uint64_t), hipHostMallocDefault));
+static uint64_t* fingerprint_parts() {
+  uint64_t*& h = ctx().dropin.fp_parts;
+  if (!h)
+    QHIP(hipHostMalloc(reinterpret_cast<void**>(&h), kFingerprintBlocks * sizeof(uint64_t), hipHostMallocDefault));
   return h;
 }
+// the fingerprint last queued, once the library stream has been synchronised
+static uint64_t fingerprint_value() {
+  uint64_t h = 0;
+  for (int k = 0; k < kFingerprintBlocks; ++k) h += ctx().dropin.fp_parts[k];
+  return h;
+}
+// after a synchronisation of the library stream: take over the fingerprint of an import
+static void dropin_settle() {
+  Context::Dropin& d = ctx().dropin;
+  if (d.fp_queued) d.fp = fingerprint_value();
+  d.fp_queued = false;
+}
 
-// remake the drop-in copy from the caller's gauge, whose fingerprint is fp
-static void dropin_rebuild(void* gauge, const QcuParam* param, bool same_geom, uint64_t fp) {
+// remake the drop-in copy from the caller's gauge: rows 0-1 packed, with their fingerprint,
+// in one pass (16^3x32: 25 us; the copy, the rebuilt row, two packed forms and the
+// fingerprint it replaces took 170)
+static void dropin_rebuild(void* gauge, const QcuParam* param, bool same_geom) {
   Context::Dropin& d = ctx().dropin;
   if (d.g) QHIP(hipStreamSynchronize(stream()));
+  d.ptr = nullptr;  // until the new links are in
   if (same_geom) {  // new links, no packed copies, no clover, in the old allocations
-    GaugeField& g = *d.g;
-    unbind_cached_batches(&g);
-    g.forget_links();
-    QHIP(hipMemcpyAsync(g.aos.p, gauge, g.aos.n, hipMemcpyDeviceToDevice, stream()));
+    unbind_cached_batches(d.g.get());
+    d.g->forget_links();
   } else {
     if (d.g) drop_cached_batches(d.g.get());
     d.g.reset();
-    d.g = make_gauge_from_aos(gauge, param->lattice_size);
+    d.g = new_gauge(param->lattice_size, false);
   }
-  launch_gauge_reconstruct(d.g->aos.p, d.g->geo.vh, stream());
+  GaugeField& g = *d.g;
+  g.take(g.packed[F64][1], gauge_bytes(F64, 12, g.geo.vh));
+  launch_gauge_import(gauge, g.packed[F64][1].p, fingerprint_parts(), g.geo.vh, stream());
   QHIP(hipGetLastError());
+  d.fp_queued = true;
   d.ptr = gauge;
-  d.fp = fp;
 }
 
 // The packed copy and clover fields behind fullDslashQcu and cg_inverter.  The
@@ -486,19 +495,21 @@ static GaugeField& dropin_gauge(void* gauge, const QcuParam* param, bool reload,
   const bool same_geom = d.g && memcmp(d.g->L, param->lattice_size, sizeof(int) * 4) == 0;
   const bool same = same_geom && d.ptr == gauge;
   if (same && !reload && dropin_trust_pointer()) return *d.g;
-  const long vh = (long)param->lattice_size[0] * param->lattice_size[1] * param->lattice_size[2] *
-                  param->lattice_size[3] / 2;
-  if (deferred && same && !reload) {
-    DevBuf* sbuf = ctx().buf("fingerprint", sizeof(uint64_t) * (kFingerprintBlocks + 1));
-    launch_fingerprint(gauge, (size_t)8 * vh * 9 * 16, static_cast<uint64_t*>(sbuf->p), stream());
-    QHIP(hipGetLastError());
-    QHIP(hipMemcpyAsync(fingerprint_host(), sbuf->p, sizeof(uint64_t), hipMemcpyDeviceToHost, stream()));
-    *deferred = true;
-    return *d.g;
+  if (d.fp_queued) {  // an import whose caller did not get to settle it
+    QHIP(hipStreamSynchronize(stream()));
+    dropin_settle();
   }
-  const uint64_t fp = gauge_fingerprint(gauge, vh);
-  if (same && !reload && fp == d.fp) return *d.g;
-  dropin_rebuild(gauge, param, same_geom, fp);
+  if (same && !reload) {
+    launch_fingerprint(gauge, fingerprint_parts(), d.g->geo.vh, stream());
+    QHIP(hipGetLastError());
+    if (deferred) {
+      *deferred = true;
+      return *d.g;
+    }
+    QHIP(hipStreamSynchronize(stream()));
+    if (fingerprint_value() == d.fp) return *d.g;
+  }
+  dropin_rebuild(gauge, param, same_geom);
   return *d.g;
 }
 
@@ -506,9 +517,8 @@ static GaugeField& dropin_gauge(void* gauge, const QcuParam* param, bool reload,
 // when the caller's gauge had changed, in which case the copy has been remade and the
 // caller redoes its work
 static bool dropin_gauge_changed(void* gauge, const QcuParam* param) {
-  const uint64_t fp = *fingerprint_host();
-  if (fp == ctx().dropin.fp) return false;
-  dropin_rebuild(gauge, param, true, fp);
+  if (fingerprint_value() == ctx().dropin.fp) return false;
+  dropin_rebuild(gauge, param, true);
   return true;
 }
 
@@ -525,16 +535,20 @@ extern "C" void initGridSize(QcuGrid_t* grid, QcuParam* p_param, void* gauge, vo
     memcpy(c.L, p_param->lattice_size, sizeof c.L);
     c.have_geom = true;
     g_param = *p_param;
-    if (gauge) dropin_gauge(gauge, p_param, true);
+    if (gauge) {
+      dropin_gauge(gauge, p_param, true);
+      QHIP(hipStreamSynchronize(stream()));
+      dropin_settle();
+    }
   });
 }
 
 extern "C" void loadQcuGauge(void* gauge, QcuParam* param) {
   dropin("loadQcuGauge", [&] {
     ensure_init();
-    GaugeField& g = dropin_gauge(gauge, param, true);
-    g.get(F64, 12);
+    dropin_gauge(gauge, param, true);
     QHIP(hipStreamSynchronize(stream()));
+    dropin_settle();
   });
 }
 
@@ -575,6 +589,7 @@ extern "C" void fullDslashQcu(void* fermion_out, void* fermion_in, void* gauge, 
       apply_m_iface(*ctx().dropin.g, op, fermion_out, fermion_in, dagger_flag ? 1 : 0);
       QHIP(hipStreamSynchronize(stream()));
     }
+    dropin_settle();
   });
 }
 
@@ -596,6 +611,7 @@ extern "C" void cg_inverter(void* b_vector, void* x_vector, void* gauge, QcuPara
     const void* bs[1] = {b_vector};
     solve_batch(g, op, ctx().default_solve, 1, xs, bs, &st);
     QHIP(hipStreamSynchronize(stream()));
+    dropin_settle();
   });
   if (rc != QCU_SUCCESS && rc != QCU_ERROR_NOT_CONVERGED && rc != QCU_ERROR_BREAKDOWN) {
     const std::string msg = g_last_msg;
@@ -688,6 +704,7 @@ int qcuFinalize(void) {
     drop_cached_batches(nullptr);
     c.dropin.g.reset();
     c.dropin.ptr = nullptr;
+    c.dropin.fp_queued = false;
     c.scratch.clear();
     QHIP(hipStreamDestroy(c.stream));
     c.stream = nullptr;

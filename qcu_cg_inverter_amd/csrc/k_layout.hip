@@ -55,81 +55,174 @@ void launch_spinor_to_aos(int prec, Vec in, void* aos, long aos_stride, long vh,
   else hipLaunchKernelGGL(spinor_to_aos_kernel<F16>, grid, dim3(256), 0, st, in, a, aos_stride, vh);
 }
 
-// gauge: thread per (link, mu, parity); the interface link is 9 complex row-major; the
-// packed field is written in the layout LinkIO reads (LinkLayout)
+// one link, 9 complex row-major in u, to its packed words (the layout LinkIO reads)
 template <int P, int R>
-__global__ void gauge_pack_kernel(const double2* aos, void* out, long vh) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int mp = blockIdx.y;  // mu * 2 + parity
-  if (i >= vh) return;
-  const double2* s = aos + ((long)mp * vh + i) * 9;
+__device__ __forceinline__ void store_link(void* out, long vh, int mp, long i, const double2 u[9]) {
   constexpr int NE = R == 12 ? 6 : 9;
   static_assert(LinkLayout<F32, 12>::blocked && LinkLayout<F32, 18>::blocked && LinkLayout<F16, 12>::blocked &&
                     LinkLayout<F16, 18>::blocked,
                 "the FP32 and FP16 stores below step by kSiteBlock");
-  if (P == F64) {
+  auto half2 = [](double2 z) { return (unsigned)f2h((float)z.x) | ((unsigned)f2h((float)z.y) << 16); };
+  if constexpr (P == F64) {
     double2* d = link_word<F64, R>(static_cast<double2*>(out), vh, mp, i);
     const long ws = link_stride<F64, R>(vh);
 #pragma unroll
-    for (int e = 0; e < NE; ++e) d[e * ws] = s[e];
-  } else if (P == F32) {
-    if (R == 12) {
-      float4* d = link_word<F32, 12>(static_cast<float4*>(out), vh, mp, i);
+    for (int e = 0; e < NE; ++e) d[e * ws] = u[e];
+  } else if constexpr (P == F32 && R == 12) {
+    float4* d = link_word<F32, 12>(static_cast<float4*>(out), vh, mp, i);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double2 a = s[2 * k], b = s[2 * k + 1];
-        d[k * kSiteBlock] = float4{(float)a.x, (float)a.y, (float)b.x, (float)b.y};
-      }
-    } else {
-      float2* d = link_word<F32, 18>(static_cast<float2*>(out), vh, mp, i);
+    for (int k = 0; k < 3; ++k)
+      d[k * kSiteBlock] = float4{(float)u[2 * k].x, (float)u[2 * k].y, (float)u[2 * k + 1].x, (float)u[2 * k + 1].y};
+  } else if constexpr (P == F32) {
+    float2* d = link_word<F32, 18>(static_cast<float2*>(out), vh, mp, i);
 #pragma unroll
-      for (int e = 0; e < 9; ++e) d[e * kSiteBlock] = float2{(float)s[e].x, (float)s[e].y};
-    }
+    for (int e = 0; e < 9; ++e) d[e * kSiteBlock] = float2{(float)u[e].x, (float)u[e].y};
+  } else if constexpr (R == 12) {
+    uint2* d = link_word<F16, 12>(static_cast<uint2*>(out), vh, mp, i);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) d[k * kSiteBlock] = uint2{half2(u[2 * k]), half2(u[2 * k + 1])};
   } else {
-    if (R == 12) {
-      uint2* d = link_word<F16, 12>(static_cast<uint2*>(out), vh, mp, i);
+    unsigned* d = link_word<F16, 18>(static_cast<unsigned*>(out), vh, mp, i);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double2 a = s[2 * k], b = s[2 * k + 1];
-        unsigned lo = (unsigned)f2h((float)a.x) | ((unsigned)f2h((float)a.y) << 16);
-        unsigned hi = (unsigned)f2h((float)b.x) | ((unsigned)f2h((float)b.y) << 16);
-        d[k * kSiteBlock] = uint2{lo, hi};
-      }
-    } else {
-      unsigned* d = link_word<F16, 18>(static_cast<unsigned*>(out), vh, mp, i);
-#pragma unroll
-      for (int e = 0; e < 9; ++e)
-        d[e * kSiteBlock] = (unsigned)f2h((float)s[e].x) | ((unsigned)f2h((float)s[e].y) << 16);
-    }
+    for (int e = 0; e < 9; ++e) d[e * kSiteBlock] = half2(u[e]);
   }
 }
 
+// ------------------------------------------------------------ fingerprint ---
+// A 64-bit fingerprint of rows 0-1 of a gauge's links: the sum (mod 2^64) over their
+// 64-bit words w_i, i the word's place in the gauge, of mix(w_i ^ (i * 0x9E3779B97F4A7C15)),
+// mix being the splitmix64 finaliser (Steele, Lea and Flood, OOPSLA 2014).  A sum of
+// integers does not depend on the order it is taken in, so the result is the same for any
+// launch shape, and a change of any one word changes it except with probability about
+// 2^-64.  Used by the drop-in entry points, which rebuild row 2 and so never read it, to
+// notice a gauge the caller changed in place (16^3x32: 14.8 us, 21.3 + 3.8 over all nine
+// words and with a kernel for the sum).
+__device__ __forceinline__ uint64_t fp_mix(uint64_t z) {
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+// of the complex number q at 16-byte word j of the gauge
+__device__ __forceinline__ uint64_t fp_word(double2 q, long j) {
+  constexpr uint64_t K = 0x9E3779B97F4A7C15ull;
+  const uint64_t k = (uint64_t)(2 * j) * K;
+  return fp_mix(__builtin_bit_cast(uint64_t, q.x) ^ k) + fp_mix(__builtin_bit_cast(uint64_t, q.y) ^ (k + K));
+}
+
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
+    lo = __shfl_xor(lo, off, 64);
+    hi = __shfl_xor(hi, off, 64);
+    v += ((uint64_t)hi << 32) | lo;
+  }
+  return v;
+}
+// the block's sum to its word of `parts`, host memory: the host adds the words after the
+// synchronisation it needs anyway, which saves a kernel and a copy
+__device__ __forceinline__ void put_fingerprint(uint64_t h, uint64_t* parts, uint64_t* red) {
+  h = wave_sum_u64(h);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = h;
+  __syncthreads();
+  if (threadIdx.x == 0) parts[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+
+// gauge: a wave takes 64 links of one (mu, parity) field at a time as one run of 576
+// 16-byte words through its LDS tile (a lane then reads its own 9-word record: odd stride,
+// no bank conflicts), because a lane reading its own record from memory asks for 64 lines
+// per load: 16^3x32 FP64 recon-18 54 us that way, 29 this way (5.2 TB/s), 24^3x48 273 and
+// 150.  FP: with the fingerprint of rows 0-1 as they pass.
+template <int P, int R, int FP>
+__global__ void __launch_bounds__(256) gauge_pack_kernel(const double2* aos, void* out, long vh, uint64_t* parts) {
+  __shared__ double2 tile[4][576];
+  __shared__ uint64_t red[4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const long nch = (vh + 63) / 64, units = 8 * nch;
+  double2* T = tile[wv];
+  uint64_t h = 0;
+  for (long u = (long)blockIdx.x * 4 + wv; u < units; u += (long)gridDim.x * 4) {
+    const int mp = (int)(u / nch);  // mu * 2 + parity
+    const long l0 = (u - mp * nch) * 64;
+    const int n = (int)(vh - l0 < 64 ? vh - l0 : 64);
+    const long w0 = ((long)mp * vh + l0) * 9;
+    double2 q[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const int f = k * 64 + lane;
+      q[k] = f < 9 * n ? aos[w0 + f] : double2{0.0, 0.0};
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const int f = k * 64 + lane;
+      if (FP && f < 9 * n && f % 9 < 6) h += fp_word(q[k], w0 + f);
+      T[f] = q[k];
+    }
+    wave_sync();
+    if (lane < n) {
+      double2 v[9];
+#pragma unroll
+      for (int e = 0; e < (R == 12 ? 6 : 9); ++e) v[e] = T[lane * 9 + e];
+      store_link<P, R>(out, vh, mp, l0 + lane, v);
+    }
+    wave_sync();  // the tile is free again
+  }
+  if (FP) put_fingerprint(h, parts, red);
+}
+
 void launch_gauge_pack(int prec, int recon, const void* aos, void* out, long vh, hipStream_t st) {
-  dim3 grid(nblk(vh, 256), 8);
+  const dim3 grid(nblk(8 * ((vh + 63) / 64), 4));
   const double2* a = static_cast<const double2*>(aos);
-#define QCU_GP(P, R) \
-  if (prec == P && recon == R) { hipLaunchKernelGGL((gauge_pack_kernel<P, R>), grid, dim3(256), 0, st, a, out, vh); return; }
+#define QCU_GP(P, R)                                                                                  \
+  if (prec == P && recon == R) {                                                                      \
+    hipLaunchKernelGGL((gauge_pack_kernel<P, R, 0>), grid, dim3(256), 0, st, a, out, vh, (uint64_t*)nullptr); \
+    return;                                                                                           \
+  }
   QCU_GP(F64, 18) QCU_GP(F64, 12) QCU_GP(F32, 18) QCU_GP(F32, 12) QCU_GP(F16, 18) QCU_GP(F16, 12)
 #undef QCU_GP
 }
 
-// row 2 of every interface-layout link rebuilt from rows 0 and 1, the reference's
-// reading of a gauge (src/qcu_wilson_dslash_neo.cu:73-86)
-__global__ void gauge_reconstruct_kernel(double2* aos, long nlinks) {
-  long l = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= nlinks) return;
-  double2* s = aos + l * 9;
-  cx<double> u[9];
-#pragma unroll
-  for (int e = 0; e < 6; ++e) u[e] = {s[e].x, s[e].y};
-  recon_row2(u);
-#pragma unroll
-  for (int e = 6; e < 9; ++e) s[e] = double2{u[e].re, u[e].im};
+void launch_gauge_import(const void* aos, void* out, uint64_t* parts, long vh, hipStream_t st) {
+  hipLaunchKernelGGL((gauge_pack_kernel<F64, 12, 1>), dim3(kFingerprintBlocks), dim3(256), 0, st,
+                     static_cast<const double2*>(aos), out, vh, parts);
 }
 
-void launch_gauge_reconstruct(void* aos, long vh, hipStream_t st) {
-  long n = 8 * vh;
-  hipLaunchKernelGGL(gauge_reconstruct_kernel, dim3(nblk(n, 256)), dim3(256), 0, st, static_cast<double2*>(aos), n);
+__global__ void __launch_bounds__(256) fingerprint_kernel(const double2* __restrict__ aos, long nlinks,
+                                                          uint64_t* parts) {
+  __shared__ uint64_t red[4];
+  uint64_t h = 0;
+  const long stride = (long)gridDim.x * blockDim.x;
+#pragma unroll 4
+  for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j < nlinks * 6; j += stride) {
+    const long l = j / 6, w = l * 9 + (j - l * 6);
+    h += fp_word(aos[w], w);
+  }
+  put_fingerprint(h, parts, red);
+}
+
+void launch_fingerprint(const void* aos, uint64_t* parts, long vh, hipStream_t st) {
+  hipLaunchKernelGGL(fingerprint_kernel, dim3(kFingerprintBlocks), dim3(256), 0, st,
+                     static_cast<const double2*>(aos), 8 * vh, parts);
+}
+
+// packed FP64 rows 0-1 (recon-12) -> FP32 or FP16
+template <int P>
+__global__ void gauge_repack_kernel(const double2* rows, void* out, long vh) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int mp = blockIdx.y;
+  if (i >= vh) return;
+  const double2* b = link_word<F64, 12>(rows, vh, mp, i);
+  double2 v[9];
+#pragma unroll
+  for (int e = 0; e < 6; ++e) v[e] = ld_nt(b + e * kSiteBlock);
+  store_link<P, 12>(out, vh, mp, i, v);
+}
+
+void launch_gauge_repack(int prec, const void* rows, void* out, long vh, hipStream_t st) {
+  const dim3 grid(nblk(vh, 256), 8);
+  const double2* r = static_cast<const double2*>(rows);
+  if (prec == F32) hipLaunchKernelGGL(gauge_repack_kernel<F32>, grid, dim3(256), 0, st, r, out, vh);
+  else hipLaunchKernelGGL(gauge_repack_kernel<F16>, grid, dim3(256), 0, st, r, out, vh);
 }
 
 // ----------------------------------------------- reference storage shifts ---
@@ -279,69 +372,5 @@ void launch_spinor_convert(int pin, Vec in, int pout, Vec out, long vh, int nrhs
 #undef QCU_SC
 }
 
-
-// ------------------------------------------------------------ fingerprint ---
-// A 64-bit fingerprint of a buffer: the sum (mod 2^64) over its 64-bit words w_i of
-// mix(w_i ^ (i * 0x9E3779B97F4A7C15)), mix being the splitmix64 finaliser (Steele,
-// Lea and Flood, OOPSLA 2014).  A sum of integers does not depend on the order it is
-// taken in, so the result is the same for any launch shape, and a change of any one
-// word changes it except with probability about 2^-64.  Used by the drop-in entry
-// points to notice a gauge the caller changed in place.
-__device__ __forceinline__ uint64_t fp_mix(uint64_t z) {
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  return z ^ (z >> 31);
-}
-
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
-    lo = __shfl_xor(lo, off, 64);
-    hi = __shfl_xor(hi, off, 64);
-    v += ((uint64_t)hi << 32) | lo;
-  }
-  return v;
-}
-
-// partials[block] = sum over the block's grid-strided words
-__global__ void __launch_bounds__(256) fingerprint_kernel(const uint64_t* __restrict__ w, long n,
-                                                          uint64_t* __restrict__ partials) {
-  __shared__ uint64_t red[4];
-  constexpr uint64_t K = 0x9E3779B97F4A7C15ull;
-  uint64_t h = 0;
-  const long stride = (long)gridDim.x * blockDim.x;
-  const long t0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const ulonglong2* w2 = reinterpret_cast<const ulonglong2*>(w);  // 16-byte loads
-  const long n2 = n / 2;
-#pragma unroll 4
-  for (long i = t0; i < n2; i += stride) {
-    const ulonglong2 q = w2[i];
-    h += fp_mix(q.x ^ ((uint64_t)(2 * i) * K)) + fp_mix(q.y ^ ((uint64_t)(2 * i + 1) * K));
-  }
-  if ((n & 1) && t0 == 0) h += fp_mix(w[n - 1] ^ ((uint64_t)(n - 1) * K));
-  h = wave_sum_u64(h);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = h;
-  __syncthreads();
-  if (threadIdx.x == 0) partials[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-
-__global__ void __launch_bounds__(256) fingerprint_sum_kernel(const uint64_t* __restrict__ partials, int n,
-                                                              uint64_t* __restrict__ out) {
-  __shared__ uint64_t red[4];
-  uint64_t h = 0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) h += partials[i];
-  h = wave_sum_u64(h);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = h;
-  __syncthreads();
-  if (threadIdx.x == 0) out[0] = red[0] + red[1] + red[2] + red[3];
-}
-
-void launch_fingerprint(const void* buf, size_t bytes, uint64_t* scratch, hipStream_t st) {
-  const long n = (long)(bytes / 8);
-  hipLaunchKernelGGL(fingerprint_kernel, dim3(kFingerprintBlocks), dim3(256), 0, st,
-                     static_cast<const uint64_t*>(buf), n, scratch + 1);
-  hipLaunchKernelGGL(fingerprint_sum_kernel, dim3(1), dim3(256), 0, st, scratch + 1, kFingerprintBlocks, scratch);
-}
 
 }  // namespace qcu

@@ -559,4 +559,12 @@ __device__ __forceinline__ unsigned remap_block(unsigned b, unsigned nb, int on)
   return x * q + (x < r ? x : r) + k;
 }
 
+// a wave's LDS accesses are processed in order; this keeps the compiler from moving
+// the wave's own loads and stores across the point where lanes trade records
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace qcu

@@ -85,7 +85,8 @@ inline size_t solver_clover_bytes(int prec, long vh) {
 }
 
 // a gauge field resident in HBM: the interface copy plus packed variants made on
-// first use, and clover fields keyed by kappa * c_sw
+// first use, and clover fields keyed by kappa * c_sw.  The drop-in gauge has no interface
+// copy: its links are packed[F64][1], rows 0-1, and row 2 is always rebuilt from them.
 struct GaugeField {
   int L[4];
   Geom geo;
@@ -145,6 +146,8 @@ struct Context {
     const void* ptr = nullptr;
     std::unique_ptr<GaugeField> g;
     uint64_t fp = 0;
+    bool fp_queued = false;  // fp is still to be read from fp_parts, after a synchronisation
+    uint64_t* fp_parts = nullptr;  // pinned, kFingerprintBlocks words
   } dropin;
   qcuSolveParams default_solve;
   // scratch shared by calls (grow-only)

@@ -38,17 +38,19 @@ void launch_spinor_from_aos(int prec, const void* aos, long aos_stride, Vec out,
 void launch_spinor_to_aos(int prec, Vec in, void* aos, long aos_stride, long vh, int nrhs, hipStream_t st);
 // interface gauge (complex128 [4][2][Vh][3][3]) -> packed planes
 void launch_gauge_pack(int prec, int recon, const void* aos, void* out, long vh, hipStream_t st);
-// rebuild row 2 of every interface-layout link from rows 0 and 1 (in place)
-void launch_gauge_reconstruct(void* aos, long vh, hipStream_t st);
+// packed FP64 recon-12 links -> FP32 or FP16 recon-12
+void launch_gauge_repack(int prec, const void* rows, void* out, long vh, hipStream_t st);
+// 64-bit fingerprint of rows 0-1 of an interface gauge: the sum of the kFingerprintBlocks
+// words that the kernel writes to `parts` (pinned host memory); launch_gauge_import packs
+// those rows in the same pass (FP64 recon-12)
+constexpr int kFingerprintBlocks = 1024;
+void launch_fingerprint(const void* aos, uint64_t* parts, long vh, hipStream_t st);
+void launch_gauge_import(const void* aos, void* out, uint64_t* parts, long vh, hipStream_t st);
 // reference storage shifts: kind 0 half spinor [Vh][24] <-> [24][Vh] doubles; kind 1
 // gauge [8][Vh][18] -> [8][12][Vh] (back with row 2 rebuilt)
 void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long vh, hipStream_t st);
 // lexicographic <-> even-odd, nc (12 or 9) complex per site, nfields fields of V sites
 void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st);
-// 64-bit fingerprint of `bytes` (a multiple of 8) at buf, order-independent; scratch
-// holds kFingerprintBlocks + 1 words and the result lands in scratch[0]
-constexpr int kFingerprintBlocks = 1024;
-void launch_fingerprint(const void* buf, size_t bytes, uint64_t* scratch, hipStream_t st);
 // out = in (accumulate = 0) or out += in (accumulate = 1), any precisions
 void launch_spinor_convert(int pin, Vec in, int pout, Vec out, long vh, int nrhs, int accumulate, hipStream_t st);
 

@@ -174,3 +174,40 @@ def test_scalar_steps_change_kernels_mid_solve(q):
         sa = q.solve_batch_device(g, op, [xa], [bs[r]], sp)[0]
         assert sa.converged and sa.iterations == its[r], (r, its)
         assert np.array_equal(xa.to_numpy((2, vh, 4, 3)), xs[r].to_numpy((2, vh, 4, 3))), r
+
+
+@pytest.mark.parametrize("L", [(4, 6, 2, 10), (8, 8, 4, 14)])
+@pytest.mark.parametrize("prec", [0, 1, 2])
+def test_dropin_import(q, L, prec):
+    """The drop-in gauge is imported as rows 0-1 only and its FP32 and FP16 links come from
+    those: cg_inverter in each precision on links scaled by 0.12 (at the reference's kappa =
+    1 that makes the system as well conditioned as a Wilson solve; row 2 is rebuilt, so it
+    scales by 0.12 squared), on a gauge changed in one real of row 1 between calls, and
+    indifferent to row 2.  Residuals by the oracle."""
+    prm = q.param(L)
+    vh = q.half_volume(L)
+    b = orc.source_gauss(L, 13)
+    bd, xd, yd = q.DeviceBuffer.from_numpy(b), q.DeviceBuffer(2 * vh * 192), q.DeviceBuffer(2 * vh * 192)
+    u = 0.12 * orc.gauge_random(L, 46, 0.3)
+    gd = q.DeviceBuffer.from_numpy(u)
+    sp = q.default_solve_params(tol=1e-10, precision=prec)
+    q.check(q.lib().qcuSetDefaultSolve(ctypes.byref(sp)))
+    try:
+        for step in range(3):
+            if step == 1:
+                u[2, 1, vh - 1, 1, 2] += 1e-3
+            if step == 2:
+                u[:, :, :, 2, :] = 7.0
+            gd.upload(u)
+            q.lib().cg_inverter(bd.ptr, xd.ptr, gd.ptr, ctypes.byref(prm))
+            assert q.lib().qcuGetLastError() == 0
+            x = xd.to_numpy((2, vh, 4, 3))
+            A = orc.clover_fields(u, L, 1.0, 1.0, recon=12)[0]
+            r = b - orc.full_op(x, u, L, 1.0, A=A, s=1, tbc=1.0, recon=12)
+            assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b), step
+            q.lib().fullDslashQcu(yd.ptr, bd.ptr, gd.ptr, ctypes.byref(prm), 1)
+            ref = orc.full_op(b, u, L, 1.0, A=A, s=-1, tbc=1.0, recon=12)
+            assert np.linalg.norm(yd.to_numpy((2, vh, 4, 3)) - ref) <= 1e-14 * np.linalg.norm(ref), step
+    finally:
+        sp = q.default_solve_params(tol=1e-12, precision=0)
+        q.check(q.lib().qcuSetDefaultSolve(ctypes.byref(sp)))
