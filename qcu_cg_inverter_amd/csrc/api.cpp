@@ -105,7 +105,6 @@ void ensure_init() {
   if (n <= 0) throw Error(QCU_ERROR_HIP, "no HIP device");
   QHIP(hipSetDevice(c.device));
   QHIP(hipStreamCreate(&c.stream));  // default priority, blocking w.r.t. the null stream
-  QHIP(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
   noalloc_setup(c.device);           // device address of qcuHopNoAlloc's static scratch
   qcuDefaultSolveParams(&c.default_solve);
   c.default_solve.precision = QCU_PREC_DOUBLE;
@@ -384,8 +383,7 @@ static int iface_slices(const Geom& geo, const IfaceHop& p, int nrhs) {
   return eighth_of_t(geo);
 }
 
-bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, const void* const* in, hipStream_t st,
-               hipEvent_t done) {
+bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, const void* const* in, hipStream_t st) {
   QREQ(nrhs >= 1 && nrhs <= kMaxRhs, "nrhs out of range");
   const size_t n = (size_t)geo.vh * 192 * (p.parity < 0 ? 2 : 1);
   for (int r = 0; r < nrhs; ++r)
@@ -410,7 +408,7 @@ bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, c
     a.in[r] = in[r];
     a.out[r] = out[r];
   }
-  launch_hop_iface(p.prec, p.recon, p.epi, p.dagger, a, st, done);
+  launch_hop_iface(p.prec, p.recon, p.epi, p.dagger, a, st);
   QHIP(hipGetLastError());
   return true;
 }
@@ -418,12 +416,6 @@ bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, c
 }  // namespace qcu
 
 using namespace qcu;
-
-// the end of a synchronous call: its last launch recorded ctx().done, or the stream
-static void wait_call(bool recorded) {
-  if (recorded) QHIP(hipEventSynchronize(ctx().done));
-  else QHIP(hipStreamSynchronize(stream()));
-}
 
 // =================================================================== qcu.h ===
 static QcuParam g_param;
@@ -576,9 +568,9 @@ extern "C" void dslashQcu(void* fermion_out, void* fermion_in, void* gauge, QcuP
     const char* i = static_cast<const char*>(fermion_in);
     char* o = static_cast<char*>(fermion_out);
     QREQ(o + g.vh * 192 <= i || i + g.vh * 192 <= o, "dslashQcu: fermion_out and fermion_in overlap");
-    launch_dslash(fermion_in, fermion_out, gauge, g, parity, stream(), ctx().done);
+    launch_dslash(fermion_in, fermion_out, gauge, g, parity, stream());
     QHIP(hipGetLastError());
-    wait_call(true);
+    QHIP(hipStreamSynchronize(stream()));
   });
 }
 
@@ -591,9 +583,11 @@ extern "C" void fullDslashQcu(void* fermion_out, void* fermion_in, void* gauge, 
     bool deferred = false;
     GaugeField& g = dropin_gauge(gauge, param, false, &deferred);
     qcuOperator op = {1.0, 1.0, 1, 12};
-    wait_call(apply_m_iface(g, op, fermion_out, fermion_in, dagger_flag ? 1 : 0));
+    apply_m_iface(g, op, fermion_out, fermion_in, dagger_flag ? 1 : 0);
+    QHIP(hipStreamSynchronize(stream()));
     if (deferred && dropin_gauge_changed(gauge, param)) {  // the links changed in place: redo
-      wait_call(apply_m_iface(*ctx().dropin.g, op, fermion_out, fermion_in, dagger_flag ? 1 : 0));
+      apply_m_iface(*ctx().dropin.g, op, fermion_out, fermion_in, dagger_flag ? 1 : 0);
+      QHIP(hipStreamSynchronize(stream()));
     }
     dropin_settle();
   });
@@ -651,9 +645,9 @@ static void shift_storage(const char* who, int kind, void* dst, void* src, int d
   size_t soa = (size_t)vh * (kind == 0 ? 24 : 8 * 12) * 8;
   const bool to_soa = dir == TO_COALESCE;
   require_disjoint(dst, to_soa ? soa : aos, src, to_soa ? aos : soa, who);
-  launch_shift_storage(kind, to_soa, src, dst, vh, stream(), ctx().done);
+  launch_shift_storage(kind, to_soa, src, dst, vh, stream());
   QHIP(hipGetLastError());
-  wait_call(true);
+  QHIP(hipStreamSynchronize(stream()));
 }
 
 extern "C" void shiftVectorStorage(void* dst_vec, void* src_vec, int shift_direction, int Lx, int Ly, int Lz, int Lt) {
@@ -680,9 +674,9 @@ static int lex_eo(const char* who, int to_eo, void* dst, const void* src, const 
     int nc = field == QCU_FIELD_SPINOR ? 12 : 9, nf = field == QCU_FIELD_SPINOR ? 1 : 4;
     const size_t n = (size_t)vol * nc * nf * 16;
     require_disjoint(dst, n, src, n, who);
-    launch_lex_eo(to_eo, src, dst, L, nc, nf, stream(), ctx().done);
+    launch_lex_eo(to_eo, src, dst, L, nc, nf, stream());
     QHIP(hipGetLastError());
-    wait_call(true);
+    QHIP(hipStreamSynchronize(stream()));
   });
 }
 
@@ -712,7 +706,6 @@ int qcuFinalize(void) {
     c.dropin.ptr = nullptr;
     c.dropin.fp_queued = false;
     c.scratch.clear();
-    QHIP(hipEventDestroy(c.done));
     QHIP(hipStreamDestroy(c.stream));
     c.stream = nullptr;
     c.inited = false;
@@ -876,8 +869,7 @@ int qcuHop(qcuGauge h, void* out, const void* in, int parity, int dagger, int t_
     long vh = g.geo.vh;
     const IfaceHop p = {g.get(precision, recon), precision, recon, EPI_PLAIN, parity, dagger ? 1 : 0,
                         (double)t_boundary, 1.0, {nullptr, nullptr}};
-    const bool direct = hop_iface(g.geo, p, 1, &out, &in, stream(), ctx().done);
-    if (!direct) {  // in and out overlap: staged
+    if (!hop_iface(g.geo, p, 1, &out, &in, stream())) {  // in and out overlap: staged
       DevBuf* a = ctx().buf("hop_in", spinor_bytes(F64, vh));
       DevBuf* b = ctx().buf("hop_out", spinor_bytes(F64, vh));
       launch_spinor_from_aos(precision, in, 0, vec(a->p), vh, 1, stream());
@@ -886,7 +878,7 @@ int qcuHop(qcuGauge h, void* out, const void* in, int parity, int dagger, int t_
       launch_spinor_to_aos(precision, vec(b->p), out, 0, vh, 1, stream());
     }
     QHIP(hipGetLastError());
-    wait_call(direct);
+    QHIP(hipStreamSynchronize(stream()));
   });
 }
 
@@ -905,8 +897,7 @@ int qcuHopBatch(qcuGauge h, int nrhs, void* const* out, const void* const* in, i
     long vh = g.geo.vh;
     const IfaceHop p = {g.get(precision, recon), precision, recon, EPI_PLAIN, parity, dagger ? 1 : 0,
                         (double)t_boundary, 1.0, {nullptr, nullptr}};
-    const bool direct = hop_iface(g.geo, p, nrhs, out, in, stream(), ctx().done);
-    if (!direct) {  // an output overlaps an input: staged
+    if (!hop_iface(g.geo, p, nrhs, out, in, stream())) {  // an output overlaps an input: staged
       long fb = (long)spinor_bytes(precision, vh);
       DevBuf* a = ctx().buf("hopb_in", (size_t)fb * nrhs);
       DevBuf* b = ctx().buf("hopb_out", (size_t)fb * nrhs);
@@ -916,7 +907,7 @@ int qcuHopBatch(qcuGauge h, int nrhs, void* const* out, const void* const* in, i
       for (int r = 0; r < nrhs; ++r) launch_spinor_to_aos(precision, vec(b->c() + r * fb), out[r], 0, vh, 1, stream());
     }
     QHIP(hipGetLastError());
-    wait_call(direct);
+    QHIP(hipStreamSynchronize(stream()));
   });
 }
 
@@ -924,7 +915,8 @@ int qcuApplyM(qcuGauge h, const qcuOperator* op, void* out, const void* in, int 
   return guarded([&] {
     ensure_init();
     QREQ(h && op && out && in, "qcuApplyM: NULL argument");
-    wait_call(apply_m_iface(*reinterpret_cast<GaugeField*>(h), *op, out, in, dagger ? 1 : 0));
+    apply_m_iface(*reinterpret_cast<GaugeField*>(h), *op, out, in, dagger ? 1 : 0);
+    QHIP(hipStreamSynchronize(stream()));
   });
 }
 
@@ -932,7 +924,8 @@ int qcuApplyComposite(qcuGauge h, const qcuOperator* op, int kind, void* out, co
   return guarded([&] {
     ensure_init();
     QREQ(h && op && out && in, "qcuApplyComposite: NULL argument");
-    wait_call(apply_composite_iface(*reinterpret_cast<GaugeField*>(h), *op, kind, out, in, dagger ? 1 : 0));
+    apply_composite_iface(*reinterpret_cast<GaugeField*>(h), *op, kind, out, in, dagger ? 1 : 0);
+    QHIP(hipStreamSynchronize(stream()));
   });
 }
 

@@ -12,9 +12,9 @@ QCU_DECL(f64)
 QCU_DECL(f32)
 QCU_DECL(f16)
 #undef QCU_DECL
-void launch_iface_f64(int, int, int, const IfaceArgs&, hipStream_t, hipEvent_t);
-void launch_iface_f32(int, int, const IfaceArgs&, hipStream_t, hipEvent_t);
-void launch_iface_f16(int, int, const IfaceArgs&, hipStream_t, hipEvent_t);
+void launch_iface_f64(int, int, int, const IfaceArgs&, hipStream_t);
+void launch_iface_f32(int, int, const IfaceArgs&, hipStream_t);
+void launch_iface_f16(int, int, const IfaceArgs&, hipStream_t);
 
 void launch_split_f64(int, int, const HopSplit&, hipStream_t);
 void launch_split_f32(int, int, const HopSplit&, hipStream_t);
@@ -31,10 +31,10 @@ void launch_hop(int prec, int recon, int epi, const HopArgs& a, int block, int r
   table[prec][rpt - 1](recon, epi, a, block, rb, st);
 }
 
-void launch_hop_iface(int prec, int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st, hipEvent_t done) {
-  if (prec == F64) launch_iface_f64(recon, epi, dagger, a, st, done);
-  else if (prec == F32) launch_iface_f32(recon, dagger, a, st, done);
-  else launch_iface_f16(recon, dagger, a, st, done);
+void launch_hop_iface(int prec, int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st) {
+  if (prec == F64) launch_iface_f64(recon, epi, dagger, a, st);
+  else if (prec == F32) launch_iface_f32(recon, dagger, a, st);
+  else launch_iface_f16(recon, dagger, a, st);
 }
 
 void launch_hop_split(int prec, int recon, int epi, const HopSplit& a, hipStream_t st) {

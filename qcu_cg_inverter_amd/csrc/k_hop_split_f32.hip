@@ -3,9 +3,9 @@
 
 namespace qcu {
 
-void launch_iface_f32(int recon, int dagger, const IfaceArgs& a, hipStream_t st, hipEvent_t done) {
-  if (recon == 12) launch_iface<F32, 12, EPI_PLAIN>(a, dagger, st, done);
-  else launch_iface<F32, 18, EPI_PLAIN>(a, dagger, st, done);
+void launch_iface_f32(int recon, int dagger, const IfaceArgs& a, hipStream_t st) {
+  if (recon == 12) launch_iface<F32, 12, EPI_PLAIN>(a, dagger, st);
+  else launch_iface<F32, 18, EPI_PLAIN>(a, dagger, st);
 }
 
 void launch_split_f32(int recon, int epi, const HopSplit& a, hipStream_t st) {

@@ -4,16 +4,16 @@
 namespace qcu {
 
 template <int R>
-static void iface(int epi, int dagger, const IfaceArgs& a, hipStream_t st, hipEvent_t done) {
-  if (epi == EPI_PLAIN) launch_iface<F64, R, EPI_PLAIN>(a, dagger, st, done);
-  else if (epi == EPI_XPAY) launch_iface<F64, R, EPI_XPAY>(a, dagger, st, done);
-  else if (epi == EPI_CLOV) launch_iface<F64, R, EPI_CLOV>(a, dagger, st, done);
-  else launch_iface<F64, R, EPI_CLOV_XPAY>(a, dagger, st, done);
+static void iface(int epi, int dagger, const IfaceArgs& a, hipStream_t st) {
+  if (epi == EPI_PLAIN) launch_iface<F64, R, EPI_PLAIN>(a, dagger, st);
+  else if (epi == EPI_XPAY) launch_iface<F64, R, EPI_XPAY>(a, dagger, st);
+  else if (epi == EPI_CLOV) launch_iface<F64, R, EPI_CLOV>(a, dagger, st);
+  else launch_iface<F64, R, EPI_CLOV_XPAY>(a, dagger, st);
 }
 
-void launch_iface_f64(int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st, hipEvent_t done) {
-  if (recon == 12) iface<12>(epi, dagger, a, st, done);
-  else iface<18>(epi, dagger, a, st, done);
+void launch_iface_f64(int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st) {
+  if (recon == 12) iface<12>(epi, dagger, a, st);
+  else iface<18>(epi, dagger, a, st);
 }
 
 // the kernel behind dslashQcu: one half spinor, s = +1, the caller's own gauge records
@@ -24,10 +24,10 @@ __global__ void __launch_bounds__(256, 3) dslash_kernel(const double2* in, doubl
                                        (long)remap_block(blockIdx.x, gridDim.x, 1) * 64, S);
 }
 
-void launch_dslash(const void* in, void* out, const void* gauge, const Geom& g, int parity, hipStream_t st,
-                   hipEvent_t done) {
-  launch_done(dslash_kernel, dim3((unsigned)((g.vh + 63) / 64)), dim3(256), st, done, static_cast<const double2*>(in),
-              static_cast<double2*>(out), static_cast<const double2*>(gauge), g, parity);
+void launch_dslash(const void* in, void* out, const void* gauge, const Geom& g, int parity, hipStream_t st) {
+  hipLaunchKernelGGL(dslash_kernel, dim3((unsigned)((g.vh + 63) / 64)), dim3(256), 0, st,
+                     static_cast<const double2*>(in), static_cast<double2*>(out),
+                     static_cast<const double2*>(gauge), g, parity);
 }
 
 void launch_split_f64(int recon, int epi, const HopSplit& a, hipStream_t st) {

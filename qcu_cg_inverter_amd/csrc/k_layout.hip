@@ -283,18 +283,18 @@ __global__ void __launch_bounds__(256) soa_to_aos_kernel(const double* src, doub
   for (int j = threadIdx.x; j < ns * wa; j += blockDim.x) dst[j] = tile[(j % wa) * kTilePad + j / wa];
 }
 
-void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long vh, hipStream_t st, hipEvent_t done) {
+void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long vh, hipStream_t st) {
   // kind 0: half spinor [Vh][24] <-> [24][Vh]; kind 1: gauge [8][Vh][18] <-> [8][12][Vh]
   int wa = kind == 0 ? 24 : 18, w = kind == 0 ? 24 : 12, nf = kind == 0 ? 1 : 8;
   dim3 grid(nblk(vh, kTile), nf);
   const double* s = static_cast<const double*>(src);
   double* d = static_cast<double*>(dst);
   if (to_soa)
-    launch_done(aos_to_soa_kernel, grid, dim3(256), st, done, s, d, vh, wa, w, vh * wa, vh * w);
+    hipLaunchKernelGGL(aos_to_soa_kernel, grid, dim3(256), 0, st, s, d, vh, wa, w, vh * wa, vh * w);
   else if (kind == 0)
-    launch_done(soa_to_aos_kernel<false>, grid, dim3(256), st, done, s, d, vh, w, wa, vh * w, vh * wa);
+    hipLaunchKernelGGL(soa_to_aos_kernel<false>, grid, dim3(256), 0, st, s, d, vh, w, wa, vh * w, vh * wa);
   else
-    launch_done(soa_to_aos_kernel<true>, grid, dim3(256), st, done, s, d, vh, w, wa, vh * w, vh * wa);
+    hipLaunchKernelGGL(soa_to_aos_kernel<true>, grid, dim3(256), 0, st, s, d, vh, w, wa, vh * w, vh * wa);
 }
 
 // ------------------------------------------- lexicographic <-> even-odd ---
@@ -321,8 +321,7 @@ __global__ void lex_eo_kernel(const double2* src, double2* dst, long vol, FastDi
   else dst[(long)l * NC + k] = src[e * NC + k];
 }
 
-void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st,
-                   hipEvent_t done) {
+void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st) {
   long vol = (long)L[0] * L[1] * L[2] * L[3];
   long n = vol * nc;
   dim3 grid(nblk(n, 256), nfields);
@@ -331,7 +330,7 @@ void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc
   FastDiv dlx((uint32_t)L[0]), dly((uint32_t)L[1]), dlz((uint32_t)L[2]);
 #define QCU_LEX(E, N)                                                                                   \
   if (to_eo == E && nc == N) {                                                                          \
-    launch_done((lex_eo_kernel<E, N>), grid, dim3(256), st, done, s, d, vol, dlx, dly, dlz, n);         \
+    hipLaunchKernelGGL((lex_eo_kernel<E, N>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n);     \
     return;                                                                                             \
   }
   QCU_LEX(1, 12) QCU_LEX(0, 12) QCU_LEX(1, 9) QCU_LEX(0, 9)

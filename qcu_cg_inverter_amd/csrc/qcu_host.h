@@ -137,7 +137,6 @@ struct Context {
   bool inited = false;
   int device = 0;
   hipStream_t stream = nullptr;
-  hipEvent_t done = nullptr;  // completion of a synchronous call's last launch (launch_done)
   std::recursive_mutex mu;
   // state of the drop-in entry points: one resident copy, of the gauge last passed,
   // with the fingerprint of the caller's buffer it was made from
@@ -197,8 +196,7 @@ struct IfaceHop {
   const void* clov[2];        // per parity, for the clover epilogues
 };
 // false, with nothing launched, when an output overlaps an input or another output
-bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, const void* const* in, hipStream_t st,
-               hipEvent_t done);
+bool hop_iface(const Geom& geo, const IfaceHop& p, int nrhs, void* const* out, const void* const* in, hipStream_t st);
 
 // solver entry (solver.cpp)
 void solve_batch(GaugeField& g, const qcuOperator& op, const qcuSolveParams& sp, int nrhs, void* const* x,
@@ -208,8 +206,7 @@ void apply_mhat_iface(GaugeField& g, const qcuOperator& op, void* out, const voi
 void drop_cached_batches(GaugeField* g);
 // the fields of g changed: the next solve takes them up again, in the same workspace
 void unbind_cached_batches(GaugeField* g);
-// true: the last launch records ctx().done
-bool apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger);
-bool apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger);
+void apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger);
+void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger);
 
 }  // namespace qcu

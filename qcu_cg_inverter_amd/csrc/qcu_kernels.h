@@ -3,21 +3,9 @@
 // a batch of right-hand sides is strided by `stride` bytes.
 #pragma once
 
-#include <hip/hip_ext.h>
-
 #include "qcu_common.h"
 
 namespace qcu {
-
-// A launch that records `done` (may be null) as its own completion.  The last launch of a
-// synchronous call carries the event the caller then waits for: hipStreamSynchronize
-// puts a barrier packet of its own behind the kernel, 11.5 us for an empty kernel and the
-// wait against 9.6.
-template <typename... A, typename... B>
-inline void launch_done(void (*k)(A...), dim3 grid, dim3 block, hipStream_t st, hipEvent_t done, B&&... args) {
-  if (done) hipExtLaunchKernelGGL(k, grid, block, 0, st, nullptr, done, 0, A(args)...);
-  else hipLaunchKernelGGL(k, grid, block, 0, st, A(args)...);
-}
 
 struct Vec {
   void* p;
@@ -39,12 +27,10 @@ void launch_hop_split(int prec, int recon, int epi, const HopSplit& a, hipStream
 // the hop straight from and to the caller's interface fields (complex128 [Vh][4][3], or
 // full spinors), computed in `prec` (k_hop_split.inc); FP32 and FP16 take the plain
 // epilogue.  No out buffer may overlap an in buffer or another out buffer.
-void launch_hop_iface(int prec, int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st,
-                      hipEvent_t done = nullptr);
+void launch_hop_iface(int prec, int recon, int epi, int dagger, const IfaceArgs& a, hipStream_t st);
 // out(parity) = D in, FP64, periodic, with links from the caller's own gauge
 // [4][2][Vh][3][3], of which rows 0-1 are read; no overlap
-void launch_dslash(const void* in, void* out, const void* gauge, const Geom& g, int parity, hipStream_t st,
-                   hipEvent_t done);
+void launch_dslash(const void* in, void* out, const void* gauge, const Geom& g, int parity, hipStream_t st);
 
 // --------------------------------------------------------------- layout -----
 // interface spinor (complex128 [Vh][4][3]) <-> internal layout of `prec`
@@ -62,10 +48,9 @@ void launch_fingerprint(const void* aos, uint64_t* parts, long vh, hipStream_t s
 void launch_gauge_import(const void* aos, void* out, uint64_t* parts, long vh, hipStream_t st);
 // reference storage shifts: kind 0 half spinor [Vh][24] <-> [24][Vh] doubles; kind 1
 // gauge [8][Vh][18] -> [8][12][Vh] (back with row 2 rebuilt)
-void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long vh, hipStream_t st, hipEvent_t done);
+void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long vh, hipStream_t st);
 // lexicographic <-> even-odd, nc (12 or 9) complex per site, nfields fields of V sites
-void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st,
-                   hipEvent_t done);
+void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st);
 // out = in (accumulate = 0) or out += in (accumulate = 1), any precisions
 void launch_spinor_convert(int pin, Vec in, int pout, Vec out, long vh, int nrhs, int accumulate, hipStream_t st);
 

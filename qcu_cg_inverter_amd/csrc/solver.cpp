@@ -215,7 +215,7 @@ static void one_minus_ainv_d(OpView& o, int dag, const Vec in[2], const Vec out[
   for (int p = 0; p < 2; ++p) launch_axpby(F64, 1.0, in[p], -1.0, out[p], o.g->geo.vh, 1, st);
 }
 
-bool apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger) {
+void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger) {
   QREQ(kind >= QCU_COMP_AINV_D && kind <= QCU_COMP_NORMAL, "qcuApplyComposite: unknown kind");
   OpView o = make_view(g, op, F64, kind == QCU_COMP_A ? CLOVER_A : CLOVER_ALL);
   const long vh = g.geo.vh;
@@ -223,7 +223,7 @@ bool apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void*
     IfaceHop p = {g.get(F64, op.recon), F64, op.recon, o.clover ? EPI_CLOV : EPI_PLAIN, -1, dagger ? 1 : 0, o.tbc(),
                   op.kappa, {nullptr, nullptr}};
     for (int q = 0; q < 2 && o.clover; ++q) p.clov[q] = o.cf->ainv(F64, q);
-    if (hop_iface(g.geo, p, 1, &out, &in, stream(), ctx().done)) return true;
+    if (hop_iface(g.geo, p, 1, &out, &in, stream())) return;
   }
   const size_t fb = spinor_bytes(F64, vh);
   Vec vi[2] = {vec(ctx().buf("cp_i0", fb)->p), vec(ctx().buf("cp_i1", fb)->p)};
@@ -254,16 +254,15 @@ bool apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void*
   for (int p = 0; p < 2; ++p)
     launch_spinor_to_aos(F64, vo[p], static_cast<char*>(out) + p * vh * 192, 0, vh, 1, st);
   QHIP(hipGetLastError());
-  return false;
 }
 
-bool apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger) {
+void apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger) {
   OpView o = make_view(g, op, F64, CLOVER_A);
   long vh = g.geo.vh;
   IfaceHop p = {g.get(F64, op.recon), F64, op.recon, o.clover ? EPI_CLOV_XPAY : EPI_XPAY, -1, dagger, o.tbc(),
                 -op.kappa, {nullptr, nullptr}};
   for (int q = 0; q < 2 && o.clover; ++q) p.clov[q] = o.cf->a(F64, q);
-  if (hop_iface(g.geo, p, 1, &out, &in, stream(), ctx().done)) return true;
+  if (hop_iface(g.geo, p, 1, &out, &in, stream())) return;
   // in and out overlap: staged in internal fields
   Vec ie = vec(ctx().buf("m_ie", spinor_bytes(F64, vh))->p);
   Vec io = vec(ctx().buf("m_io", spinor_bytes(F64, vh))->p);
@@ -276,7 +275,6 @@ bool apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* 
   launch_spinor_to_aos(F64, oe, out, 0, vh, 1, stream());
   launch_spinor_to_aos(F64, oo, static_cast<char*>(out) + vh * 192, 0, vh, 1, stream());
   QHIP(hipGetLastError());
-  return false;
 }
 
 }  // namespace qcu
