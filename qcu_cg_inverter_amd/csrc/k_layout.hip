@@ -302,8 +302,11 @@ void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long
 // parity = (x+y+z+t) mod 2, the half-site order of include/qcu_point.cuh:20-93.  One
 // thread per 16-byte complex of a site record (NC complex per site), so consecutive
 // lanes move consecutive bytes of the lexicographic field; blockIdx.y picks the field.
-// The launcher guarantees vol < 2^31, the range of FastDiv.
-template <bool TO_EO, int NC>
+// The launcher guarantees vol < 2^31, the range of FastDiv.  NT: a field too large to be
+// found in the Infinity Cache by what reads it next is streamed past it: gauge and two
+// spinors of 24^3x48 254 -> 242 us for the three calls (6.1 TB/s but for the waits), 32^3x64
+// 718 -> 695.
+template <bool TO_EO, int NC, int NT>
 __global__ void lex_eo_kernel(const double2* src, double2* dst, long vol, FastDiv dlx, FastDiv dly, FastDiv dlz,
                               long field) {
   long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -317,8 +320,8 @@ __global__ void lex_eo_kernel(const double2* src, double2* dst, long vol, FastDi
   long e = (long)parity * (vol / 2) + (l >> 1);
   src += blockIdx.y * field;
   dst += blockIdx.y * field;
-  if (TO_EO) dst[e * NC + k] = src[(long)l * NC + k];
-  else dst[(long)l * NC + k] = src[e * NC + k];
+  if (TO_EO) stp<NT>(dst + e * NC + k, ldp<NT>(src + (long)l * NC + k));
+  else stp<NT>(dst + (long)l * NC + k, ldp<NT>(src + e * NC + k));
 }
 
 void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st) {
@@ -328,10 +331,12 @@ void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc
   const double2* s = static_cast<const double2*>(src);
   double2* d = static_cast<double2*>(dst);
   FastDiv dlx((uint32_t)L[0]), dly((uint32_t)L[1]), dlz((uint32_t)L[2]);
-#define QCU_LEX(E, N)                                                                                   \
-  if (to_eo == E && nc == N) {                                                                          \
-    hipLaunchKernelGGL((lex_eo_kernel<E, N>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n);     \
-    return;                                                                                             \
+  const bool nt = (size_t)n * nfields * 16 > kNtStoreBytes / 2;
+#define QCU_LEX(E, N)                                                                                          \
+  if (to_eo == E && nc == N) {                                                                                 \
+    if (nt) hipLaunchKernelGGL((lex_eo_kernel<E, N, 1>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n); \
+    else hipLaunchKernelGGL((lex_eo_kernel<E, N, 0>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n);    \
+    return;                                                                                                    \
   }
   QCU_LEX(1, 12) QCU_LEX(0, 12) QCU_LEX(1, 9) QCU_LEX(0, 9)
 #undef QCU_LEX
