@@ -2,7 +2,7 @@
 //
 // The reference does each BLAS-1 op as its own kernel plus a host round trip per
 // reduction (src/qcu_complex_computation.cu:10-134, src/cg_inverter.cu:181-256).
-// Here reductions are per-16-site partials (fixed butterfly order within 16 lanes)
+// Here reductions are per-64-site partials (fixed butterfly order within a wave)
 // summed by a one-block kernel in a fixed order, so every result is bitwise reproducible and
 // independent of how right-hand sides are batched, and all scalars stay on the
 // device: a CG iteration needs no host synchronisation.
@@ -13,17 +13,10 @@ namespace qcu {
 
 static inline unsigned nblk(long n, int b) { return (unsigned)((n + b - 1) / b); }
 
-// the same 16-lane butterfly as the hopping kernel's partials
-__device__ __forceinline__ double group16_sum(double v) {
-#pragma unroll
-  for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 16);
-  return v;
-}
-
-// write each 16-lane group's partial sum (its first lane) at slot site/16
+// a wave's partial, the sum over its 64-site chunk (first lane i), at slot i / 64
 __device__ __forceinline__ void put_partial(double* part, long vh, int r, long i, double v) {
-  v = group16_sum(v);
-  if ((threadIdx.x & 15) == 0 && i < vh) part[(long)r * n_partials(vh) + i / 16] = v;
+  v = group64_sum(v);
+  if ((threadIdx.x & 63) == 0 && i < vh) part[(long)r * n_partials(vh) + i / 64] = v;
 }
 
 template <int P>
@@ -255,143 +248,120 @@ __device__ __forceinline__ double alpha_step(CgScal& s, const double* part_tt, l
   return alpha;
 }
 
+// The share of a site that one thread of the two kernels below takes: half of it in FP64
+// and FP32 (a wave takes one half of a 64-site chunk, so a launch has twice the waves and
+// each keeps half the registers: 16^3x32 is otherwise one wave per SIMD), all of it in FP16.
+// x and p update, s update, of 16^3x32 FP64 14.9 -> 12.7 and 9.6 -> 8.7 us, 8^4 FP32 5.5 ->
+// 4.4 and 4.8 -> 3.8; 32^3x64 solves 3.3 % (FP32) and 4 % (FP16) faster.
+template <int P>
+struct Share {
+  static constexpr int H = P == F16 ? 1 : 2, N = 12 / H;
+  int h;
+  long first, site;  // the chunk's first site, this thread's
+  bool live;
+  __device__ __forceinline__ explicit Share(long vh) {
+    const long w = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    h = (int)(w % H);
+    first = w / H * 64;
+    const long i = first + (threadIdx.x & 63);
+    live = i < vh;
+    site = live ? i : vh - 1;
+  }
+  static unsigned blocks(long vh) { return nblk((vh + 63) / 64 * H, 4); }
+  template <int PX, typename T>
+  __device__ __forceinline__ void load(const void* p, long vh, cx<T> v[N]) const {
+    if constexpr (H == 2) SpinorIO<PX>::template load_half<1>(p, vh, site, h, v);
+    else SpinorIO<PX>::load(p, vh, site, v);
+  }
+  template <int PX, typename T>
+  __device__ __forceinline__ void store(void* p, long vh, const cx<T> v[N], int nts) const {
+    if (!live) return;
+    if constexpr (H == 2) {
+      if (nts) SpinorIO<PX>::template store_half<1>(p, vh, site, h, v);
+      else SpinorIO<PX>::template store_half<0>(p, vh, site, h, v);
+    } else {
+      if (nts) SpinorIO<PX>::template store<1>(p, vh, site, v);
+      else SpinorIO<PX>::template store<0>(p, vh, site, v);
+    }
+  }
+};
+
 // x += alpha_k p_k of the previous iteration (still pending: alpha is that iteration's,
 // p not yet overwritten), then p = r + beta p.  Folding the iterate update in here
 // saves one read of p per iteration against doing it in the s update; the host
 // applies a pending update itself (cg_xflush) before it reads x.  K > 0: the blocks take
-// the beta step themselves (beta_step), while their first fields load.
+// the beta step themselves (beta_step), while their fields load.
 template <int P, int PX, int K>
 __global__ void __launch_bounds__(256) cg_xpay_kernel(Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr,
                                                       const double* part_ss, long nw, long vh, int nts) {
   using T = typename Real<P>::T;
   using TX = typename Real<PX>::T;
+  constexpr int N = Share<P>::N;
   __shared__ double red[K ? 2 : 1][kSumThreads / 64];
-  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const Share<P> sh(vh);
   const int k = blockIdx.y;
   if (!sc[k].active) return;
-  if (K == 0 && i0 >= vh) return;
-  const bool live = i0 < vh;
-  const long i = live ? i0 : vh - 1;
+  if (K == 0 && !sh.live) return;
   const double alpha = sc[k].alpha;
   char* pp = static_cast<char*>(p.p) + k * p.stride;
   char* xp = static_cast<char*>(x.p) + k * x.stride;
   const char* rp = static_cast<const char*>(r.p) + k * r.stride;
-  if constexpr (P == F64 && PX == F64) {
-    // FP64 in halves of 6 components (p, r and x at once would spill)
-    cx<double> pv[6], rv[6], xv[6];
-    double beta = K ? 1.0 : sc[k].beta;
+  cx<T> pv[N], rv[N];
+  cx<TX> xv[N];
+  T beta = K ? T(1) : T(sc[k].beta);
+  if (alpha != 0.0 || beta != T(0)) sh.template load<P>(pp, vh, pv);
+  if (alpha != 0.0) sh.template load<PX>(xp, vh, xv);
+  sh.template load<P>(rp, vh, rv);
+  if constexpr (K > 0)
+    beta = T(beta_step<K>(sc[k], part_rr + k * nw, part_ss ? part_ss + k * nw : nullptr, nw, red));
+  if (alpha != 0.0) {
+    const TX ax = TX(alpha);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (alpha != 0.0 || beta != 0.0) SpinorIO<F64>::load_half<1>(pp, vh, i, h, pv);
-      if (alpha != 0.0) SpinorIO<F64>::load_half<1>(xp, vh, i, h, xv);
-      SpinorIO<F64>::load_half<1>(rp, vh, i, h, rv);
-      if constexpr (K > 0)
-        if (h == 0) beta = beta_step<K>(sc[k], part_rr + k * nw, part_ss ? part_ss + k * nw : nullptr, nw, red);
-      if (alpha != 0.0) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) xv[c] = {xv[c].re + alpha * pv[c].re, xv[c].im + alpha * pv[c].im};
-        if (live) {
-          if (nts) SpinorIO<F64>::store_half<1>(xp, vh, i, h, xv);
-          else SpinorIO<F64>::store_half<0>(xp, vh, i, h, xv);
-        }
-      }
-      if (beta != 0.0) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) rv[c] = rv[c] + beta * pv[c];
-      }
-      if (live) {
-        if (nts) SpinorIO<F64>::store_half<1>(pp, vh, i, h, rv);
-        else SpinorIO<F64>::store_half<0>(pp, vh, i, h, rv);
-      }
-    }
-  } else {
-    cx<T> pv[12], rv[12];
-    cx<TX> xv[12];
-    T beta = K ? T(1) : T(sc[k].beta);
-    if (alpha != 0.0 || beta != T(0)) SpinorIO<P>::load(pp, vh, i, pv);
-    if constexpr (K > 0) {
-      if (alpha != 0.0) SpinorIO<PX>::load(xp, vh, i, xv);
-      SpinorIO<P>::load(rp, vh, i, rv);
-      beta = T(beta_step<K>(sc[k], part_rr + k * nw, part_ss ? part_ss + k * nw : nullptr, nw, red));
-    }
-    if (alpha != 0.0) {
-      const TX ax = TX(alpha);
-      if (K == 0) SpinorIO<PX>::load(xp, vh, i, xv);
-#pragma unroll
-      for (int c = 0; c < 12; ++c) xv[c] = {xv[c].re + ax * TX(pv[c].re), xv[c].im + ax * TX(pv[c].im)};
-      if (live) {
-        if (nts) SpinorIO<PX>::template store<1>(xp, vh, i, xv);
-        else SpinorIO<PX>::template store<0>(xp, vh, i, xv);
-      }
-    }
-    if (K == 0) SpinorIO<P>::load(rp, vh, i, rv);
-    if (beta == T(0)) {
-      // restart (first iteration, after a restart, or converged): p = r
-#pragma unroll
-      for (int c = 0; c < 12; ++c) pv[c] = rv[c];
-    } else {
-#pragma unroll
-      for (int c = 0; c < 12; ++c) pv[c] = rv[c] + beta * pv[c];
-    }
-    if (live) {
-      if (nts) SpinorIO<P>::template store<1>(pp, vh, i, pv);
-      else SpinorIO<P>::template store<0>(pp, vh, i, pv);
-    }
+    for (int c = 0; c < N; ++c) xv[c] = {xv[c].re + ax * TX(pv[c].re), xv[c].im + ax * TX(pv[c].im)};
+    sh.template store<PX>(xp, vh, xv, nts);
   }
+  if (beta != T(0)) {  // else a restart (first iteration, after a restart, or converged): p = r
+#pragma unroll
+    for (int c = 0; c < N; ++c) rv[c] = rv[c] + beta * pv[c];
+  }
+  sh.template store<P>(pp, vh, rv, nts);
 }
 
-// s -= alpha t, with the 16-site partials of |s|^2.  K > 0: the blocks take the alpha step
-// themselves (alpha_step), while their fields load.
+// s -= alpha t, with the 64-site partials of |s|^2, a chunk's two halves added by the wave
+// of its first.  K > 0: the blocks take the alpha step themselves (alpha_step), while their
+// fields load.
 template <int P, int K>
 __global__ void __launch_bounds__(256) cg_update_kernel(Vec t, Vec s, CgScal* sc, const double* part_tt, long nw,
                                                         double* part, long vh, int nts) {
   using T = typename Real<P>::T;
-  __shared__ double red[kSumThreads / 64];
-  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr int N = Share<P>::N;
+  __shared__ double red[kSumThreads / 64], half[4];
+  const Share<P> sh(vh);
   const int k = blockIdx.y;
   if (!sc[k].active) return;
-  const bool live = i0 < vh;
-  const long i = live ? i0 : vh - 1;
   char* sp = static_cast<char*>(s.p) + k * s.stride;
   const char* tp = static_cast<const char*>(t.p) + k * t.stride;
+  cx<T> tv[N], sv[N];
+  sh.template load<P>(tp, vh, tv);
+  sh.template load<P>(sp, vh, sv);
+  T a;
+  if constexpr (K > 0) a = T(alpha_step<K>(sc[k], part_tt + k * nw, nw, red));
+  else a = T(sc[k].alpha);
   T n = T(0);
-  if constexpr (P == F64) {
-    double a = K ? 0.0 : sc[k].alpha;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      cx<double> tv[6], sv[6];
-      SpinorIO<F64>::load_half<1>(tp, vh, i, h, tv);
-      SpinorIO<F64>::load_half<1>(sp, vh, i, h, sv);
-      if constexpr (K > 0)
-        if (h == 0) a = alpha_step<K>(sc[k], part_tt + k * nw, nw, red);
-#pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        sv[c] = sv[c] - a * tv[c];
-        n += norm2(sv[c]);
-      }
-      if (live) {
-        if (nts) SpinorIO<F64>::store_half<1>(sp, vh, i, h, sv);
-        else SpinorIO<F64>::store_half<0>(sp, vh, i, h, sv);
-      }
-    }
-  } else {
-    cx<T> tv[12], sv[12];
-    SpinorIO<P>::load(tp, vh, i, tv);
-    SpinorIO<P>::load(sp, vh, i, sv);
-    T a;
-    if constexpr (K > 0) a = T(alpha_step<K>(sc[k], part_tt + k * nw, nw, red));
-    else a = T(sc[k].alpha);
-#pragma unroll
-    for (int c = 0; c < 12; ++c) {
-      sv[c] = sv[c] - a * tv[c];
-      n += norm2(sv[c]);
-    }
-    if (live) {
-      if (nts) SpinorIO<P>::template store<1>(sp, vh, i, sv);
-      else SpinorIO<P>::template store<0>(sp, vh, i, sv);
-    }
+  for (int c = 0; c < N; ++c) {
+    sv[c] = sv[c] - a * tv[c];
+    n += norm2(sv[c]);
   }
-  put_partial(part, vh, k, i0, live ? (double)n : 0.0);
+  sh.template store<P>(sp, vh, sv, nts);
+  double v = group64_sum(sh.live ? (double)n : 0.0);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if constexpr (Share<P>::H == 2) {
+    if (lane == 0) half[w] = v;
+    __syncthreads();
+    if (sh.h == 0) v = half[w] + half[w | 1];
+  }
+  if (lane == 0 && sh.h == 0 && sh.first < vh) part[(long)k * nw + sh.first / 64] = v;
 }
 
 // x += alpha p for one slot: a pending iterate update applied by the host
@@ -458,23 +428,23 @@ void launch_cg_ss(const double* part, long nw, CgScal* sc, int nrhs, hipStream_t
   hipLaunchKernelGGL(cg_ss_kernel, dim3(nrhs), dim3(kSumThreads), 0, st, part, nw, sc);
 }
 // Every block sums all the partials, which costs nrhs nw^2 reads and saves two one-block
-// launches and most of a third, about 13 us an iteration of one right-hand side.  Solves
-// with the steps apart and in the vector kernels (ms): 8^4 FP32 2.61 / 2.27, 16^3x32 FP64
-// 10.87 / 10.26, FP32 6.74 / 5.98, 6 RHS 19.6 / 18.7; 16^3x64 (nw 8192) FP32 11.8 / 11.0 but
-// 6 RHS, at nrhs nw^2 = 4e8, 42.6 / 43.2.
+// launches and most of a third.  Solves with the steps apart and in the vector kernels
+// (ms): 8^4 FP32 2.67 / 2.29, 16^3x32 FP64 16.61 / 15.58, FP32 7.97 / 7.32, 12 RHS 45.8 /
+// 45.3, 16^3x64 6 RHS (nrhs nw^2 = 2.5e7) 53.3 / 52.6; but 24^3x48 (nw 5184) FP16 25.8 /
+// 26.3, FP64 64.1 / 64.0, 4 RHS 102 / 106.
 int cg_step_chains(long nw, int nrhs) {
-  if (nw > 8 * kSumThreads || nrhs * nw * nw > 250000000) return 0;
-  return nw <= 4 * kSumThreads ? 4 : 8;
+  if (nw > 4 * kSumThreads || nrhs * nw * nw > 26000000) return 0;
+  return nw <= kSumThreads ? 1 : 4;
 }
 
 template <int P, int PX>
 static void xpay(Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr, const double* part_ss, long nw, long vh,
                  int nrhs, hipStream_t st) {
-  const dim3 g(nblk(vh, 256), nrhs), b(256);
+  const dim3 g(Share<P>::blocks(vh), nrhs), b(256);
   const int n = nt_store(P, vh, nrhs);  // p decides for x as well
   const int k = part_rr ? cg_step_chains(nw, nrhs) : 0;
-  if (k == 4) hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 4>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
-  else if (k) hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 8>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
+  if (k == 1) hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 1>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
+  else if (k) hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 4>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
   else hipLaunchKernelGGL((cg_xpay_kernel<P, PX, 0>), g, b, 0, st, r, p, x, sc, part_rr, part_ss, nw, vh, n);
 }
 void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, CgScal* sc, const double* part_rr,
@@ -494,11 +464,11 @@ void launch_cg_xflush(int prec, int xprec, Vec x, Vec p, double alpha, long vh, 
 template <int P>
 static void update(Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part, long vh, int nrhs,
                    hipStream_t st) {
-  const dim3 g(nblk(vh, 256), nrhs), b(256);
+  const dim3 g(Share<P>::blocks(vh), nrhs), b(256);
   const int n = nt_store(P, vh, nrhs);
   const int k = part_tt ? cg_step_chains(nw, nrhs) : 0;
-  if (k == 4) hipLaunchKernelGGL((cg_update_kernel<P, 4>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
-  else if (k) hipLaunchKernelGGL((cg_update_kernel<P, 8>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
+  if (k == 1) hipLaunchKernelGGL((cg_update_kernel<P, 1>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
+  else if (k) hipLaunchKernelGGL((cg_update_kernel<P, 4>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
   else hipLaunchKernelGGL((cg_update_kernel<P, 0>), g, b, 0, st, t, s, sc, part_tt, nw, part, vh, n);
 }
 void launch_cg_update(int prec, Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part_ss, long vh,

@@ -221,6 +221,13 @@ struct SpinorIO<F32> {
     for (int k = 0; k < 6; ++k)
       stp<NTS>(b + k * kSiteBlock, float4{v[2 * k].re, v[2 * k].im, v[2 * k + 1].re, v[2 * k + 1].im});
   }
+  template <int NTS = 0>
+  static __device__ __forceinline__ void store_half(void* base, long vh, long i, int h, const cx<T> v[6]) {
+    float4* b = site_block<6>(static_cast<float4*>(base), i) + 3 * h * kSiteBlock;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      stp<NTS>(b + k * kSiteBlock, float4{v[2 * k].re, v[2 * k].im, v[2 * k + 1].re, v[2 * k + 1].im});
+  }
 };
 
 __device__ __forceinline__ float h2f(unsigned short h) { return __half2float(__ushort_as_half(h)); }
@@ -557,6 +564,15 @@ __device__ __forceinline__ unsigned remap_block(unsigned b, unsigned nb, int on)
   if (!on) return b;
   unsigned x = b & 7u, k = b >> 3, q = nb >> 3, r = nb & 7u;
   return x * q + (x < r ? x : r) + k;
+}
+
+// deterministic butterfly sum over a wave, 16-lane groups first: one reduction partial per
+// 64-site chunk, with the same bits in every kernel that writes partials
+__device__ __forceinline__ double group64_sum(double v) {
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 16);
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
 }
 
 // a wave's LDS accesses are processed in order; this keeps the compiler from moving

@@ -13,8 +13,8 @@ struct Vec {
 };
 inline Vec vec(void* p, long stride = 0) { return Vec{p, stride}; }
 
-// number of 16-site reduction partials of one half lattice
-__host__ __device__ inline long n_partials(long vh) { return (vh + 15) / 16; }
+// number of 64-site reduction partials of one half lattice
+__host__ __device__ inline long n_partials(long vh) { return (vh + 63) / 64; }
 
 // ------------------------------------------------------------------ hop -----
 // block threads = sg * rb; the rb groups share sites (and link loads); a.rpw
