@@ -11,7 +11,7 @@ namespace qcu {
 size_t CgBatch::bytes_for(long vh, int prec, int cap) {
   size_t fb = spinor_bytes(F64, vh), pb = spinor_bytes(prec, vh), xb = spinor_bytes(iterate_precision(prec), vh);
   size_t s = 4 * fb * cap + (prec == F64 ? 4 : 5) * pb * cap + (prec == F64 ? 0 : xb * cap);
-  s += sizeof(double) * (4 * n_partials(vh) * cap + cap) + sizeof(CgScal) * cap + 2 * (size_t)vh * 192;
+  s += sizeof(double) * 4 * n_partials(vh) * cap + sizeof(CgScal) * cap + 2 * (size_t)vh * 192;
   return s;
 }
 
@@ -52,15 +52,15 @@ CgBatch::CgBatch(GaugeField& g, int prec, int recon, int t_boundary, bool clover
     xlo_.alloc((size_t)xb_ * cap_);
     X_ = vec(xlo_.p, xb_);
   }
-  part_.alloc(sizeof(double) * (4 * nw_ * cap_ + cap_));
+  part_.alloc(sizeof(double) * 4 * nw_ * cap_);
   double* pp = static_cast<double*>(part_.p);
   part_rr_ = pp;
   part_tt_ = pp + nw_ * cap_;
   part_ss_ = pp + 2 * nw_ * cap_;
-  sums_ = pp + 4 * nw_ * cap_;
   scal_.alloc(sizeof(CgScal) * cap_);
   dsc_ = static_cast<CgScal*>(scal_.p);
   QHIP(hipHostMalloc((void**)&hsc_, sizeof(CgScal) * cap_, 0));
+  QHIP(hipHostMalloc((void**)&hsum_, sizeof(double) * 3 * cap_, 0));
   rebind(g);
   const char* e = getenv("QCU_DEBUG");
   debug_ = e && e[0] && e[0] != '0';
@@ -78,6 +78,7 @@ void CgBatch::rebind(GaugeField& g) {
 CgBatch::~CgBatch() {
   clear_graphs();
   if (hsc_) (void)hipHostFree(hsc_);
+  if (hsum_) (void)hipHostFree(hsum_);
 }
 
 void CgBatch::clear_graphs() {
@@ -102,18 +103,6 @@ Vec CgBatch::at(Vec v, int r) const {
   return vec(static_cast<char*>(v.p) + (long)r * v.stride, v.stride);
 }
 
-double CgBatch::norm2_slot(Vec v, int r) {
-  double* part = part_ss_ + nw_ * cap_;  // spare partials region
-  launch_norm2(F64, at(v, r), vh_, 1, part, st_);
-  launch_sum_partials(part, nw_, 1, sums_, st_);
-  double out = 0.0;
-  QHIP(hipMemcpyAsync(&out, sums_, sizeof(double), hipMemcpyDeviceToHost, st_));
-  QHIP(hipStreamSynchronize(st_));
-  return out;
-}
-
-// out = Mhat in (Mhat^dag if dag) for slots [r0, r0 + n), each with its own kappa and
-// clover; tmp holds the odd intermediate
 void CgBatch::mhat(int prec, int dag, Vec in, Vec out, Vec tmp, int r0, int n, double* partials) {
   if (r0 < 0 || n < 1 || r0 + n > n_) throw Error(QCU_ERROR_STATE, "internal: batch slot range out of range");
   const void* c1[kMaxRhs];
@@ -135,8 +124,7 @@ void CgBatch::mhat(int prec, int dag, Vec in, Vec out, Vec tmp, int r0, int n, d
 void CgBatch::add(const SlotSpec& spec) { add_slots(&spec, 1); }
 
 // The m new slots take [n_, n_ + m); their FP64 set-up runs batched over that run (a
-// batched hop gives every slot the bits of its own launch), with two synchronisations
-// in all.
+// batched hop gives every slot the bits of its own launch), with one synchronisation.
 void CgBatch::add_slots(const SlotSpec* specs, int m) {
   QREQ(m >= 1 && n_ + m <= cap_, "batch is full");
   for (int j = 0; j < m; ++j) check_operator(specs[j]);
@@ -145,6 +133,7 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
     Slot sl;
     sl.spec = specs[j];
     sl.updates = 0;
+    sl.folded = true;
     sl.cf = nullptr;
     if (clover_) {
       sl.cf = g_->clover(sl.spec.kappa * sl.spec.csw, F64);
@@ -154,7 +143,7 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
     slots_.push_back(sl);
   }
   n_ += m;
-  if (clover_) QHIP(hipStreamSynchronize(ctx().stream));  // clover fields built there
+  if (clover_ && st_ != ctx().stream) QHIP(hipStreamSynchronize(ctx().stream));  // clover fields built there
   // b_e in shi_, b_o in t64_ (both scratch until the iteration starts)
   for (int r = r0; r <= r1; ++r) {
     const char* b = static_cast<const char*>(source_aos(slots_[r]));
@@ -162,18 +151,8 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
     launch_spinor_from_aos(F64, b + vh_ * 192, 0, at(t64_, r), vh_, 1, st_);
   }
   QHIP(hipGetLastError());
-  std::vector<double> ne(m), no(m);
-  norm2_run(shi_, r0, r1, ne.data());
-  norm2_run(t64_, r0, r1, no.data());
-  QHIP(hipStreamSynchronize(st_));
-  for (int j = 0; j < m; ++j) {
-    slots_[r0 + j].bnorm2 = ne[j] + no[j];
-    if (!std::isfinite(slots_[r0 + j].bnorm2)) {
-      slots_.resize(r0);
-      n_ = r0;
-      throw Error(QCU_ERROR_NOT_FINITE, "source contains NaN or Inf");
-    }
-  }
+  const double* ne = norm2_run(shi_, r0, r1, 0);
+  const double* no = norm2_run(t64_, r0, r1, 1);
   // b^ = b_e + kappa D_eo A_oo^-1 b_o, A_oo^-1 b_o in place over runs sharing a clover
   const void* none[kMaxRhs];
   double kap[kMaxRhs];
@@ -192,17 +171,22 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
   hop_v(*g_, F64, recon_, EPI_XPAY, 0, 0, (double)tbc_, at(t64_, r0), at(bh_, r0), at(shi_, r0), none, kap, m,
         nullptr, st_);
   launch_zero(F64, at(xe_, r0), vh_, m, st_);
-  for (int r = r0; r <= r1; ++r)
-    QHIP(hipMemcpyAsync(at(shi_, r).p, at(bh_, r).p, fb_, hipMemcpyDeviceToDevice, st_));
+  launch_spinor_convert(F64, at(bh_, r0), prec_, at(S_, r0), vh_, m, 0, st_);
   if (prec_ != F64) {
-    launch_spinor_convert(F64, at(shi_, r0), prec_, at(S_, r0), vh_, m, 0, st_);
     launch_zero(xprec_, at(X_, r0), vh_, m, st_);
   }
   launch_zero(prec_, at(P_, r0), vh_, m, st_);  // scratch may hold stale, non-finite bits
   QHIP(hipGetLastError());
-  std::vector<double> ss0(m);
-  norm2_run(shi_, r0, r1, ss0.data());
+  const double* ss0 = norm2_run(bh_, r0, r1, 2);
   QHIP(hipStreamSynchronize(st_));
+  for (int j = 0; j < m; ++j) {
+    slots_[r0 + j].bnorm2 = ne[j] + no[j];
+    if (!std::isfinite(slots_[r0 + j].bnorm2)) {
+      slots_.resize(r0);
+      n_ = r0;
+      throw Error(QCU_ERROR_NOT_FINITE, "source contains NaN or Inf");
+    }
+  }
   const auto t0 = std::chrono::steady_clock::now();
   std::vector<char> done(n_, 0);
   bool any = false;
@@ -222,12 +206,13 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
   }
   clear_graphs();
   if (any) finish_slots(done);  // compaction moves slots within [r0, n_) only
-  if (n_ > r0) QHIP(hipMemcpyAsync(dsc_ + r0, hsc_ + r0, sizeof(CgScal) * (n_ - r0), hipMemcpyHostToDevice, st_));
+  if (n_ > r0) launch_cg_put(hsc_ + r0, dsc_ + r0, n_ - r0, st_);
 }
 
 void CgBatch::launch_chunk() {
   const int n = n_;
   if (n == 0) return;
+  for (Slot& sl : slots_) sl.folded = false;
   // few partials: the vector kernels take the scalar steps, six launches an iteration
   // instead of nine; the last iteration's |s|^2 is looked at by the one-block kernel
   const bool in_step = cg_step_chains(nw_, n) != 0;
@@ -239,7 +224,8 @@ void CgBatch::launch_chunk() {
     mhat(prec_, 0, P_, T_, TO_, 0, n, part_tt_);
     if (!in_step) launch_cg_alpha(part_tt_, nw_, dsc_, n, st_);
     launch_cg_update(prec_, T_, S_, dsc_, in_step ? part_tt_ : nullptr, nw_, part_ss_, vh_, n, st_);
-    if (!in_step || i == sp_.chunk - 1) launch_cg_ss(part_ss_, nw_, dsc_, n, st_);
+    const bool last = i == sp_.chunk - 1;
+    if (!in_step || last) launch_cg_ss(part_ss_, nw_, dsc_, last ? hsc_ : nullptr, n, st_);
   };
   if (!sp_.graph) {
     for (int i = 0; i < sp_.chunk; ++i) iteration(i);
@@ -258,35 +244,29 @@ void CgBatch::launch_chunk() {
 }
 
 // The iterate update x += alpha p of a chunk's last iteration is applied by the next
-// iteration's p update; before the host reads x it applies it here (with the host's
-// copy of alpha, which it then clears, so the device does not apply it again).
-void CgBatch::flush_x(int r) {
-  CgScal& c = hsc_[r];
-  if (c.alpha != 0.0) launch_cg_xflush(prec_, xprec_, at(X_, r), at(P_, r), c.alpha, vh_, st_);
-  c.alpha = 0.0;
-}
-
-// s = b^ - Mhat x in FP64 for slot r (the low-precision iterate folded into x first)
-double CgBatch::reliable_update(int r) {
-  flush_x(r);
-  if (prec_ != F64) {
-    launch_spinor_convert(xprec_, at(X_, r), F64, at(xe_, r), vh_, 1, 1, st_);
-    launch_zero(xprec_, at(X_, r), vh_, 1, st_);
+// iteration's p update; before the host reads the iterates of the slots in mask (bit r -
+// lo) it applies it here (with its copy of alpha, which it then clears, so the device does
+// not apply it again), and folds a low-precision iterate into xe_.
+void CgBatch::fold_x(int lo, int hi, unsigned mask) {
+  SlotScal a;
+  a.mask = 0;
+  for (int r = lo; r <= hi; ++r) {
+    CgScal& c = hsc_[r];
+    a.v[r - lo] = c.alpha;
+    if (!((mask >> (r - lo)) & 1u) || slots_[r].folded) continue;
+    a.mask |= 1u << (r - lo);
+    if (prec_ == F64 && c.alpha != 0.0) launch_cg_xflush(at(X_, r), at(P_, r), c.alpha, vh_, st_);
+    c.alpha = 0.0;
+    slots_[r].folded = true;
   }
-  mhat(F64, 0, xe_, shi_, t64_, r, 1, nullptr);
-  launch_axpby(F64, 1.0, at(bh_, r), -1.0, at(shi_, r), vh_, 1, st_);
-  double ss = norm2_slot(shi_, r);
-  if (prec_ != F64) launch_spinor_convert(F64, at(shi_, r), prec_, at(S_, r), vh_, 1, 0, st_);
-  slots_[r].updates++;
-  if (debug_) fprintf(stderr, "qcu cg reliable update tag=%llu |s|^2=%.6e\n", (unsigned long long)slots_[r].spec.tag, ss);
-  return ss;
+  if (prec_ != F64 && a.mask)
+    launch_cg_fold(prec_, at(X_, lo), at(P_, lo), at(xe_, lo), a, vh_, hi - lo + 1, st_);
 }
 
 void CgBatch::harvest() {
   const int n = n_;
   if (n == 0) return;
-  QHIP(hipMemcpyAsync(hsc_, dsc_, sizeof(CgScal) * n, hipMemcpyDeviceToHost, st_));
-  QHIP(hipStreamSynchronize(st_));
+  QHIP(hipStreamSynchronize(st_));  // the chunk's last kernel has written hsc_
   if (debug_)
     for (int r = 0; r < n; ++r)
       fprintf(stderr, "qcu cg tag=%llu it=%d ss=%.6e gamma=%.6e tt=%.6e alpha=%.6e beta=%.6e conv=%d brk=%d\n",
@@ -330,7 +310,7 @@ void CgBatch::harvest() {
     else if (upd[r] && (hsc_[r].converged || cap[r])) done[r] = 1;
   }
   finish_slots(done);
-  if (n_ > 0) QHIP(hipMemcpyAsync(dsc_, hsc_, sizeof(CgScal) * n_, hipMemcpyHostToDevice, st_));
+  if (n_ > 0 && (hi >= lo || n_ < n)) launch_cg_put(hsc_, dsc_, n_, st_);
 }
 
 // s = b^ - Mhat x in FP64 for the slots r in [lo, hi] with upd[r] set, the
@@ -341,34 +321,29 @@ void CgBatch::harvest() {
 std::vector<double> CgBatch::reliable_updates(int lo, int hi, const std::vector<char>& upd) {
   const int n = hi - lo + 1;
   std::vector<double> out(n, 0.0);
-  if (prec_ == F64) {
+  unsigned mask = 0;
+  for (int r = lo; r <= hi; ++r)
+    if (upd[r]) mask |= 1u << (r - lo);
+  auto run = [&](int a, int b, unsigned m) {  // slots [a, b], those in m updated
+    fold_x(a, b, m);
+    mhat(F64, 0, xe_, shi_, t64_, a, b - a + 1, nullptr);
+    const double* ss = residual_run(bh_, shi_, a, b, m, 0);
+    QHIP(hipStreamSynchronize(st_));
+    std::copy(ss, ss + (b - a + 1), out.begin() + (a - lo));
+  };
+  if (prec_ != F64) {
+    run(lo, hi, mask);
+  } else {
     for (int r = lo; r <= hi; ++r)
-      if (upd[r]) out[r - lo] = reliable_update(r);
-    return out;
+      if (upd[r]) run(r, r, 1u);
   }
   for (int r = lo; r <= hi; ++r) {
     if (!upd[r]) continue;
-    flush_x(r);
-    launch_spinor_convert(xprec_, at(X_, r), F64, at(xe_, r), vh_, 1, 1, st_);
-    launch_zero(xprec_, at(X_, r), vh_, 1, st_);
-  }
-  mhat(F64, 0, xe_, shi_, t64_, lo, n, nullptr);
-  launch_axpby(F64, 1.0, at(bh_, lo), -1.0, at(shi_, lo), vh_, n, st_);
-  double* part = part_ss_ + nw_ * cap_;
-  launch_norm2(F64, at(shi_, lo), vh_, n, part, st_);
-  launch_sum_partials(part, nw_, n, sums_, st_);
-  QHIP(hipMemcpyAsync(out.data(), sums_, sizeof(double) * n, hipMemcpyDeviceToHost, st_));
-  for (int r = lo; r <= hi; ++r) {
-    if (!upd[r]) continue;
-    launch_spinor_convert(F64, at(shi_, r), prec_, at(S_, r), vh_, 1, 0, st_);
     slots_[r].updates++;
+    if (debug_)
+      fprintf(stderr, "qcu cg reliable update tag=%llu |s|^2=%.6e\n", (unsigned long long)slots_[r].spec.tag,
+              out[r - lo]);
   }
-  QHIP(hipStreamSynchronize(st_));
-  if (debug_)
-    for (int r = lo; r <= hi; ++r)
-      if (upd[r])
-        fprintf(stderr, "qcu cg reliable update tag=%llu |s|^2=%.6e\n", (unsigned long long)slots_[r].spec.tag,
-                out[r - lo]);
   return out;
 }
 
@@ -381,14 +356,22 @@ const void* CgBatch::source_aos(const Slot& sl) {
   return aos_.p;
 }
 
-// |v|^2 of slots [lo, hi] of field v into out[0 .. hi - lo] (enqueued; read after a
-// synchronisation); the per-slot sums are those of norm2_slot
-void CgBatch::norm2_run(Vec v, int lo, int hi, double* out) {
-  const int m = hi - lo + 1;
-  double* part = part_ss_ + nw_ * cap_;  // spare partials region
-  launch_norm2(F64, at(v, lo), vh_, m, part, st_);
-  launch_sum_partials(part, nw_, m, sums_, st_);
-  QHIP(hipMemcpyAsync(out, sums_, sizeof(double) * m, hipMemcpyDeviceToHost, st_));
+// the sums of m slots' partials in the spare partials region, straight to pinned memory
+const double* CgBatch::sum_run(int m, int which) {
+  double* out = hsum_ + which * cap_;
+  launch_sum_partials(part_ss_ + nw_ * cap_, nw_, m, out, st_);
+  return out;
+}
+
+const double* CgBatch::norm2_run(Vec v, int lo, int hi, int which) {
+  launch_norm2(F64, at(v, lo), vh_, hi - lo + 1, part_ss_ + nw_ * cap_, st_);
+  return sum_run(hi - lo + 1, which);
+}
+
+// |b - t|^2 of slots [lo, hi]; the residual of those in mask goes to the loop's s
+const double* CgBatch::residual_run(Vec b, Vec t, int lo, int hi, unsigned mask, int which) {
+  launch_residual(prec_, at(b, lo), at(t, lo), at(S_, lo), mask, vh_, hi - lo + 1, part_ss_ + nw_ * cap_, st_);
+  return sum_run(hi - lo + 1, which);
 }
 
 // x_o = A_oo^-1 (b_o + kappa D_oe x_e) and the true residual |b - M x|^2 of slots
@@ -397,11 +380,7 @@ void CgBatch::norm2_run(Vec v, int lo, int hi, double* out) {
 // bh_, shi_ and t64_ as scratch (b^ is no longer needed).
 void CgBatch::finish_run(int lo, int hi, std::vector<double>& nr) {
   const int m = hi - lo + 1;
-  for (int r = lo; r <= hi; ++r) flush_x(r);
-  if (prec_ != F64) {
-    launch_spinor_convert(xprec_, at(X_, lo), F64, at(xe_, lo), vh_, m, 1, st_);
-    launch_zero(xprec_, at(X_, lo), vh_, m, st_);
-  }
+  fold_x(lo, hi, (1u << m) - 1);
   const void* none[kMaxRhs];
   const void* a_o[kMaxRhs];
   const void* a_e[kMaxRhs];
@@ -427,16 +406,14 @@ void CgBatch::finish_run(int lo, int hi, std::vector<double>& nr) {
     hop_v(*g_, F64, recon_, EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), xo, bq, none, kap, m, nullptr, st_);
   }
   // r = b - M x with M = A - kappa D, odd then even parity
-  std::vector<double> ro(m), re(m);
   hop_v(*g_, F64, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 1, 0, (double)tbc_, at(xe_, lo), tmp, xo,
         clover_ ? a_o : none, mkap, m, nullptr, st_);
-  launch_axpby(F64, 1.0, bq, -1.0, tmp, vh_, m, st_);
-  norm2_run(bh_, lo, hi, ro.data());
+  const double* ro = residual_run(t64_, bh_, lo, hi, 0, 0);
   for (int r = lo; r <= hi; ++r)  // b_e
     launch_spinor_from_aos(F64, source_aos(slots_[r]), 0, at(t64_, r), vh_, 1, st_);
   hop_v(*g_, F64, recon_, clover_ ? EPI_CLOV_XPAY : EPI_XPAY, 0, 0, (double)tbc_, xo, tmp, at(xe_, lo),
         clover_ ? a_e : none, mkap, m, nullptr, st_);
-  launch_axpby(F64, 1.0, bq, -1.0, tmp, vh_, m, st_);
+  const double* re = residual_run(t64_, bh_, lo, hi, 0, 1);
   for (int r = lo; r <= hi; ++r) {
     const Slot& sl = slots_[r];
     if (sl.spec.x) {
@@ -444,7 +421,6 @@ void CgBatch::finish_run(int lo, int hi, std::vector<double>& nr) {
       launch_spinor_to_aos(F64, at(shi_, r), static_cast<char*>(sl.spec.x) + vh_ * 192, 0, vh_, 1, st_);
     }
   }
-  norm2_run(bh_, lo, hi, re.data());
   QHIP(hipGetLastError());
   QHIP(hipStreamSynchronize(st_));
   for (int r = lo; r <= hi; ++r) nr[r] = re[r - lo] + ro[r - lo];  // |r_e|^2 + |r_o|^2

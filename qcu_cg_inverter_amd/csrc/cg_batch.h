@@ -73,26 +73,29 @@ class CgBatch {
     SlotSpec spec;
     double bnorm2;
     int updates;
+    bool folded;  // x is all in xe_ (no iteration since)
     CloverField* cf;
     std::chrono::steady_clock::time_point t0;
   };
   void check_operator(const SlotSpec& s) const;
   void mhat(int prec, int dag, Vec in, Vec out, Vec tmp, int r0, int n, double* partials);
-  void flush_x(int r);
-  double reliable_update(int r);
+  void fold_x(int lo, int hi, unsigned mask);
   std::vector<double> reliable_updates(int lo, int hi, const std::vector<char>& upd);
   // finish the slots marked in `done` (1 converged or capped, 2 broke down), their FP64
   // work batched over contiguous runs of marked slots, then compact top down
   void finish_slots(const std::vector<char>& done);
   // x_o and |b - M x|^2 (into nr[r]) for slots [lo, hi], solutions written out
   void finish_run(int lo, int hi, std::vector<double>& nr);
-  // |v|^2 of slots [lo, hi] of field v, in order (asynchronous: valid after a sync)
-  void norm2_run(Vec v, int lo, int hi, double* out);
+  // |v|^2 of slots [lo, hi] of field v, in order (asynchronous: valid after a sync, until
+  // the run `which` of hsum_, 0 to 2, is used again)
+  const double* norm2_run(Vec v, int lo, int hi, int which);
+  // |b - t|^2 likewise; the residual of those in mask (bit r - lo) goes to the loop's s
+  const double* residual_run(Vec b, Vec t, int lo, int hi, unsigned mask, int which);
+  const double* sum_run(int m, int which);
   const void* source_aos(const Slot& sl);
   void move_slot(int from, int to);
   // slot r of a batch field; v must be the field's base (slot 0), never a slot view
   Vec at(Vec v, int r) const;
-  double norm2_slot(Vec v, int r);
   void clear_graphs();
 
   GaugeField* g_;
@@ -104,9 +107,10 @@ class CgBatch {
   long vh_, nw_, fb_, pb_, xb_;
   DevBuf f64_, slo_, xlo_, part_, scal_, tmp_, aos_;
   Vec bh_, xe_, shi_, t64_, S_, R_, P_, T_, TO_, X_;
-  double *part_rr_, *part_tt_, *part_ss_, *sums_;
+  double *part_rr_, *part_tt_, *part_ss_;
   CgScal* dsc_;
-  CgScal* hsc_;
+  CgScal* hsc_ = nullptr;  // pinned: the last chunk's scalars
+  double* hsum_ = nullptr;  // pinned: sums the host waits for, of three runs
   std::vector<Slot> slots_;
   std::vector<SlotResult> finished_;
   std::vector<std::pair<hipGraph_t, hipGraphExec_t>> graphs_;  // per active count, built lazily

@@ -155,17 +155,26 @@ __global__ void __launch_bounds__(kSumThreads) cg_alpha_kernel(const double* par
   }
 }
 
-__global__ void __launch_bounds__(kSumThreads) cg_ss_kernel(const double* part, long nw, CgScal* sc) {
+// host: the scalars as they leave the chunk, to the batch's pinned copy (a copy command
+// and its hand-over from kernel to kernel take about 20 us)
+__global__ void __launch_bounds__(kSumThreads) cg_ss_kernel(const double* part, long nw, CgScal* sc, CgScal* host) {
   CgScal& s = sc[blockIdx.x];
-  if (!s.active) return;
-  double ss = block_sum_partials(part + (long)blockIdx.x * nw, nw);
-  if (threadIdx.x == 0) {
-    if (!s.converged) {
-      s.ss = ss;
-      s.iter += 1;
-      if (ss <= s.target2) s.converged = 1;
+  if (s.active) {
+    double ss = block_sum_partials(part + (long)blockIdx.x * nw, nw);
+    if (threadIdx.x == 0) {
+      if (!s.converged) {
+        s.ss = ss;
+        s.iter += 1;
+        if (ss <= s.target2) s.converged = 1;
+      }
     }
   }
+  if (host && threadIdx.x == 0) host[blockIdx.x] = s;
+}
+
+// the way back, of n slots the host has changed
+__global__ void cg_put_kernel(const CgScal* host, CgScal* sc, int n) {
+  if ((int)threadIdx.x < n) sc[threadIdx.x] = host[threadIdx.x];
 }
 
 // The sum of a right-hand side's nw partials, by every block that needs it (256 threads, nw
@@ -364,21 +373,75 @@ __global__ void __launch_bounds__(256) cg_update_kernel(Vec t, Vec s, CgScal* sc
   if (lane == 0 && sh.h == 0 && sh.first < vh) part[(long)k * nw + sh.first / 64] = v;
 }
 
-// x += alpha p for one slot: a pending iterate update applied by the host
-template <int P, int PX>
+// x += alpha p for one slot of an FP64 loop: a pending iterate update applied by the host
 __global__ void cg_xflush_kernel(Vec x, Vec p, double alpha, long vh) {
-  using T = typename Real<P>::T;
-  using TX = typename Real<PX>::T;
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= vh) return;
-  cx<T> pv[12];
-  cx<TX> xv[12];
-  SpinorIO<P>::load(p.p, vh, i, pv);
-  SpinorIO<PX>::load(x.p, vh, i, xv);
-  const TX ax = TX(alpha);
+  cx<double> pv[12], xv[12];
+  SpinorIO<F64>::load(p.p, vh, i, pv);
+  SpinorIO<F64>::load(x.p, vh, i, xv);
 #pragma unroll
-  for (int c = 0; c < 12; ++c) xv[c] = {xv[c].re + ax * TX(pv[c].re), xv[c].im + ax * TX(pv[c].im)};
-  SpinorIO<PX>::store(x.p, vh, i, xv);
+  for (int c = 0; c < 12; ++c) xv[c] = {xv[c].re + alpha * pv[c].re, xv[c].im + alpha * pv[c].im};
+  SpinorIO<F64>::store(x.p, vh, i, xv);
+}
+
+// The slots of a low-precision loop in `mask`: the pending update x += alpha p, xe += x in
+// FP64, and x = 0, in one pass (24^3x48 FP16: 35 us, 50 in three passes).
+template <int P>
+__global__ void cg_fold_kernel(Vec x, Vec p, Vec xe, const SlotScal a, long vh, int nts) {
+  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int r = blockIdx.y;
+  if (i >= vh || !((a.mask >> r) & 1u)) return;
+  char* xp = static_cast<char*>(x.p) + r * x.stride;
+  char* ep = static_cast<char*>(xe.p) + r * xe.stride;
+  cx<float> xv[12], z[12];
+  SpinorIO<F32>::load(xp, vh, i, xv);
+  if (a.v[r] != 0.0) {
+    cx<float> pv[12];
+    SpinorIO<P>::load(static_cast<const char*>(p.p) + r * p.stride, vh, i, pv);
+    const float ax = (float)a.v[r];
+#pragma unroll
+    for (int c = 0; c < 12; ++c) xv[c] = {xv[c].re + ax * pv[c].re, xv[c].im + ax * pv[c].im};
+  }
+#pragma unroll
+  for (int c = 0; c < 12; ++c) z[c] = {0.f, 0.f};
+  SpinorIO<F32>::store(xp, vh, i, z);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    cx<double> e[6];
+    SpinorIO<F64>::load_half<1>(ep, vh, i, h, e);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) e[c] = {e[c].re + (double)xv[6 * h + c].re, e[c].im + (double)xv[6 * h + c].im};
+    if (nts) SpinorIO<F64>::store_half<1>(ep, vh, i, h, e);
+    else SpinorIO<F64>::store_half<0>(ep, vh, i, h, e);
+  }
+}
+
+// The FP64 residual b - t of the slots, its |.|^2 partials, and for those in `mask` its
+// store to s in the loop's precision (t itself in an FP64 loop); nothing else is kept.
+template <int P>
+__global__ void residual_kernel(Vec b, Vec t, Vec s, unsigned mask, double* part, long vh) {
+  using T = typename Real<P>::T;
+  const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int r = blockIdx.y;
+  const bool live = i0 < vh;
+  const long i = live ? i0 : vh - 1;
+  cx<double> bv[12], tv[12];
+  SpinorIO<F64>::load(static_cast<const char*>(b.p) + r * b.stride, vh, i, bv);
+  SpinorIO<F64>::load(static_cast<const char*>(t.p) + r * t.stride, vh, i, tv);
+  double n = 0.0;
+#pragma unroll
+  for (int c = 0; c < 12; ++c) {
+    tv[c] = bv[c] - tv[c];
+    n += norm2(tv[c]);
+  }
+  if (live && ((mask >> r) & 1u)) {
+    cx<T> o[12];
+#pragma unroll
+    for (int c = 0; c < 12; ++c) o[c] = {T(tv[c].re), T(tv[c].im)};
+    SpinorIO<P>::store(static_cast<char*>(s.p) + r * s.stride, vh, i, o);
+  }
+  put_partial(part, vh, r, i0, live ? n : 0.0);
 }
 
 // plain streaming copy, the bandwidth and PMC-counter reference kernel: one 16-byte
@@ -424,8 +487,20 @@ void launch_cg_beta(const double* part, long nw, CgScal* sc, int nrhs, hipStream
 void launch_cg_alpha(const double* part, long nw, CgScal* sc, int nrhs, hipStream_t st) {
   hipLaunchKernelGGL(cg_alpha_kernel, dim3(nrhs), dim3(kSumThreads), 0, st, part, nw, sc);
 }
-void launch_cg_ss(const double* part, long nw, CgScal* sc, int nrhs, hipStream_t st) {
-  hipLaunchKernelGGL(cg_ss_kernel, dim3(nrhs), dim3(kSumThreads), 0, st, part, nw, sc);
+void launch_cg_ss(const double* part, long nw, CgScal* sc, CgScal* host, int nrhs, hipStream_t st) {
+  hipLaunchKernelGGL(cg_ss_kernel, dim3(nrhs), dim3(kSumThreads), 0, st, part, nw, sc, host);
+}
+void launch_cg_put(const CgScal* host, CgScal* sc, int n, hipStream_t st) {
+  hipLaunchKernelGGL(cg_put_kernel, dim3(1), dim3(64), 0, st, host, sc, n);
+}
+void launch_cg_fold(int prec, Vec x, Vec p, Vec xe, const SlotScal& a, long vh, int nrhs, hipStream_t st) {
+  const dim3 g(nblk(vh, 256), nrhs), b(256);
+  const int nts = nt_store(F64, vh, nrhs);
+  if (prec == F32) hipLaunchKernelGGL(cg_fold_kernel<F32>, g, b, 0, st, x, p, xe, a, vh, nts);
+  else hipLaunchKernelGGL(cg_fold_kernel<F16>, g, b, 0, st, x, p, xe, a, vh, nts);
+}
+void launch_residual(int prec, Vec b, Vec t, Vec s, unsigned mask, long vh, int nrhs, double* part, hipStream_t st) {
+  QCU_PSW(prec, residual_kernel, dim3(nblk(vh, 256), nrhs), dim3(256), 0, st, b, t, s, mask, part, vh);
 }
 // Every block sums all the partials, which costs nrhs nw^2 reads and saves two one-block
 // launches and most of a third.  Solves with the steps apart and in the vector kernels
@@ -453,13 +528,8 @@ void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, CgScal* sc, const 
   else if (prec == F32) xpay<F32, F32>(r, p, x, sc, part_rr, part_ss, nw, vh, nrhs, st);
   else xpay<F16, F32>(r, p, x, sc, part_rr, part_ss, nw, vh, nrhs, st);
 }
-void launch_cg_xflush(int prec, int xprec, Vec x, Vec p, double alpha, long vh, hipStream_t st) {
-  dim3 g(nblk(vh, 256)), b(256);
-  if (prec == F64) hipLaunchKernelGGL((cg_xflush_kernel<F64, F64>), g, b, 0, st, x, p, alpha, vh);
-  else if (prec == F32 && xprec == F64) hipLaunchKernelGGL((cg_xflush_kernel<F32, F64>), g, b, 0, st, x, p, alpha, vh);
-  else if (prec == F32) hipLaunchKernelGGL((cg_xflush_kernel<F32, F32>), g, b, 0, st, x, p, alpha, vh);
-  else if (xprec == F64) hipLaunchKernelGGL((cg_xflush_kernel<F16, F64>), g, b, 0, st, x, p, alpha, vh);
-  else hipLaunchKernelGGL((cg_xflush_kernel<F16, F32>), g, b, 0, st, x, p, alpha, vh);
+void launch_cg_xflush(Vec x, Vec p, double alpha, long vh, hipStream_t st) {
+  hipLaunchKernelGGL(cg_xflush_kernel, dim3(nblk(vh, 256)), dim3(256), 0, st, x, p, alpha, vh);
 }
 template <int P>
 static void update(Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part, long vh, int nrhs,

@@ -68,7 +68,8 @@ void launch_zero(int prec, Vec v, long vh, int nrhs, hipStream_t st);
 void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t st);
 // partials[r][w] = sum over wave w of |v_r|^2
 void launch_norm2(int prec, Vec v, long vh, int nrhs, double* partials, hipStream_t st);
-// out[r] = sum_w partials[r][w] in a fixed order (one block per right-hand side)
+// out[r] = sum_w partials[r][w] in a fixed order (one block per right-hand side); out may
+// be pinned host memory
 void launch_sum_partials(const double* partials, long nw, int nrhs, double* out, hipStream_t st);
 // y = a x + b y (F64 or same-precision fields)
 void launch_axpby(int prec, double a, Vec x, double b, Vec y, long vh, int nrhs, hipStream_t st);
@@ -78,7 +79,10 @@ void launch_clover_apply(int prec, const void* clov, Vec in, Vec out, long vh, i
 // CGLS steps (see solver.cpp).  All skip right-hand sides with active == 0.
 void launch_cg_beta(const double* part_rr, long nw, CgScal* sc, int nrhs, hipStream_t st);
 void launch_cg_alpha(const double* part_tt, long nw, CgScal* sc, int nrhs, hipStream_t st);
-void launch_cg_ss(const double* part_ss, long nw, CgScal* sc, int nrhs, hipStream_t st);
+// host: null, or pinned memory that receives a copy of the scalars
+void launch_cg_ss(const double* part_ss, long nw, CgScal* sc, CgScal* host, int nrhs, hipStream_t st);
+// sc[0 .. n) = host[0 .. n), pinned memory that stays as it is until the kernel has run
+void launch_cg_put(const CgScal* host, CgScal* sc, int n, hipStream_t st);
 // nonzero: nrhs right-hand sides of nw partials take their scalar steps inside the vector
 // kernels below (pass the partials); 0: by the one-block kernels above, before them
 int cg_step_chains(long nw, int nrhs);
@@ -90,8 +94,18 @@ void launch_cg_xpay(int prec, int xprec, Vec r, Vec p, Vec x, CgScal* sc, const 
 // s -= alpha t ; partials of |s|^2.  With part_tt (|t|^2) the blocks take the alpha step.
 void launch_cg_update(int prec, Vec t, Vec s, CgScal* sc, const double* part_tt, long nw, double* part_ss, long vh,
                       int nrhs, hipStream_t st);
-// x += alpha p for one right-hand side (a pending iterate update, applied by the host)
-void launch_cg_xflush(int prec, int xprec, Vec x, Vec p, double alpha, long vh, hipStream_t st);
+// x += alpha p for one right-hand side of an FP64 loop (a pending iterate update, applied
+// by the host)
+void launch_cg_xflush(Vec x, Vec p, double alpha, long vh, hipStream_t st);
+// a scalar per right-hand side, and those a launch is about (bit r of mask)
+struct SlotScal {
+  double v[kMaxRhs];
+  unsigned mask;
+};
+// x += v p ; xe += x ; x = 0, with x in FP32 and p in `prec` (FP32 or FP16)
+void launch_cg_fold(int prec, Vec x, Vec p, Vec xe, const SlotScal& a, long vh, int nrhs, hipStream_t st);
+// partials of |b - t|^2 in FP64; the residual of those in mask stored to s in `prec`
+void launch_residual(int prec, Vec b, Vec t, Vec s, unsigned mask, long vh, int nrhs, double* part, hipStream_t st);
 
 // --------------------------------------------------------------- clover -----
 // A = 1 + ck T and A^-1, packed F64, of both parities (only = -1) or one; any null output

@@ -211,3 +211,27 @@ def test_dropin_import(q, L, prec):
     finally:
         sp = q.default_solve_params(tol=1e-12, precision=0)
         q.check(q.lib().qcuSetDefaultSolve(ctypes.byref(sp)))
+
+
+@pytest.mark.parametrize("L", LATS)
+@pytest.mark.parametrize("prec", [0, 1, 2])
+def test_solve_residual_by_oracle(q, L, prec):
+    """Residual updates, iterate folds and finishes of slots that converge apart, on half
+    volumes off the 64-site chunk: the true residual the solve reports is the oracle's (both
+    in FP64, whose rounding of b - M x is below 1e-14 |b|) and is below the tolerance."""
+    g = q.Gauge.random(L, seed=45, eps=0.2)
+    gref = g.to_numpy()
+    for csw in (0.0, 1.0):
+        op = q.Operator(0.12, csw, -1, 12)
+        A = orc.clover_fields(gref, L, 0.12, csw, recon=12)[0] if csw else None
+        bs = [orc.source_gauss(L, 60 + k) for k in range(3)]
+        bs[1] = np.zeros_like(bs[1])
+        bs[1][0, 0, 1, 2] = 1.0
+        sp = q.default_solve_params(tol=1e-9, precision=prec, chunk=3, delta=0.3, max_iter=400)
+        xs, sts = q.solve_batch(g, op, bs, sp)
+        for b, x, st in zip(bs, xs, sts):
+            r = b - orc.full_op(x, gref, L, 0.12, A=A, s=1, tbc=-1.0, recon=12)
+            res = np.linalg.norm(r) / np.linalg.norm(b)
+            assert st.converged and res <= 1e-9 + 1e-14
+            assert abs(res - st.true_residual) <= 1e-14
+            assert st.reliable_updates >= 1
