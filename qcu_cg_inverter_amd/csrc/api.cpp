@@ -265,17 +265,18 @@ static int eighth_of_t(const Geom& geo) {
 // shape was tuned or pinned for it: while the launch's links and spinors come from the
 // Infinity Cache, the split's four waves per chunk keep more of that latency in flight;
 // past it the two kernels wait for the same HBM bytes, and the LDS kernel's one read of
-// the links per batch wins.  Per launch, hop_kernel / hop_lds_kernel against this one
-// (us): 8^4 FP64 9.2 / 5.1, FP32 6.9 / 4.2, 12-RHS FP32 14.2 / 6.0; 16^3x32 FP64 recon-18
-// 20.2 / 17.3, FP32 10.9 / 7.4, FP16 9.4 / 6.4, 12-RHS FP32 55.5 / 45.5; 24^3x48 FP32
-// 43.6 / 29.2 (190 MB); above the line: FP32 4 RHS (382 MB) 111 / 118, 32^3x64 (600 MB)
-// 113 / 127, FP64 recon-18 on 24^4 4 RHS (445 MB) 133 / 140.  FP64 recon-12 gains up to
-// 509 MB (24^3x48 95 / 75, 2 RHS 142 / 127) and is even at 1.2 GB.  FP16 spends its time
-// on unpacking and rebuilding the links, which the LDS kernel does once per batch: 24^3x48
-// 27 / 18.5, 4 RHS 63 / 59, but 16^3x32 12 RHS 31.6 / 36.
+// the links per batch wins.  Per launch, hop_kernel against this one (us): 8^4 FP64 9.2 /
+// 5.1, FP32 6.9 / 4.2; 16^3x32 FP64 recon-18 20.2 / 17.3, FP32 10.9 / 7.4, FP16 9.4 / 6.4;
+// 24^3x48 FP32 43.6 / 29.2 (190 MB), FP16 27 / 18.5; above the line 32^3x64 FP32 (600 MB)
+// 113 / 127; FP64 recon-12 gains up to 509 MB (24^3x48 95 / 75) and is even at 1.2 GB.
+// hop_lds_kernel against this one: 24^3x48 FP32 2 RHS (243 MB) 64 / 43, 3 RHS (303 MB) 74 /
+// 90; 16^2x32x64 FP32 240 MB 66 / 46, recon-18 288 MB 70 / 82; 12^2x16x64 FP64 216 MB 59 /
+// 52, 297 MB 83 / 107.  FP16 spends its time on unpacking and rebuilding the links, which
+// the LDS kernel does once per batch: 24^3x48 4 RHS 61 / 62, 16^3x32 6 RHS 21 / 20, 12 RHS
+// 33 / 36.
 static bool split_pays(int prec, int recon, long vh, int nrhs) {
   const size_t bytes = gauge_bytes(prec, recon, vh) + 2 * (size_t)nrhs * spinor_bytes(prec, vh);
-  if (bytes > ((size_t)(prec == F64 && recon == 12 ? 550 : 320) << 20)) return false;
+  if (bytes > ((size_t)(nrhs > 1 ? 256 : prec == F64 && recon == 12 ? 550 : 320) << 20)) return false;
   return prec != F16 || nrhs <= 4 || (vh + 63) / 64 * nrhs <= 6144;
 }
 // t-slices its chunks are taken at a time (ChunkOrder): an eighth of Lt, one tile per XCD
@@ -297,13 +298,21 @@ Tune tuned_hop(int prec, int recon, long vh, int nrhs, int epi) {
   t.split = split_pays(prec, recon, vh, nrhs);
   if (nrhs > 1) {  // every right-hand side in one block per 64-site chunk, its links
     // staged in LDS once (hop_lds_kernel; on 32^3x64 with 12 right-hand sides 22-29 %
-    // faster than the best shape sharing link loads within a wave), 4 waves per block,
-    // blocks round-robin over the XCDs
+    // faster than the best shape sharing link loads within a wave), blocks round-robin over
+    // the XCDs.  Four waves per block, of which FP32 and FP64 gain with two right-hand sides
+    // already (32^3x64 2 RHS, two waves / four: FP32 184 / 175 us, FP64 421 / 376); FP16 two
+    // while the links weigh more than the right-hand sides (2 RHS 104 / 128, 6 249 / 269, 12
+    // 474 / 472, 24^3x48 6 RHS 80 / 85).
     t.lds = 2;  // a clover shared by every right-hand side staged in LDS as well
-    t.block = nrhs >= 4 ? 256 : 128;
+    t.block = prec == F16 && nrhs <= 6 ? 128 : 256;
+    // and then eight waves where four leave a CU short of them: beside the clover an LDS
+    // holds one block in FP64 and two in FP32.  32^3x64 four waves / eight: FP64 A^-1 D 5 RHS
+    // 1,089 / 891 us, 12 1,762 / 1,687, its M^ 12 2,183 / 2,009; FP32 A^-1 D 12 RHS 856 / 815,
+    // M^ 1,024 / 1,003, but with one right-hand side a wave 602 / 649 (8 RHS)
+    t.clw = (prec == F64 && nrhs >= 5) || (prec == F32 && nrhs > 8) ? 8 : 0;
     t.xcd = 0;
-    t.tz = -1;  // tiles of all of z by 8 t-planes (ignored where they do not fit)
-    t.tt = 8;
+    t.tz = -1;  // tiles of all of z by 8 t-planes, or launch_shape's chunk order where they
+    t.tt = 8;   // do not fit
   }
   return t;
 }
@@ -329,6 +338,15 @@ void launch_shape(int prec, int recon, int epi, HopArgs& a, const Tune& t, hipSt
   a.cached = t.cached;
   a.lds = t.lds;
   a.walk = make_walk(a.geo, t.ty, t.tz < 0 ? a.geo.L[2] : t.tz, t.tt);
+  a.order = make_chunk_order(a.geo, 1);
+  a.clw = t.clw;
+  // planes that are no whole chunks: t-slices in eighths of Lt, one per XCD, instead of
+  // storage order round-robin.  24^3x48 12 RHS FP32 327 -> 270 us, FP64 708 -> 560, FP16 166
+  // -> 147, 20^2x24x40 FP32 193 -> 151, FP64 399 -> 324, 24x20x32x48 3 RHS FP32 93 -> 77
+  if (t.lds && (t.tz < 0 || t.order) && !a.walk.tile_z) {
+    a.order = make_chunk_order(a.geo, eighth_of_t(a.geo));
+    a.xcd_remap = 1;
+  }
   launch_hop(prec, recon, epi, a, t.block, t.rb, t.rpt, st);
 }
 

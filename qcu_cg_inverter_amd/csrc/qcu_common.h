@@ -122,60 +122,6 @@ enum Epi : int {
 
 constexpr int kMaxRhs = 16;
 
-// One hopping-kernel launch.  Fields of a batch of right-hand sides are strided in
-// memory (rhs r at base + r * stride bytes); clover / coefficient may differ per rhs.
-struct HopArgs {
-  const void* in;
-  void* out;
-  const void* x;
-  const void* gauge;
-  long in_stride, out_stride, x_stride;  // bytes between right-hand sides
-  const void* clov[kMaxRhs];             // packed clover of parity p per rhs (may repeat)
-  double coef[kMaxRhs];
-  double* partials;                      // |out|^2 per block per rhs, or null
-  Geom geo;
-  int parity;
-  int dagger;                            // 0: s = +1, 1: s = -1
-  double tbc;                            // t boundary sign
-  int nrhs;
-  int xcd_remap;                         // contiguous site ranges per XCD
-  int sg;                                // sites per right-hand side group (set by the launcher)
-  int ngroups;                           // blocks per site range (set by the launcher)
-  int gmajor;                            // 1: right-hand side group is the slowest block index
-  int rpw;                               // right-hand sides per wave (1, 2 or 4)
-  int spt;                               // site blocks walked by each block (sites per thread)
-  int cached;                            // 1: ordinary loads of links / clover / x, 0: streaming
-  long nsb;                              // site blocks of the lattice (set by the launcher)
-  int clov_shared;                       // every right-hand side uses clov[0]
-  int nt_store;                          // nontemporal stores of out and loads of x (set by the launcher)
-  Walk walk;                             // site traversal order
-  int lds;                               // 1: hop_lds_kernel (every right-hand side per block, links in LDS),
-                                         // 2: and a shared clover in LDS
-  int cgw, cgq, cgr;                     // XCD column groups (xcd_remap >= 2, set by the launcher): W chunks
-  long cgnp;                             // per XCD of each Q-chunk sub-plane, R ranges of the NP sub-planes
-};
-
-// walk with (tile_z, tile_t) tiles, or storage order when the tiles do not divide the
-// lattice or a plane is not a multiple of 64 sites
-inline Walk make_walk(const Geom& g, int ty, int tz, int tt) {
-  Walk w;
-  w.tile_y = w.tile_z = w.tile_t = w.ny = w.ntz = 0;
-  if (ty <= 0) ty = g.L[1];
-  const long sub = (long)g.lxh * ty;
-  if (tz <= 0 || tt <= 0 || g.L[1] % ty != 0 || sub % 64 != 0 || g.L[2] % tz != 0 || g.L[3] % tt != 0) return w;
-  w.tile_y = ty;
-  w.tile_z = tz;
-  w.tile_t = tt;
-  w.ny = g.L[1] / ty;
-  w.ntz = g.L[2] / tz;
-  w.dsp = FastDiv((uint32_t)sub);
-  w.dtt = FastDiv((uint32_t)tt);
-  w.dtz = FastDiv((uint32_t)tz);
-  w.dny = FastDiv((uint32_t)w.ny);
-  w.dntz = FastDiv((uint32_t)w.ntz);
-  return w;
-}
-
 // Order in which a launch takes the 64-site storage chunks of a half lattice.  tt = 0:
 // storage order.  Otherwise the t-slices are taken tt at a time, t fastest: a chunk's t
 // neighbours are then one step away and its z neighbours tt planes, instead of a whole
@@ -204,6 +150,62 @@ inline ChunkOrder make_chunk_order(const Geom& g, int tt) {
     o.dslice = FastDiv(o.slice);
   }
   return o;
+}
+
+// One hopping-kernel launch.  Fields of a batch of right-hand sides are strided in
+// memory (rhs r at base + r * stride bytes); clover / coefficient may differ per rhs.
+struct HopArgs {
+  const void* in;
+  void* out;
+  const void* x;
+  const void* gauge;
+  long in_stride, out_stride, x_stride;  // bytes between right-hand sides
+  const void* clov[kMaxRhs];             // packed clover of parity p per rhs (may repeat)
+  double coef[kMaxRhs];
+  double* partials;                      // |out|^2 per block per rhs, or null
+  Geom geo;
+  int parity;
+  int dagger;                            // 0: s = +1, 1: s = -1
+  double tbc;                            // t boundary sign
+  int nrhs;
+  int xcd_remap;                         // contiguous site ranges per XCD
+  int sg;                                // sites per right-hand side group (set by the launcher)
+  int ngroups;                           // blocks per site range (set by the launcher)
+  int gmajor;                            // 1: right-hand side group is the slowest block index
+  int rpw;                               // right-hand sides per wave (1, 2 or 4)
+  int spt;                               // site blocks walked by each block (sites per thread)
+  int cached;                            // 1: ordinary loads of links / clover / x, 0: streaming
+  long nsb;                              // site blocks of the lattice (set by the launcher)
+  int clov_shared;                       // every right-hand side uses clov[0]
+  int nt_store;                          // nontemporal stores of out and loads of x (set by the launcher)
+  Walk walk;                             // site traversal order
+  ChunkOrder order;                      // hop_lds_kernel's order of chunks where the walk has no tiles
+  int lds;                               // 1: hop_lds_kernel (every right-hand side per block, links in LDS),
+                                         // 2: and a shared clover in LDS
+  int clw;                               // waves of a block with the clover in LDS, or 0: as without
+  int cgw, cgq, cgr;                     // XCD column groups (xcd_remap >= 2, set by the launcher): W chunks
+  long cgnp;                             // per XCD of each Q-chunk sub-plane, R ranges of the NP sub-planes
+};
+
+// walk with (tile_z, tile_t) tiles, or storage order when the tiles do not divide the
+// lattice or a plane is not a multiple of 64 sites
+inline Walk make_walk(const Geom& g, int ty, int tz, int tt) {
+  Walk w;
+  w.tile_y = w.tile_z = w.tile_t = w.ny = w.ntz = 0;
+  if (ty <= 0) ty = g.L[1];
+  const long sub = (long)g.lxh * ty;
+  if (tz <= 0 || tt <= 0 || g.L[1] % ty != 0 || sub % 64 != 0 || g.L[2] % tz != 0 || g.L[3] % tt != 0) return w;
+  w.tile_y = ty;
+  w.tile_z = tz;
+  w.tile_t = tt;
+  w.ny = g.L[1] / ty;
+  w.ntz = g.L[2] / tz;
+  w.dsp = FastDiv((uint32_t)sub);
+  w.dtt = FastDiv((uint32_t)tt);
+  w.dtz = FastDiv((uint32_t)tz);
+  w.dny = FastDiv((uint32_t)w.ny);
+  w.dntz = FastDiv((uint32_t)w.ntz);
+  return w;
 }
 
 // One launch of the leg-split kernel on internal fields (k_hop_split.inc); h's launch

@@ -130,6 +130,8 @@ struct Tune {
   int cached = 0;
   int lds = 0;  // 1: every right-hand side in one block per 64-site chunk, its links staged in LDS;
                 // 2: a clover shared by every right-hand side staged too
+  int clw = 0;  // waves of a block that stages the clover (8), or 0: as many as without
+  int order = 0;  // 1: the LDS kernel on untiled planes takes its chunks in eighths of Lt (launch_shape)
   int split = 0;  // 1: the leg-split kernel; the rest does not apply
 };
 

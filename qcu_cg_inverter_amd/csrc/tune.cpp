@@ -67,11 +67,11 @@ void load_tune_cache() {
   fclose(f);
 }
 
-// the leg-split kernel has no shape to write: where it won, later processes take it by
-// the default rule
+// the leg-split kernel and the LDS kernel's chunk order have no shape to write: where they
+// won, later processes take them by the default rule
 static void append_cache(const std::string& key, const Tune& t, double ms) {
   const char* path = cache_file();
-  if (!path || t.split) return;
+  if (!path || t.split || t.order) return;
   FILE* f = fopen(path, "a");
   if (!f) return;
   fprintf(f, "%s %d %d %d %d %d %d %d %d %d %d %d %d %.6f\n", key.c_str(), t.block, t.rb, t.rpt, t.xcd, t.tz, t.tt,
@@ -223,6 +223,15 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
     timed.push_back({time_shape(split, EPI_PLAIN), split});
     std::stable_sort(timed.begin(), timed.end(), by_time);
   }
+  if (nrhs > 1 && !make_walk(g.geo, 0, g.geo.L[2], 8).tile_z)  // the default's chunk order, likewise
+    for (const auto& c : timed)
+      if (c.second.lds && !c.second.split && c.second.tz == 0 && c.second.spt == 1) {
+        Tune t = c.second;
+        t.order = 1;
+        timed.push_back({time_shape(t, EPI_PLAIN), t});
+        std::stable_sort(timed.begin(), timed.end(), by_time);
+        break;
+      }
   const Tune best = timed.front().second;
   const double bms = timed.front().first;
   std::string key = tune_key(prec, recon, vh, nrhs, EPI_PLAIN);
@@ -236,7 +245,7 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
   auto same = [](const Tune& x, const Tune& y) {
     return x.block == y.block && x.rb == y.rb && x.rpt == y.rpt && x.xcd == y.xcd && x.tz == y.tz &&
            x.tt == y.tt && x.gm == y.gm && x.ty == y.ty && x.rpw == y.rpw && x.spt == y.spt && x.cached == y.cached &&
-           x.lds == y.lds && x.split == y.split;
+           x.lds == y.lds && x.split == y.split && x.order == y.order;
   };
   auto add_shape = [&](const Tune& t) {
     for (const Tune& u : epi_shapes)

@@ -235,3 +235,21 @@ def test_solve_residual_by_oracle(q, L, prec):
             assert st.converged and res <= 1e-9 + 1e-14
             assert abs(res - st.true_residual) <= 1e-14
             assert st.reliable_updates >= 1
+
+
+@pytest.mark.parametrize("prec,nrhs", [(0, 5), (2, 7)])
+def test_lds_hop_chunk_order_bits(q, prec, nrhs):
+    """Past the Infinity Cache a batch takes the LDS kernel, which orders the chunks of a
+    lattice whose planes are no whole chunks (20^2 / 2 = 200 sites) by eighths of Lt, with
+    eight waves a block in FP64 clover: the bits of right-hand sides solved alone."""
+    L = (20, 20, 24, 24)
+    g = q.Gauge.random(L, seed=46, eps=0.2)
+    op = q.Operator(0.12, 1.0, -1, 12)
+    sp = q.default_solve_params(tol=1e-12, precision=prec, chunk=4, max_iter=8)
+    bs = [orc.source_gauss(L, 80 + k) for k in range(2)]
+    bs += [bs[k % 2] * (1.0 + k) for k in range(2, nrhs)]
+    xs, sts = q.solve_batch(g, op, bs, sp, raise_on_error=False)
+    for k in (0, 1, nrhs - 1):
+        x, st = q.solve(g, op, bs[k], sp, raise_on_error=False)
+        assert np.array_equal(x, xs[k]) and st.iterations == sts[k].iterations
+        assert st.true_residual == sts[k].true_residual
