@@ -165,61 +165,76 @@ void GaugeField::forget_links() {
   clovers.clear();
 }
 
+// Fields are put together in buffers of their own and handed over once the launches that
+// fill them are queued, so that a buffer a gauge or a clover field holds is always a built
+// one: a step that throws (an allocation above all) leaves everything as it was.
 const void* GaugeField::get(int prec, int recon) {
   DevBuf& b = packed[prec][recon == 12 ? 1 : 0];
   if (!b.p) {
     if (!aos.p && (prec == F64 || recon != 12)) throw Error(QCU_ERROR_STATE, "internal: drop-in links are recon-12");
-    take(b, gauge_bytes(prec, recon, geo.vh));
-    if (aos.p) launch_gauge_pack(prec, recon, aos.p, b.p, geo.vh, stream());
-    else launch_gauge_repack(prec, packed[F64][1].p, b.p, geo.vh, stream());
+    DevBuf d;
+    take(d, gauge_bytes(prec, recon, geo.vh));
+    if (aos.p) launch_gauge_pack(prec, recon, aos.p, d.p, geo.vh, stream());
+    else launch_gauge_repack(prec, packed[F64][1].p, d.p, geo.vh, stream());
     QHIP(hipGetLastError());
+    b.swap(d);
   }
   return b.p;
 }
 
 CloverField* GaugeField::clover(double ck, int prec, CloverParts parts) {
-  auto it = clovers.find(ck);
-  CloverField* cf;
-  if (it == clovers.end()) {
-    std::unique_ptr<CloverField> c(new CloverField);
-    c->ck = ck;
-    c->vh = geo.vh;
-    cf = c.get();
-    clovers[ck] = std::move(c);
-  } else {
-    cf = it->second.get();
+  std::unique_ptr<CloverField>& slot = clovers[ck];
+  if (!slot) {
+    slot.reset(new CloverField);
+    slot->ck = ck;
+    slot->vh = geo.vh;
   }
-  const size_t half64 = clover_bytes(F64, geo.vh) / 2;
-  CloverBuild b;
-  bool need[2];
+  CloverField* cf = slot.get();
+  bool need_a[2], need_inv[2];
   for (int p = 0; p < 2; ++p) {
     const bool inv = parts == CLOVER_ALL || (parts == CLOVER_SOLVE && p == 1);
-    b.A[p] = cf->A[F64][p].p ? nullptr : take(cf->A[F64][p], half64);
-    b.Ainv[p] = !inv || cf->Ainv[F64][p].p ? nullptr : take(cf->Ainv[F64][p], half64);
-    need[p] = b.A[p] || b.Ainv[p];
-    if (b.Ainv[p] && !cf->bad.p) {
-      cf->bad.alloc(sizeof(int));
-      QHIP(hipMemsetAsync(cf->bad.p, 0, sizeof(int), stream()));
-    }
+    need_a[p] = !cf->A[F64][p].p;
+    need_inv[p] = inv && !cf->Ainv[F64][p].p;
   }
+  const bool need[2] = {need_a[0] || need_inv[0], need_a[1] || need_inv[1]};
   if (need[0] || need[1]) {
+    const size_t half = clover_bytes(F64, geo.vh) / 2;
     const int recon = aos.p ? 18 : 12;
+    CloverBuild b;
+    DevBuf A[2], Ainv[2], bad;
     b.gauge = get(F64, recon);
-    b.nbad = static_cast<int*>(cf->bad.p);
+    for (int p = 0; p < 2; ++p) {
+      b.A[p] = need_a[p] ? take(A[p], half) : nullptr;
+      b.Ainv[p] = need_inv[p] ? take(Ainv[p], half) : nullptr;
+    }
+    const bool first_inv = (need_inv[0] || need_inv[1]) && !cf->bad.p;
+    if (first_inv) {
+      bad.alloc(sizeof(int));
+      QHIP(hipMemsetAsync(bad.p, 0, sizeof(int), stream()));
+    }
+    b.nbad = static_cast<int*>(first_inv ? bad.p : cf->bad.p);
     b.ck = ck;
     b.only = need[0] && need[1] ? -1 : need[1];
     b.geo = geo;
     launch_clover_build(recon, b, stream());
     QHIP(hipGetLastError());
+    for (int p = 0; p < 2; ++p) {
+      if (need_a[p]) cf->A[F64][p].swap(A[p]);
+      if (need_inv[p]) cf->Ainv[F64][p].swap(Ainv[p]);
+    }
+    if (first_inv) cf->bad.swap(bad);
   }
   // inner-precision parts: A_ee and A^-1_oo
   if (parts != CLOVER_A && prec != F64 && !cf->A[prec][0].p) {
     const size_t half = clover_bytes(prec, geo.vh) / 2;
-    take(cf->A[prec][0], half);
-    take(cf->Ainv[prec][1], half);
-    launch_clover_convert(prec, cf->a(F64, 0), cf->A[prec][0].p, geo.vh, stream());
-    launch_clover_convert(prec, cf->ainv(F64, 1), cf->Ainv[prec][1].p, geo.vh, stream());
+    DevBuf A, Ainv;
+    take(A, half);
+    take(Ainv, half);
+    launch_clover_convert(prec, cf->a(F64, 0), A.p, geo.vh, stream());
+    launch_clover_convert(prec, cf->ainv(F64, 1), Ainv.p, geo.vh, stream());
     QHIP(hipGetLastError());
+    cf->A[prec][0].swap(A);
+    cf->Ainv[prec][1].swap(Ainv);
   }
   return cf;
 }

@@ -1,0 +1,80 @@
+"""libqcu.so's host side on a stand-in for the HIP runtime (tests/host/host_hip.cpp): what
+a call leaves behind when an allocation fails, and the bookkeeping of resident fields.
+Kernels do not run here; the stand-in logs their launches and finds one that reads links
+or clover blocks that no earlier launch wrote.  Each scenario is a process of its own."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+PRELUDE = """
+import ctypes, sys
+H = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)   # before libqcu.so: its symbols win
+H.host_hip_wrong.restype = ctypes.c_char_p
+H.host_hip_live.restype = ctypes.c_size_t
+H.host_hip_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
+import numpy as np
+import qcu_cg_inverter_amd as q
+ref = ctypes.byref
+q.init(0)
+L = (4, 4, 4, 4)
+VH = q.half_volume(L)
+def spinor(): return q.DeviceBuffer(2 * VH * 192)
+"""
+
+
+@pytest.fixture(scope="session")
+def host_hip(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "host_hip.so")
+    src = os.path.join(ROOT, "tests", "host", "host_hip.cpp")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(ROCM, "include"), src, "-o", so], check=True)
+    return so
+
+
+def run(host_hip, script, *args, **env):
+    e = dict(os.environ, PYTHONPATH=ROOT, QCU_EXIT_ON_ERROR="0", **env)
+    p = subprocess.run([sys.executable, "-c", PRELUDE + script, host_hip, *map(str, args)],
+                       capture_output=True, text=True, env=e, cwd=ROOT, timeout=300)
+    assert p.returncode == 0, p.stdout + p.stderr
+    return p.stdout
+
+
+CALLS = """
+op = q.Operator(0.12, 1.0, -1, 12)
+a, b = spinor(), spinor()
+def call(g, name):
+    l = q.lib()
+    if name == "apply_m": return l.qcuApplyM(g.handle, ref(op), b.ptr, a.ptr, 0)
+    if name == "ainv": return l.qcuApplyComposite(g.handle, ref(op), q.COMP_AINV, b.ptr, a.ptr, 0)
+    if name == "export": return l.qcuCloverExport(g.handle, ref(op), A.ptr, Ai.ptr, None)
+    if name.startswith("mhat"): return l.qcuApplyMhat(g.handle, ref(op), b.ptr, a.ptr, 0, int(name[-1]))
+    return l.qcuSolve(g.handle, ref(op), ref(q.default_solve_params(precision=int(name[-1]))), b.ptr, a.ptr, None)
+A, Ai = q.DeviceBuffer(2 * VH * 72 * 16), q.DeviceBuffer(2 * VH * 72 * 16)
+"""
+
+
+@pytest.mark.parametrize("name", ["apply_m", "ainv", "export", "mhat0", "mhat1", "mhat2", "solve0", "solve1", "solve2"])
+def test_retry_after_failed_allocation(host_hip, name):
+    """Whichever allocation of a call fails, the call says so, and the same call made again
+    reads no links and no clover block that was not built."""
+    run(host_hip, CALLS + textwrap.dedent("""
+    name = sys.argv[2]
+    for k in range(100):
+        g = q.Gauge.random(L, seed=1, eps=0.2)
+        H.host_hip_fail_after(k)
+        rc = call(g, name)
+        H.host_hip_fail_after(-1)
+        if rc == 0: break
+        assert rc == 3, (k, rc)
+        rcs = [call(g, name) for _ in range(3)]
+        assert rcs[-1] == 0, (k, rcs, q.lib().qcuGetLastErrorString())
+        assert H.host_hip_wrong() == b"", (k, H.host_hip_wrong())
+        g.destroy()
+    assert 2 < k < 99, k
+    """), name)
