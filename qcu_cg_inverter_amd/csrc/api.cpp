@@ -17,6 +17,7 @@ static std::string g_last_msg;
 
 void check_hip(hipError_t e, const char* what, const char* file, int line) {
   if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here: left in place, it would fail the next call's launch check
   char buf[512];
   snprintf(buf, sizeof buf, "HIP error %d (%s) from %s at %s:%d", (int)e, hipGetErrorString(e), what, file, line);
   throw Error(e == hipErrorOutOfMemory ? QCU_ERROR_OUT_OF_MEMORY : QCU_ERROR_HIP, buf);

@@ -78,3 +78,14 @@ def test_retry_after_failed_allocation(host_hip, name):
         g.destroy()
     assert 2 < k < 99, k
     """), name)
+
+
+def test_error_of_one_call_is_not_the_next_ones(host_hip):
+    """A call that runs out of memory leaves no error behind for the calls after it."""
+    run(host_hip, textwrap.dedent("""
+    g = q.Gauge.random(L, seed=1, eps=0.2)
+    a, b = spinor(), spinor()
+    p = ctypes.c_void_p()
+    assert q.lib().qcuMalloc(ref(p), 1 << 50) == 3
+    assert q.lib().qcuHop(g.handle, b.ptr, a.ptr, 0, 0, 1, 12, 0) == 0, q.lib().qcuGetLastErrorString()
+    """))
