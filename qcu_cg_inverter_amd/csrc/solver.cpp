@@ -80,9 +80,12 @@ static void full_op_parity(OpView& o, int p, int dag, Vec in_p, Vec in_q, Vec ou
 
 // A batch object kept between calls, so repeated solves of the same shape reuse its device
 // buffers, also for another gauge of the same lattice (a 16^3x32 batch is seven
-// allocations, about 1 ms to free and make again).  Dropped with the gauge it last served.
+// allocations, about 1 ms to free and make again).  Dropped with the gauge it last served,
+// also when that gauge's fields have changed since (bound = false: the next solve takes
+// them up again).
 struct CachedBatch {
   GaugeField* g = nullptr;
+  bool bound = false;
   int L[4] = {0, 0, 0, 0};
   int prec = -1, recon = 0, tbc = 0, clover = -1, cap = 0, chunk = 0, graph = -1;
   double delta = 0.0;
@@ -94,11 +97,12 @@ void drop_cached_batches(GaugeField* g) {
   if (!g || g_cached.g == g) {
     g_cached.batch.reset();
     g_cached.g = nullptr;
+    g_cached.bound = false;
   }
 }
 
 void unbind_cached_batches(GaugeField* g) {
-  if (g_cached.g == g) g_cached.g = nullptr;
+  if (g_cached.g == g) g_cached.bound = false;
 }
 
 static CgBatch& batch_for(GaugeField& g, int prec, const qcuOperator& op, int nrhs, const qcuSolveParams& sp) {
@@ -118,11 +122,12 @@ static CgBatch& batch_for(GaugeField& g, int prec, const qcuOperator& op, int nr
     c.chunk = sp.chunk;
     c.graph = sp.graph;
     c.delta = sp.delta;
-  } else if (c.g != &g) {
-    c.g = nullptr;  // a rebind that throws is tried again by the next solve
+  } else if (c.g != &g || !c.bound) {
+    c.bound = false;  // a rebind that throws is tried again by the next solve
     c.batch->rebind(g);
   }
   c.g = &g;
+  c.bound = true;
   return *c.batch;
 }
 

@@ -89,3 +89,38 @@ def test_error_of_one_call_is_not_the_next_ones(host_hip):
     assert q.lib().qcuMalloc(ref(p), 1 << 50) == 3
     assert q.lib().qcuHop(g.handle, b.ptr, a.ptr, 0, 0, 1, 12, 0) == 0, q.lib().qcuGetLastErrorString()
     """))
+
+
+DROPIN = """
+prm = q.param(L)
+def dropin(name, *args):
+    q.lib().qcuClearLastError()
+    getattr(q.lib(), name)(*args)
+    return q.lib().qcuGetLastError()
+def new_links(seed):
+    u = np.random.default_rng(seed).standard_normal((4, 2, VH, 3, 3, 2))
+    gd.upload(u)
+gd = q.DeviceBuffer(4 * 2 * VH * 9 * 16)
+a, b = spinor(), spinor()
+"""
+
+
+def test_solver_workspace_goes_with_its_dropin_gauge(host_hip):
+    """A drop-in gauge that changed after a solve and is then replaced by one of another
+    lattice takes the solve's workspace with it."""
+    run(host_hip, DROPIN + textwrap.dedent("""
+    big = q.param((4, 4, 4, 8))
+    gbig, abig, bbig = (q.DeviceBuffer(2 * n) for n in (gd.nbytes, a.nbytes, b.nbytes))
+    def apply_big(): assert dropin("fullDslashQcu", bbig.ptr, abig.ptr, gbig.ptr, ref(big), 0) == 0
+    def apply(): assert dropin("fullDslashQcu", b.ptr, a.ptr, gd.ptr, ref(prm), 0) == 0
+    new_links(1)
+    apply()
+    apply_big()
+    live = H.host_hip_live()
+    apply()
+    assert dropin("cg_inverter", a.ptr, b.ptr, gd.ptr, ref(prm)) == 0
+    new_links(2)
+    apply()
+    apply_big()
+    assert H.host_hip_live() == live
+    """))
