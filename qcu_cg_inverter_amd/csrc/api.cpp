@@ -72,10 +72,30 @@ void DevBuf::release() {
   p = nullptr;
   n = 0;
 }
+// hipMalloc; when the card is full, what is only kept to save a later allocation (a changed
+// drop-in gauge's old fields and solver workspace) is given back first
+static void* device_malloc(size_t bytes) {
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    bool freed = drop_unbound_batch();
+    GaugeField* g = ctx().dropin.g.get();
+    if (g && !g->spare.empty()) {
+      g->spare.clear();
+      freed = true;
+    }
+    if (freed) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, bytes);
+    }
+  }
+  check_hip(e, "hipMalloc", __FILE__, __LINE__);
+  return p;
+}
 void* DevBuf::alloc(size_t bytes) {
   release();
   if (bytes == 0) return nullptr;
-  QHIP(hipMalloc(&p, bytes));
+  p = device_malloc(bytes);
   n = bytes;
   return p;
 }
@@ -140,12 +160,6 @@ void* GaugeField::take(DevBuf& b, size_t bytes) {
       spare.erase(it);
       return b.p;
     }
-  try {
-    return b.alloc(bytes);
-  } catch (const Error& e) {
-    if (e.code != QCU_ERROR_OUT_OF_MEMORY || spare.empty()) throw;
-  }
-  spare.clear();
   return b.alloc(bytes);
 }
 
@@ -755,7 +769,8 @@ int qcuMalloc(void** ptr, size_t bytes) {
   return guarded([&] {
     ensure_init();
     QREQ(ptr, "qcuMalloc: NULL");
-    QHIP(hipMalloc(ptr, bytes));
+    *ptr = nullptr;
+    *ptr = device_malloc(bytes);
   });
 }
 int qcuFree(void* ptr) {

@@ -96,7 +96,7 @@ struct GaugeField {
   // Allocations of the fields dropped by forget_links, for the next ones of their size: a
   // drop-in gauge that changes remakes the same fields, and freeing and allocating one of
   // 76 MB takes 265 us, several times what its kernel takes.  At most what this gauge
-  // held before; freed with it.
+  // held before; freed with it, or when another allocation fails.
   std::list<DevBuf> spare;
   void* take(DevBuf& b, size_t bytes);  // b (empty) gets a spare of that size, or a new allocation
   // drop every packed and clover field, keeping the allocations; the context stream is idle
@@ -208,6 +208,8 @@ void apply_mhat_iface(GaugeField& g, const qcuOperator& op, void* out, const voi
 void drop_cached_batches(GaugeField* g);
 // the fields of g changed: the next solve takes them up again, in the same workspace
 void unbind_cached_batches(GaugeField* g);
+// free a workspace that waits for its gauge's new fields; true if there was one
+bool drop_unbound_batch();
 void apply_m_iface(GaugeField& g, const qcuOperator& op, void* out, const void* in, int dagger);
 void apply_composite_iface(GaugeField& g, const qcuOperator& op, int kind, void* out, const void* in, int dagger);
 

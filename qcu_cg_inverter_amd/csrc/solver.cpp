@@ -105,6 +105,12 @@ void unbind_cached_batches(GaugeField* g) {
   if (g_cached.g == g) g_cached.bound = false;
 }
 
+bool drop_unbound_batch() {
+  if (!g_cached.batch || g_cached.bound) return false;
+  drop_cached_batches(nullptr);
+  return true;
+}
+
 static CgBatch& batch_for(GaugeField& g, int prec, const qcuOperator& op, int nrhs, const qcuSolveParams& sp) {
   CachedBatch& c = g_cached;
   const int clov = op.csw != 0.0;
@@ -123,8 +129,13 @@ static CgBatch& batch_for(GaugeField& g, int prec, const qcuOperator& op, int nr
     c.graph = sp.graph;
     c.delta = sp.delta;
   } else if (c.g != &g || !c.bound) {
-    c.bound = false;  // a rebind that throws is tried again by the next solve
-    c.batch->rebind(g);
+    c.bound = true;  // in use: its own allocations must not give it back
+    try {
+      c.batch->rebind(g);
+    } catch (...) {
+      c.bound = false;  // tried again by the next solve
+      throw;
+    }
   }
   c.g = &g;
   c.bound = true;

@@ -99,7 +99,13 @@ void model(const std::string& k, void** a) {
 extern "C" {
 
 // ------------------------------------------------------------ for the tests ---
-void host_hip_fail_after(long n) { g_until_fail = n; }
+// the n-th allocation from now fails (-1: none); returns how many were left until the last
+// one that was asked for, -1 when it has failed
+long host_hip_fail_after(long n) {
+  const long left = g_until_fail;
+  g_until_fail = n;
+  return left;
+}
 size_t host_hip_live() { return g_live; }
 void host_hip_clear_log() {
   g_log.clear();

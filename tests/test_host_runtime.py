@@ -17,6 +17,7 @@ import ctypes, sys
 H = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)   # before libqcu.so: its symbols win
 H.host_hip_wrong.restype = ctypes.c_char_p
 H.host_hip_live.restype = ctypes.c_size_t
+H.host_hip_fail_after.argtypes, H.host_hip_fail_after.restype = [ctypes.c_long], ctypes.c_long
 H.host_hip_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
 import numpy as np
 import qcu_cg_inverter_amd as q
@@ -123,4 +124,40 @@ def test_solver_workspace_goes_with_its_dropin_gauge(host_hip):
     apply()
     apply_big()
     assert H.host_hip_live() == live
+    """))
+
+
+def test_dropin_gives_up_kept_allocations_for_a_new_one(host_hip):
+    """When an allocation fails, whichever it is, while a changed drop-in gauge keeps old
+    ones, they are freed and the call goes on, on fields of the new links."""
+    run(host_hip, DROPIN + textwrap.dedent("""
+    def solve(prec):
+        q.check(q.lib().qcuSetDefaultSolve(ref(q.default_solve_params(precision=prec))))
+        return dropin("cg_inverter", a.ptr, b.ptr, gd.ptr, ref(prm))
+    for k in range(20):
+        new_links(2 * k)
+        assert solve(1) == 0
+        new_links(2 * k + 1)          # FP32 links and clover are kept for the next of their size
+        H.host_hip_fail_after(k)
+        assert solve(2) == 0, (k, q.lib().qcuGetLastErrorString())
+        if H.host_hip_fail_after(-1) >= 0: break
+        assert H.host_hip_wrong() == b"", (k, H.host_hip_wrong())
+    assert k > 3, k
+    """))
+
+
+def test_kept_workspace_is_given_back(host_hip):
+    """The workspace of a solve on links that have changed since does not stand in the way
+    of another allocation."""
+    run(host_hip, DROPIN + textwrap.dedent("""
+    new_links(1)
+    assert dropin("cg_inverter", a.ptr, b.ptr, gd.ptr, ref(prm)) == 0
+    new_links(2)
+    assert dropin("fullDslashQcu", b.ptr, a.ptr, gd.ptr, ref(prm), 0) == 0
+    live = H.host_hip_live()
+    H.host_hip_fail_after(0)
+    extra = q.DeviceBuffer(64)
+    assert H.host_hip_fail_after(-1) == -1 and H.host_hip_live() < live
+    assert dropin("cg_inverter", a.ptr, b.ptr, gd.ptr, ref(prm)) == 0
+    assert H.host_hip_wrong() == b"", H.host_hip_wrong()
     """))
