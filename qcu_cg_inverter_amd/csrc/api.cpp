@@ -479,6 +479,12 @@ static void require_aligned(const void* p, const char* what) {
   QREQ((reinterpret_cast<uintptr_t>(p) & 15) == 0, std::string(what) + " must be 16-byte aligned (complex128)");
 }
 
+static bool overlap(const void* a, const void* b, size_t n) {
+  const char* x = static_cast<const char*>(a);
+  const char* y = static_cast<const char*>(b);
+  return x < y + n && y < x + n;
+}
+
 static uint64_t* fingerprint_parts() {
   uint64_t*& h = ctx().dropin.fp_parts;
   if (!h)
@@ -630,6 +636,12 @@ extern "C" void fullDslashQcu(void* fermion_out, void* fermion_in, void* gauge, 
     require_aligned(fermion_out, "fermion_out");
     bool deferred = false;
     GaugeField& g = dropin_gauge(gauge, param, false, &deferred);
+    if (deferred && overlap(fermion_out, fermion_in, (size_t)2 * g.geo.vh * 192)) {
+      // what overwrites its input cannot be redone: the fingerprint is looked at first
+      QHIP(hipStreamSynchronize(stream()));
+      dropin_gauge_changed(gauge, param);
+      deferred = false;
+    }
     qcuOperator op = {1.0, 1.0, 1, 12};
     apply_m_iface(g, op, fermion_out, fermion_in, dagger_flag ? 1 : 0);
     QHIP(hipStreamSynchronize(stream()));

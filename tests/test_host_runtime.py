@@ -161,3 +161,25 @@ def test_kept_workspace_is_given_back(host_hip):
     assert dropin("cg_inverter", a.ptr, b.ptr, gd.ptr, ref(prm)) == 0
     assert H.host_hip_wrong() == b"", H.host_hip_wrong()
     """))
+
+
+@pytest.mark.parametrize("shift", [0, 192])
+def test_in_place_dropin_operator_sees_new_links_first(host_hip, shift):
+    """fullDslashQcu whose output overlaps its input cannot be redone once it has written:
+    on links that changed, it imports them before anything of the operator is stored."""
+    run(host_hip, DROPIN + textwrap.dedent("""
+    shift = int(sys.argv[2])
+    buf = q.DeviceBuffer(2 * VH * 192 + shift)
+    def apply(out, x): assert dropin("fullDslashQcu", out, x, gd.ptr, ref(prm), 0) == 0
+    new_links(1)
+    apply(buf.ptr + shift, buf.ptr)
+    new_links(2)
+    H.host_hip_clear_log()
+    apply(buf.ptr + shift, buf.ptr)
+    assert H.host_hip_launches(b"gauge_pack_kernelILi0ELi12ELi1E") == 1
+    assert H.host_hip_first(b"gauge_pack_kernel") < H.host_hip_first(b"spinor_to_aos_kernel")
+    assert H.host_hip_launches(b"spinor_to_aos_kernel") == 2
+    H.host_hip_clear_log()           # unchanged links: the operator once, nothing imported
+    apply(buf.ptr + shift, buf.ptr)
+    assert H.host_hip_launches(b"gauge_pack_kernel") == 0 and H.host_hip_launches(b"spinor_to_aos_kernel") == 2
+    """), shift)
