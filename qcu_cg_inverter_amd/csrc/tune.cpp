@@ -41,6 +41,9 @@ static const char* shape_error(const Tune& t, int precision) {
     return "xcd is 0 or 1 (2 or 4: XCD column groups, LDS kernel only); group order is 0 or 1";
   if (!(t.tz >= 0 && t.tt >= 0 && t.ty >= 0 && (t.tz == 0) == (t.tt == 0)))
     return "tile extents must be non-negative, tz and tt both 0 or both positive";
+  // of the cache file only: qcuSetHopShape leaves them at 0
+  if (!((t.clw == 0 || t.clw == 8) && (t.order == 0 || t.order == 1) && (t.split == 0 || t.split == 1)))
+    return "waves beside a staged clover are 0 or 8; chunk order and leg split are 0 or 1";
   return nullptr;
 }
 
@@ -58,24 +61,29 @@ void load_tune_cache() {
     Tune t;
     double ms;
     int prec = -1;
-    // lines that do not parse, or whose shape qcuSetHopShape would refuse, are skipped
-    if (sscanf(line, "%127s %d %d %d %d %d %d %d %d %d %d %d %d %lf", key, &t.block, &t.rb, &t.rpt, &t.xcd, &t.tz,
-               &t.tt, &t.gm, &t.ty, &t.rpw, &t.spt, &t.cached, &t.lds, &ms) == 14 &&
-        sscanf(key, "hop:%d:", &prec) == 1 && prec >= 0 && prec <= 2 && !shape_error(t, prec))
+    // 15 values and the time, or the 12 of a shape that can be pinned and the time; lines
+    // that do not parse, or whose shape qcuSetHopShape would refuse, are skipped
+    bool ok = sscanf(line, "%127s %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %lf", key, &t.block, &t.rb, &t.rpt,
+                     &t.xcd, &t.tz, &t.tt, &t.gm, &t.ty, &t.rpw, &t.spt, &t.cached, &t.lds, &t.clw, &t.order, &t.split,
+                     &ms) == 17;
+    if (!ok) {
+      t.clw = t.order = t.split = 0;
+      ok = sscanf(line, "%127s %d %d %d %d %d %d %d %d %d %d %d %d %lf", key, &t.block, &t.rb, &t.rpt, &t.xcd, &t.tz,
+                  &t.tt, &t.gm, &t.ty, &t.rpw, &t.spt, &t.cached, &t.lds, &ms) == 14;
+    }
+    if (ok && sscanf(key, "hop:%d:", &prec) == 1 && prec >= 0 && prec <= 2 && !shape_error(t, prec))
       ctx().tune[key] = t;
   }
   fclose(f);
 }
 
-// the leg-split kernel and the LDS kernel's chunk order have no shape to write: where they
-// won, later processes take them by the default rule
 static void append_cache(const std::string& key, const Tune& t, double ms) {
   const char* path = cache_file();
-  if (!path || t.split || t.order) return;
+  if (!path) return;
   FILE* f = fopen(path, "a");
   if (!f) return;
-  fprintf(f, "%s %d %d %d %d %d %d %d %d %d %d %d %d %.6f\n", key.c_str(), t.block, t.rb, t.rpt, t.xcd, t.tz, t.tt,
-          t.gm, t.ty, t.rpw, t.spt, t.cached, t.lds, ms);
+  fprintf(f, "%s %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %.6f\n", key.c_str(), t.block, t.rb, t.rpt, t.xcd, t.tz,
+          t.tt, t.gm, t.ty, t.rpw, t.spt, t.cached, t.lds, t.clw, t.order, t.split, ms);
   fclose(f);
 }
 

@@ -183,3 +183,33 @@ def test_in_place_dropin_operator_sees_new_links_first(host_hip, shift):
     apply(buf.ptr + shift, buf.ptr)
     assert H.host_hip_launches(b"gauge_pack_kernel") == 0 and H.host_hip_launches(b"spinor_to_aos_kernel") == 2
     """), shift)
+
+
+@pytest.mark.parametrize("plain", [10.0, 0.01])
+@pytest.mark.parametrize("older_line", [False, True])
+def test_tuned_kernels_outlive_the_process(host_hip, tmp_path, plain, older_line):
+    """The tuner's winners come back from QCU_TUNE_CACHE, also where the leg-split kernel
+    won (for every epilogue, or for all but the plain one), and over an older line of the
+    same key; a process with QCU_TUNE=1 does not tune them again."""
+    cache = tmp_path / "tune.cache"
+    if older_line:
+        cache.write_text("hop:1:12:128:1 64 1 1 0 0 0 0 0 1 1 1 0 0.1\n")
+    script = textwrap.dedent("""
+    phase, plain = sys.argv[2], float(sys.argv[3])
+    g = q.Gauge.random(L, seed=1, eps=0.2)
+    split = b"hop_split_kernelILi1ELi12ELi"
+    if phase == "tune":
+        H.host_hip_cost(split, 0.01)
+        H.host_hip_cost(split + b"0E", plain)    # the plain epilogue
+        q.tune_hop(g, 1, 12, 1)
+    H.host_hip_clear_log()
+    op = q.Operator(0.12, 0.0, -1, 12)
+    q.apply_mhat(g, op, np.zeros((VH, 4, 3), complex), precision=1)   # one plain hop, one x + a h
+    assert H.host_hip_launches(split + b"1E") == 1
+    assert H.host_hip_launches(split + b"0E") == (plain < 1)
+    a, b = spinor(), spinor()
+    q.check(q.lib().qcuSolve(g.handle, ref(op), ref(q.default_solve_params(precision=1)), b.ptr, a.ptr, None))
+    assert H.host_hip_launches(b"hop") < 20
+    """)
+    run(host_hip, script, "tune", plain, QCU_TUNE_CACHE=str(cache))
+    run(host_hip, script, "use", plain, QCU_TUNE_CACHE=str(cache), QCU_TUNE="1")
