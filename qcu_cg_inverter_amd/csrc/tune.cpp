@@ -169,6 +169,7 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
   // a clover-sized scratch field for the clover epilogues (its values do not matter)
   DevBuf* cl = ctx().buf("tune_clov", clover_bytes(prec, vh) / 2);
   QHIP(hipMemsetAsync(cl->p, 0, clover_bytes(prec, vh) / 2, stream()));
+  DevBuf* part = ctx().buf("tune_part", sizeof(double) * n_partials(vh) * nrhs);
   const void* gauge = g.get(prec, recon);
   HopArgs args;
   memset(&args, 0, sizeof args);
@@ -190,6 +191,8 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
   QHIP(hipEventCreate(&e1));
   const int iters = vh * nrhs > (1 << 22) ? 10 : 30;
   auto time_shape = [&](const Tune& t, int epi) -> double {
+    // as a solve launches them, the epilogues that read x also sum |out|^2
+    args.partials = epi == EPI_XPAY || epi == EPI_CLOV_XPAY ? static_cast<double*>(part->p) : nullptr;
     for (int w = 0; w < 2; ++w) launch_shape(prec, recon, epi, args, t, stream());
     QHIP(hipEventRecord(e0, stream()));
     for (int i = 0; i < iters; ++i) {

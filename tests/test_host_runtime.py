@@ -213,3 +213,17 @@ def test_tuned_kernels_outlive_the_process(host_hip, tmp_path, plain, older_line
     """)
     run(host_hip, script, "tune", plain, QCU_TUNE_CACHE=str(cache))
     run(host_hip, script, "use", plain, QCU_TUNE_CACHE=str(cache), QCU_TUNE="1")
+
+
+def test_tuner_times_reducing_hops_as_solves_launch_them(host_hip):
+    """The epilogues that read x sum |out|^2 in a solve, which takes one right-hand side per
+    wave: the tuner times them that way."""
+    run(host_hip, textwrap.dedent("""
+    g = q.Gauge.random(L, seed=1, eps=0.2)
+    H.host_hip_clear_log()
+    q.tune_hop(g, 1, 12, 4)
+    # hop_kernel<FP32, 12, epilogue, dagger 0, 1 per thread, several per wave, ...>
+    kernel = lambda epi, several: b"10hop_kernelILi1ELi12ELi%dELi0ELi1ELi%dE" % (epi, several)
+    assert H.host_hip_launches(kernel(0, 1)) > 0 and H.host_hip_launches(kernel(1, 0)) > 0
+    assert H.host_hip_launches(kernel(1, 1)) == 0 and H.host_hip_launches(kernel(3, 1)) == 0
+    """))
