@@ -35,6 +35,7 @@ def test_full_dslash_in_place_on_changed_links(q):
         A = orc.clover_fields(u, L, 1.0, 1.0, recon=12)[0]
         ref = orc.full_op(v, u, L, 1.0, A=A, s=1, tbc=1.0, recon=12)
         a = q.DeviceBuffer.from_numpy(v)
+        q.lib().qcuClearLastError()
         q.lib().fullDslashQcu(a.ptr, a.ptr, gd.ptr, ctypes.byref(prm), 0)
         assert q.lib().qcuGetLastError() == 0
         got = a.to_numpy((2, vh, 4, 3))
@@ -42,3 +43,103 @@ def test_full_dslash_in_place_on_changed_links(q):
         a.upload(v)
         q.lib().fullDslashQcu(out.ptr, a.ptr, gd.ptr, ctypes.byref(prm), 0)
         assert np.array_equal(out.to_numpy((2, vh, 4, 3)), got), step
+
+
+@pytest.mark.parametrize("prec", [0, 1, 2])
+def test_hop_shapes_keep_bits_on_internal_fields(q, prec):
+    """Every launch shape of a 12-RHS hop gives the bits of single launches from and to the
+    caller's buffers.  A batch whose outputs are its inputs goes through internal fields,
+    where the pinned shape is the one that runs."""
+    L = (16, 16, 16, 16)  # 128-site planes: whole-plane and 8-row (y, z, t) walk tiles apply
+    g = q.Gauge.random(L, seed=34, eps=0.3)
+    vh = q.half_volume(L)
+    vs = [orc.source_gauss(L, 80 + r)[1] for r in range(12)]
+    singles = [q.hop(g, v, 0, dagger=0, t_boundary=-1, recon=12, precision=prec) for v in vs]
+    bufs = [q.DeviceBuffer(vh * 192) for _ in vs]
+    ptrs = (ctypes.c_void_p * 12)(*[b.ptr for b in bufs])
+    # (block, rb, rpt, xcd, tile_z, tile_t, group_major, tile_y, rpw, spt, cached, lds)
+    shapes = [None,  # the default
+              (256, 4, 1, 1, 4, 4, 1, 0, 1, 1, 0, 0), (128, 2, 3, 1, 4, 4, 1, 8, 1, 2, 1, 0),
+              (64, 1, 2, 0, 0, 0, 1, 0, 1, 1, 0, 0), (256, 2, 1, 1, 8, 8, 0, 8, 1, 4, 1, 0),
+              (128, 1, 4, 0, 4, 4, 0, 0, 1, 1, 0, 0), (192, 3, 1, 1, 4, 4, 0, 0, 4, 1, 1, 0),
+              (64, 1, 1, 1, 0, 0, 1, 0, 4, 2, 0, 0), (128, 2, 1, 0, 4, 4, 1, 8, 2, 4, 1, 0),
+              (256, 2, 1, 1, 8, 8, 1, 0, 2, 2, 1, 0), (256, 1, 1, 1, 4, 4, 0, 8, 1, 1, 0, 1),
+              (128, 1, 1, 0, 0, 0, 0, 0, 1, 2, 1, 1), (64, 1, 1, 1, 8, 8, 0, 0, 1, 3, 0, 1),
+              (256, 1, 1, 0, 2, 4, 0, 8, 1, 1, 1, 1), (256, 1, 1, 2, 8, 16, 0, 0, 1, 1, 1, 1),
+              (128, 1, 1, 2, 0, 0, 0, 0, 1, 1, 0, 1), (256, 1, 1, 4, 8, 8, 0, 0, 1, 1, 1, 2)]
+    for sh in shapes:
+        if sh:
+            shape = dict(zip(q.SHAPE_KEYS, sh))
+            if prec == 0:
+                shape["rpt"] = 1
+            q.set_hop_shape(g, prec, 12, 12, shape)
+        for b, v in zip(bufs, vs):
+            b.upload(v)
+        q.check(q.lib().qcuHopBatch(g.handle, 12, ptrs, ptrs, 0, 0, -1, 12, prec))
+        for r in range(12):
+            assert np.array_equal(bufs[r].to_numpy((vh, 4, 3)), singles[r]), (sh, r)
+
+
+# half volumes that no other test pins a shape for: off the 64-site chunk and of whole chunks
+@pytest.mark.parametrize("L", [(10, 2, 2, 6), (6, 6, 6, 10), (12, 8, 6, 14), (8, 8, 6, 10)])
+def test_split_kernel_bits_equal_pinned_shape_every_epilogue(q, L):
+    """The leg-split kernel (the default here) against hop_kernel under a pinned shape, on
+    internal fields: Mhat, Wilson and clover, in each precision and link storage, and a
+    solve's iterations, solution and true residual.  A pin holds for the process, so every
+    default result comes before the first of them."""
+    b = orc.source_gauss(L, 5)
+    cases = [(p, r, csw) for p in (0, 1, 2) for r in (12, 18) for csw in (0.0, 1.0)]
+
+    def results():
+        out = {}
+        for prec, recon, csw in cases:
+            g = q.Gauge.random(L, seed=43, eps=0.2)
+            op = q.Operator(0.12, csw, -1, recon)
+            sp = q.default_solve_params(tol=1e-9, precision=prec, chunk=4, max_iter=200)
+            x, st = q.solve(g, op, b, sp, raise_on_error=False)
+            assert st.true_residual <= 1e-9
+            out[prec, recon, csw] = [q.apply_mhat(g, op, b[0], dagger=d, precision=prec) for d in (0, 1)] + [
+                x, np.array([st.iterations, st.true_residual])]
+            g.destroy()
+        return out
+
+    want = results()
+    g = q.Gauge.random(L, seed=43, eps=0.2)
+    for prec in (0, 1, 2):
+        for recon in (12, 18):
+            q.set_hop_shape(g, prec, recon, 1, {"block": 128, "rb": 1, "rpt": 1})
+    got = results()
+    for k in cases:
+        for i, (a, c) in enumerate(zip(want[k], got[k])):
+            assert np.array_equal(a, c), (k, i)
+
+
+def test_scalar_steps_hand_over_mid_solve(q):
+    """Eight right-hand sides of 16^3x64, checked after every iteration: with 2,048 partials
+    seven and more take their scalar steps in one-block kernels, six and fewer in the vector
+    kernels.  Source r is M^r of a Gaussian one, its low modes the weaker the higher r, so
+    the sources converge apart and the solve goes from one to the other.  Each right-hand
+    side keeps the bits and iterations of its solve alone."""
+    L = (16, 16, 16, 64)
+    chains = q.lib()["_ZN3qcu14cg_step_chainsEli"]
+    chains.argtypes, chains.restype = [ctypes.c_long, ctypes.c_int], ctypes.c_int
+    nw = q.half_volume(L) // 64
+    g = q.Gauge.random(L, seed=45, eps=0.2)
+    op = q.Operator(0.115, 0.0, -1, 12)
+    sp = q.default_solve_params(tol=1e-8, precision=1, chunk=1)
+    bs = [q.source_gaussian_device(L, 60)]
+    for r in range(7):
+        bs.append(q.DeviceBuffer(bs[0].nbytes))
+        q.check(q.lib().qcuApplyM(g.handle, ctypes.byref(op), bs[-1].ptr, bs[-2].ptr, 0))
+    vh = q.half_volume(L)
+    xs = [q.DeviceBuffer(2 * vh * 192) for _ in bs]
+    sts = q.solve_batch_device(g, op, xs, bs, sp)
+    its = [s.iterations for s in sts]
+    assert all(s.converged for s in sts)
+    left = {sum(i > t for i in its) for t in its} - {0}  # right-hand sides still active after a harvest
+    assert chains(nw, 8) == 0 and any(chains(nw, n) != 0 for n in left), (its, left)
+    xa = q.DeviceBuffer(2 * vh * 192)
+    for r in range(8):
+        sa = q.solve_batch_device(g, op, [xa], [bs[r]], sp)[0]
+        assert sa.converged and sa.iterations == its[r], (r, its)
+        assert np.array_equal(xa.to_numpy((2, vh, 4, 3)), xs[r].to_numpy((2, vh, 4, 3))), r
