@@ -143,3 +143,23 @@ def test_scalar_steps_hand_over_mid_solve(q):
         sa = q.solve_batch_device(g, op, [xa], [bs[r]], sp)[0]
         assert sa.converged and sa.iterations == its[r], (r, its)
         assert np.array_equal(xa.to_numpy((2, vh, 4, 3)), xs[r].to_numpy((2, vh, 4, 3))), r
+
+
+@pytest.mark.parametrize("L", [(24, 20, 20, 40), (20, 18, 22, 46)])
+def test_dslash_past_the_cache(q, L):
+    """dslashQcu on data beyond the 256 MB Infinity Cache takes its chunks in storage order;
+    half volumes on and off the 64-site chunk, the bits of the hop on packed links."""
+    g = q.Gauge.random(L, seed=49, eps=0.25)
+    vh = q.half_volume(L)
+    assert vh * (8 * 144 + 2 * 192) > 256 << 20
+    prm = q.param(L)
+    gd, a = q.DeviceBuffer(8 * vh * 144), q.source_gaussian_device(L, 15)
+    q.check(q.lib().qcuGaugeExport(g.handle, gd.ptr))
+    b, c = q.DeviceBuffer(vh * 192), q.DeviceBuffer(vh * 192)
+    q.lib().qcuClearLastError()
+    for parity in (0, 1):
+        src = a.ptr + (1 - parity) * vh * 192
+        q.lib().dslashQcu(b.ptr, src, gd.ptr, ctypes.byref(prm), parity)
+        assert q.lib().qcuGetLastError() == 0
+        q.check(q.lib().qcuHop(g.handle, c.ptr, src, parity, 0, 1, 12, 0))
+        assert np.array_equal(b.to_numpy((vh, 4, 3)), c.to_numpy((vh, 4, 3))), parity
