@@ -304,9 +304,20 @@ static int eighth_of_t(const Geom& geo) {
 // 52, 297 MB 83 / 107.  FP16 spends its time on unpacking and rebuilding the links, which
 // the LDS kernel does once per batch: 24^3x48 4 RHS 61 / 62, 16^3x32 6 RHS 21 / 20, 12 RHS
 // 33 / 36.
-static bool split_pays(int prec, int recon, long vh, int nrhs) {
-  const size_t bytes = gauge_bytes(prec, recon, vh) + 2 * (size_t)nrhs * spinor_bytes(prec, vh);
+//
+// A clover epilogue reads the clover once per right-hand side here, where the LDS kernel
+// stages it once: each after the second counts as bytes.  Clover solves, LDS kernel / this
+// (ms): FP64 16^3x32 4 RHS (237 MB with the clover) 29.3 / 25.3, 6 (352) 36.6 / 39.1, 16^4
+// 8 (239) 20.9 / 19.2, 16 (491) 37.1 / 42.1, 20^3x40 2 (246) 48.1 / 38.8; FP32 20^3x40 3 (200)
+// 28.0 / 27.3, 4 (276) 33.6 / 35.6, 16^3x32 6 (176) 20.9 / 18.5, 16 (491) 44.7 / 53.6.  FP16
+// up to 3 RHS (24^3x48 50.9 / 43.5), and beyond them to 80 MB: 16^4 6 (46) 10.0 / 8.6, 12 (94)
+// 13.9 / 14.6, 16^3x32 8 (124) 18.1 / 18.7, 24^3x48 4 (297) 51.2 / 56.5.
+static bool split_pays(int prec, int recon, long vh, int nrhs, int epi) {
+  const bool clover = (epi == EPI_CLOV || epi == EPI_CLOV_XPAY) && nrhs > 2;
+  const size_t bytes = gauge_bytes(prec, recon, vh) + 2 * (size_t)nrhs * spinor_bytes(prec, vh) +
+                       (clover ? (size_t)(nrhs - 2) * (clover_bytes(prec, vh) / 2) : 0);
   if (bytes > ((size_t)(nrhs > 1 ? 256 : prec == F64 && recon == 12 ? 550 : 320) << 20)) return false;
+  if (prec == F16 && clover) return nrhs <= 3 || bytes <= (size_t)80 << 20;
   return prec != F16 || nrhs <= 4 || (vh + 63) / 64 * nrhs <= 6144;
 }
 // t-slices its chunks are taken at a time (ChunkOrder): an eighth of Lt, one tile per XCD
@@ -325,16 +336,17 @@ Tune tuned_hop(int prec, int recon, long vh, int nrhs, int epi) {
   it = ctx().tune.find(tune_key(prec, recon, vh, nrhs, EPI_PLAIN));
   if (it != ctx().tune.end()) return it->second;
   Tune t;
-  t.split = split_pays(prec, recon, vh, nrhs);
+  t.split = split_pays(prec, recon, vh, nrhs, epi);
   if (nrhs > 1) {  // every right-hand side in one block per 64-site chunk, its links
     // staged in LDS once (hop_lds_kernel; on 32^3x64 with 12 right-hand sides 22-29 %
     // faster than the best shape sharing link loads within a wave), blocks round-robin over
     // the XCDs.  Four waves per block, of which FP32 and FP64 gain with two right-hand sides
     // already (32^3x64 2 RHS, two waves / four: FP32 184 / 175 us, FP64 421 / 376); FP16 two
     // while the links weigh more than the right-hand sides (2 RHS 104 / 128, 6 249 / 269, 12
-    // 474 / 472, 24^3x48 6 RHS 80 / 85).
+    // 474 / 472, 24^3x48 6 RHS 80 / 85), or with a clover up to three of them (24^3x48 clover
+    // solves of 4 RHS, two / four, 58.6 / 51.2 ms, 6 RHS 80.3 / 72.6).
     t.lds = 2;  // a clover shared by every right-hand side staged in LDS as well
-    t.block = prec == F16 && nrhs <= 6 ? 128 : 256;
+    t.block = prec == F16 && nrhs <= (epi == EPI_CLOV || epi == EPI_CLOV_XPAY ? 3 : 6) ? 128 : 256;
     // and then eight waves where four leave a CU short of them: beside the clover an LDS
     // holds one block in FP64 and two in FP32.  32^3x64 four waves / eight: FP64 A^-1 D 5 RHS
     // 1,089 / 891 us, 12 1,762 / 1,687, its M^ 12 2,183 / 2,009; FP32 A^-1 D 12 RHS 856 / 815,

@@ -227,3 +227,26 @@ def test_tuner_times_reducing_hops_as_solves_launch_them(host_hip):
     assert H.host_hip_launches(kernel(0, 1)) > 0 and H.host_hip_launches(kernel(1, 0)) > 0
     assert H.host_hip_launches(kernel(1, 1)) == 0 and H.host_hip_launches(kernel(3, 1)) == 0
     """))
+
+
+def test_clover_batches_leave_the_split_kernel_in_time(host_hip):
+    """The leg-split kernel reads the clover once per right-hand side: points on both sides
+    of where that costs more than it gains, each measured.  Without a clover, or with one
+    or two right-hand sides, the line is where it was."""
+    run(host_hip, textwrap.dedent("""
+    f = q.lib()["_ZN3qcu9tuned_hopEiilii"]
+    f.restype = None
+    def split(prec, L, n, epi):
+        t = (ctypes.c_int * 15)()      # struct Tune, returned through memory
+        f(t, ctypes.c_int(prec), ctypes.c_int(12), ctypes.c_long(q.half_volume(L)), ctypes.c_int(n), ctypes.c_int(epi))
+        return t[14] == 1
+    A, B, C, D, E, F = (16,) * 4, (16, 16, 16, 32), (20, 20, 20, 40), (24, 24, 24, 32), (24, 24, 24, 48), (8,) * 4
+    for epi in (2, 3):
+        for prec, L, n in ((0, A, 8), (0, B, 4), (0, C, 2), (1, B, 8), (1, C, 3), (1, A, 12), (1, E, 2), (2, E, 3),
+                           (2, A, 6), (2, B, 4), (0, F, 16), (1, F, 16), (2, F, 16)):
+            assert split(prec, L, n, epi), (prec, L, n)
+        for prec, L, n in ((0, A, 16), (0, B, 8), (0, B, 6), (1, B, 12), (1, B, 16), (1, C, 4), (1, C, 6), (1, D, 4),
+                           (2, E, 4), (2, D, 4), (2, A, 12), (2, B, 8)):
+            assert not split(prec, L, n, epi), (prec, L, n)
+        assert split(0, A, 16, epi - 2) and split(1, C, 6, epi - 2) and split(2, A, 12, epi - 2)
+    """))
