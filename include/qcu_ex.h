@@ -257,8 +257,9 @@ int qcuServerDestroy(qcuServer s);
  * right-hand side is staged in LDS too).
  * A tile that does not divide the lattice falls back to storage order.  A hop that also
  * sums |out|^2 (in a solve) takes one right-hand side per wave whatever the shape says.
- * Where the kernel that splits a site's legs over four waves is the fastest (it takes no
- * shape), it is kept, and shape receives the fastest of the others.  QCU_TUNE=1 makes
+ * Where the fastest launch has no such shape (the kernel that splits a site's legs over
+ * four waves, or what the default adds to a shape: more waves beside a staged clover, an
+ * order of the chunks), it is kept, and shape receives the shape without that.  QCU_TUNE=1 makes
  * solves tune on first use; QCU_TUNE_CACHE=<file> persists results across processes. */
 int qcuTuneHop(qcuGauge g, int precision, int recon, int nrhs, int* shape, double* ms);
 /* Sets the launch shape (the 12 ints above, for every epilogue) used for (precision, recon, nrhs) on this

@@ -212,9 +212,20 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
     if (t.tz && !make_walk(g.geo, t.ty, t.tz, t.tt).tile_z) continue;  // tile does not fit this lattice
     timed.push_back({time_shape(t, EPI_PLAIN), t});
   }
-  // the kernel that takes no shape, where the default rule would (no entry yet for this key)
-  ctx().tune.erase(tune_key(prec, recon, vh, nrhs, EPI_PLAIN));
-  Tune split = tuned_hop(prec, recon, vh, nrhs);
+  // what the default rule launches for each epilogue (no entries yet for these keys), in
+  // the form of a shape that can be pinned where it is one
+  Tune rule[4];
+  for (int epi = EPI_PLAIN; epi <= EPI_CLOV_XPAY; ++epi) ctx().tune.erase(tune_key(prec, recon, vh, nrhs, epi));
+  for (int epi = EPI_PLAIN; epi <= EPI_CLOV_XPAY; ++epi) {
+    Tune& t = rule[epi] = tuned_hop(prec, recon, vh, nrhs, epi);
+    if (t.tz >= 0) continue;
+    if (make_walk(g.geo, t.ty, g.geo.L[2], t.tt).tile_z) {
+      t.tz = g.geo.L[2];
+    } else {
+      t.tz = t.tt = 0;
+      t.order = 1;
+    }
+  }
   auto by_time = [](const std::pair<double, Tune>& x, const std::pair<double, Tune>& y) { return x.first < y.first; };
   std::stable_sort(timed.begin(), timed.end(), by_time);
   // ... then the fastest few walking 2 or 4 site blocks per block (sites per thread),
@@ -228,21 +239,15 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
       timed.push_back({time_shape(t, EPI_PLAIN), t});
     }
   std::stable_sort(timed.begin(), timed.end(), by_time);
-  if (split.split) {  // it carries the fastest shape that can be pinned, which callers are told
-    split = timed.front().second;
-    split.split = 1;
-    timed.push_back({time_shape(split, EPI_PLAIN), split});
-    std::stable_sort(timed.begin(), timed.end(), by_time);
-  }
-  if (nrhs > 1 && !make_walk(g.geo, 0, g.geo.L[2], 8).tile_z)  // the default's chunk order, likewise
-    for (const auto& c : timed)
-      if (c.second.lds && !c.second.split && c.second.tz == 0 && c.second.spt == 1) {
-        Tune t = c.second;
-        t.order = 1;
-        timed.push_back({time_shape(t, EPI_PLAIN), t});
-        std::stable_sort(timed.begin(), timed.end(), by_time);
-        break;
-      }
+  // the leg-split kernel carries the fastest shape that can be pinned, which callers are told
+  const Tune pinnable = timed.front().second;
+  for (Tune& t : rule)
+    if (t.split) {
+      t = pinnable;
+      t.split = 1;
+    }
+  timed.push_back({time_shape(rule[EPI_PLAIN], EPI_PLAIN), rule[EPI_PLAIN]});
+  std::stable_sort(timed.begin(), timed.end(), by_time);
   const Tune best = timed.front().second;
   const double bms = timed.front().first;
   std::string key = tune_key(prec, recon, vh, nrhs, EPI_PLAIN);
@@ -256,7 +261,7 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
   auto same = [](const Tune& x, const Tune& y) {
     return x.block == y.block && x.rb == y.rb && x.rpt == y.rpt && x.xcd == y.xcd && x.tz == y.tz &&
            x.tt == y.tt && x.gm == y.gm && x.ty == y.ty && x.rpw == y.rpw && x.spt == y.spt && x.cached == y.cached &&
-           x.lds == y.lds && x.split == y.split && x.order == y.order;
+           x.lds == y.lds && x.clw == y.clw && x.split == y.split && x.order == y.order;
   };
   auto add_shape = [&](const Tune& t) {
     for (const Tune& u : epi_shapes)
@@ -264,7 +269,7 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
     epi_shapes.push_back(t);
   };
   for (size_t k = 0; k < top; ++k) add_shape(timed[k].second);
-  if (split.split) add_shape(split);
+  for (const Tune& t : rule) add_shape(t);
   // the LDS kernel's shapes also with the clover staged in LDS (lds = 2; the clover
   // epilogues use it when every right-hand side shares one clover field)
   for (size_t k = 0; k < top; ++k)
@@ -287,7 +292,7 @@ Tune autotune_hop(GaugeField& g, int prec, int recon, int nrhs, double* best_ms)
     Tune be = best;
     double bt = 1e30;
     for (const Tune& t : epi_shapes) {
-      double ms = time_shape(t, epi);
+      const double ms = time_shape(t, epi);
       if (ms < bt) {
         bt = ms;
         be = t;

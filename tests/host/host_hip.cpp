@@ -153,8 +153,8 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, hipStream_t* 
   *st = g_stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) {
-  const std::string& k = g_names[f];
+hipError_t hipLaunchKernel(const void* f, dim3, dim3 block, void** args, size_t, hipStream_t) {
+  const std::string k = g_names[f] + "/" + std::to_string(block.x);  // with its threads per block
   g_log.push_back(k);
   double ms = 1.0;
   for (auto& c : g_cost)

@@ -250,3 +250,25 @@ def test_clover_batches_leave_the_split_kernel_in_time(host_hip):
             assert not split(prec, L, n, epi), (prec, L, n)
         assert split(0, A, 16, epi - 2) and split(1, C, 6, epi - 2) and split(2, A, 12, epi - 2)
     """))
+
+
+def test_tuner_times_the_default_too(host_hip):
+    """What the default rule would launch is among the tuner's candidates, per epilogue: here
+    eight waves beside a staged clover, which no shape that can be pinned has.  What the
+    caller is told can be pinned all the same."""
+    run(host_hip, textwrap.dedent("""
+    L = (16, 16, 16, 12)
+    VH = q.half_volume(L)
+    g = q.Gauge.random(L, seed=1, eps=0.2)
+    op = q.Operator(0.12, 1.0, -1, 12)
+    a, b = ([spinor() for _ in range(12)] for _ in range(2))
+    def finish():      # a zero source: set up and finished, with two A x + a h hops of 12
+        H.host_hip_clear_log()
+        q.solve_batch_device(g, op, a, b, q.default_solve_params(precision=0))
+        return H.host_hip_launches(b"/512")
+    assert finish() == 2
+    H.host_hip_cost(b"/512", 0.01)
+    shape, _ = q.tune_hop(g, 0, 12, 12)
+    assert finish() == 2
+    q.set_hop_shape(g, 0, 12, 12, shape)
+    """))
