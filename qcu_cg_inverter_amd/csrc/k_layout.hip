@@ -302,11 +302,9 @@ void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long
 // parity = (x+y+z+t) mod 2, the half-site order of include/qcu_point.cuh:20-93.  One
 // thread per 16-byte complex of a site record (NC complex per site), so consecutive
 // lanes move consecutive bytes of the lexicographic field; blockIdx.y picks the field.
-// The launcher guarantees vol < 2^31, the range of FastDiv.  NT: a field too large to be
-// found in the Infinity Cache by what reads it next is streamed past it: gauge and two
-// spinors of 24^3x48 254 -> 242 us for the three calls (6.1 TB/s but for the waits), 32^3x64
-// 718 -> 695.
-template <bool TO_EO, int NC, int NT>
+// The launcher guarantees vol < 2^31, the range of FastDiv.  NTL, NTS: streamed past the
+// caches, loads and stores.
+template <bool TO_EO, int NC, int NTL, int NTS>
 __global__ void lex_eo_kernel(const double2* src, double2* dst, long vol, FastDiv dlx, FastDiv dly, FastDiv dlz,
                               long field) {
   long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -320,10 +318,18 @@ __global__ void lex_eo_kernel(const double2* src, double2* dst, long vol, FastDi
   long e = (long)parity * (vol / 2) + (l >> 1);
   src += blockIdx.y * field;
   dst += blockIdx.y * field;
-  if (TO_EO) stp<NT>(dst + e * NC + k, ldp<NT>(src + (long)l * NC + k));
-  else stp<NT>(dst + (long)l * NC + k, ldp<NT>(src + e * NC + k));
+  if (TO_EO) stp<NTS>(dst + e * NC + k, ldp<NTL>(src + (long)l * NC + k));
+  else stp<NTS>(dst + (long)l * NC + k, ldp<NTL>(src + e * NC + k));
 }
 
+// A spinor of more than 128 MiB, which overflows the Infinity Cache together with its copy,
+// is streamed past it (24^3x64 there and back 139 -> 132 us).  Up to there an even-odd one
+// stays in it for what reads it next, and of those above 64 MiB the lexicographic output,
+// which the library does not read again, is streamed: there and back with a hop between
+// them, through the caches / both sides streamed / this: 24^3x32 (85 MB) 123 / 133 / 126,
+// 24^3x48 (127 MB) 163 / 179 / 169, without the hop 73 / 79 / 74 and 100 / 105 / 97.  A gauge is
+// streamed above 64 MiB: three states in turn of a gauge and two spinors, through the caches /
+// this: 16^3x32 83 / 78, 16^3x48 105 / 97, 24^3x48 254 / 246.
 void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st) {
   long vol = (long)L[0] * L[1] * L[2] * L[3];
   long n = vol * nc;
@@ -331,14 +337,16 @@ void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc
   const double2* s = static_cast<const double2*>(src);
   double2* d = static_cast<double2*>(dst);
   FastDiv dlx((uint32_t)L[0]), dly((uint32_t)L[1]), dlz((uint32_t)L[2]);
-  const bool nt = (size_t)n * nfields * 16 > kNtStoreBytes / 2;
-#define QCU_LEX(E, N)                                                                                          \
-  if (to_eo == E && nc == N) {                                                                                 \
-    if (nt) hipLaunchKernelGGL((lex_eo_kernel<E, N, 1>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n); \
-    else hipLaunchKernelGGL((lex_eo_kernel<E, N, 0>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n);    \
-    return;                                                                                                    \
+  const size_t bytes = (size_t)n * nfields * 16;
+  const bool half = bytes > kNtStoreBytes / 2;
+  const int ntl = nc == 12 ? bytes > kNtStoreBytes : half, nts = ntl || (!to_eo && half);
+#define QCU_LEX(E, N, NTL, NTS)                                                                                       \
+  if (to_eo == E && nc == N && ntl == NTL && nts == NTS) {                                                            \
+    hipLaunchKernelGGL((lex_eo_kernel<E, N, NTL, NTS>), grid, dim3(256), 0, st, s, d, vol, dlx, dly, dlz, n);         \
+    return;                                                                                                           \
   }
-  QCU_LEX(1, 12) QCU_LEX(0, 12) QCU_LEX(1, 9) QCU_LEX(0, 9)
+  QCU_LEX(1, 12, 0, 0) QCU_LEX(1, 12, 1, 1) QCU_LEX(0, 12, 0, 0) QCU_LEX(0, 12, 0, 1) QCU_LEX(0, 12, 1, 1)
+  QCU_LEX(1, 9, 0, 0) QCU_LEX(1, 9, 1, 1) QCU_LEX(0, 9, 0, 0) QCU_LEX(0, 9, 1, 1)
 #undef QCU_LEX
 }
 

@@ -163,3 +163,23 @@ def test_dslash_past_the_cache(q, L):
         assert q.lib().qcuGetLastError() == 0
         q.check(q.lib().qcuHop(g.handle, c.ptr, src, parity, 0, 1, 12, 0))
         assert np.array_equal(b.to_numpy((vh, 4, 3)), c.to_numpy((vh, 4, 3))), parity
+
+
+@pytest.mark.parametrize("L,field,n", [((24, 24, 24, 32), 0, 12), ((16, 16, 16, 32), 1, 36), ((24, 24, 24, 64), 0, 12)])
+def test_layout_round_trip_at_each_cache_policy(q, L, field, n):
+    """A spinor of 85 MB, whose lexicographic output alone is streamed, and a gauge of 75 MB and
+    a spinor of 170 MB, streamed on both sides: there and back gives the same words, and the even-odd field is the
+    one numpy makes."""
+    vol = 2 * q.half_volume(L)
+    a, b, c = (q.DeviceBuffer(vol * n * 16) for _ in range(3))
+    src = np.random.default_rng(7).standard_normal((n // (12 if field == 0 else 9), vol, 12 if field == 0 else 9, 2))
+    a.upload(src)
+    I = (ctypes.c_int * 4)(*L)
+    q.check(q.lib().qcuLexToEvenOdd(b.ptr, a.ptr, I, field))
+    q.check(q.lib().qcuEvenOddToLex(c.ptr, b.ptr, I, field))
+    assert np.array_equal(c.to_numpy((vol * n * 2,), np.float64), src.ravel())
+    t, z, y, x = np.indices(L[::-1]).reshape(4, -1)
+    par = (t + z + y + x) & 1
+    eo = b.to_numpy(src.shape, np.float64)
+    for p in (0, 1):
+        assert np.array_equal(eo[:, p * vol // 2:(p + 1) * vol // 2], src[:, par == p]), p

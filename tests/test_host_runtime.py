@@ -272,3 +272,24 @@ def test_tuner_times_the_default_too(host_hip):
     assert finish() == 2
     q.set_hop_shape(g, 0, 12, 12, shape)
     """))
+
+
+def test_layout_streams_what_is_not_read_next(host_hip):
+    """A converted spinor that overflows the Infinity Cache beside its copy is streamed past
+    it; a smaller even-odd one is left there for what reads it next."""
+    run(host_hip, textwrap.dedent("""
+    # lattice, field, complex per site, fields, (loads, stores) streamed to even-odd, and back
+    for L, field, nc, nf, there, back in (((24, 24, 24, 48), 0, 12, 1, (0, 0), (0, 1)),
+                                          ((24, 24, 24, 48), 1, 9, 4, (1, 1), (1, 1)),
+                                          ((24, 24, 24, 64), 0, 12, 1, (1, 1), (1, 1)),
+                                          ((20, 20, 20, 40), 0, 12, 1, (0, 0), (0, 0)),
+                                          ((16, 16, 16, 32), 1, 9, 4, (1, 1), (1, 1)),
+                                          ((16, 16, 16, 16), 1, 9, 4, (0, 0), (0, 0))):
+        n = 2 * q.half_volume(L) * nc * nf * 16
+        a, b = q.DeviceBuffer(n), q.DeviceBuffer(n)
+        for f, to_eo, nt in ((q.lib().qcuLexToEvenOdd, 1, there), (q.lib().qcuEvenOddToLex, 0, back)):
+            H.host_hip_clear_log()
+            q.check(f(b.ptr, a.ptr, (ctypes.c_int * 4)(*L), field))
+            assert H.host_hip_launches(b"lex_eo_kernelILb%dELi%dELi%dELi%dE" % (to_eo, nc, *nt)) == 1, (L, field, to_eo)
+        del a, b
+    """))
