@@ -171,7 +171,7 @@ void CgBatch::add_slots(const SlotSpec* specs, int m) {
   hop_v(*g_, F64, recon_, EPI_XPAY, 0, 0, (double)tbc_, at(t64_, r0), at(bh_, r0), at(shi_, r0), none, kap, m,
         nullptr, st_);
   launch_zero(F64, at(xe_, r0), vh_, m, st_);
-  launch_spinor_convert(F64, at(bh_, r0), prec_, at(S_, r0), vh_, m, 0, st_);
+  launch_spinor_convert(at(bh_, r0), prec_, at(S_, r0), vh_, m, st_);
   if (prec_ != F64) {
     launch_zero(xprec_, at(X_, r0), vh_, m, st_);
   }

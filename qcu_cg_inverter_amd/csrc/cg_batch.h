@@ -105,7 +105,7 @@ class CgBatch {
   qcuSolveParams sp_;
   hipStream_t st_;
   long vh_, nw_, fb_, pb_, xb_;
-  DevBuf f64_, slo_, xlo_, part_, scal_, tmp_, aos_;
+  DevBuf f64_, slo_, xlo_, part_, scal_, aos_;
   Vec bh_, xe_, shi_, t64_, S_, R_, P_, T_, TO_, X_;
   double *part_rr_, *part_tt_, *part_ss_;
   CgScal* dsc_;

@@ -350,40 +350,26 @@ void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc
 #undef QCU_LEX
 }
 
-template <int PI, int PO>
-__global__ void spinor_convert_kernel(Vec in, Vec out, long vh, int accumulate) {
+// FP64 field -> internal layout of another precision (or a copy)
+template <int P>
+__global__ void spinor_convert_kernel(Vec in, Vec out, long vh) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   int r = blockIdx.y;
   if (i >= vh) return;
-  using TI = typename Real<PI>::T;
-  using TO = typename Real<PO>::T;
-  cx<TI> a[12];
-  SpinorIO<PI>::load(static_cast<const char*>(in.p) + r * in.stride, vh, i, a);
-  cx<TO> b[12];
-  char* o = static_cast<char*>(out.p) + r * out.stride;
-  if (accumulate) {
-    SpinorIO<PO>::load(o, vh, i, b);
+  using T = typename Real<P>::T;
+  cx<double> a[12];
+  SpinorIO<F64>::load(static_cast<const char*>(in.p) + r * in.stride, vh, i, a);
+  cx<T> b[12];
 #pragma unroll
-    for (int c = 0; c < 12; ++c) b[c] = {b[c].re + TO(a[c].re), b[c].im + TO(a[c].im)};
-  } else {
-#pragma unroll
-    for (int c = 0; c < 12; ++c) b[c] = {TO(a[c].re), TO(a[c].im)};
-  }
-  SpinorIO<PO>::store(o, vh, i, b);
+  for (int c = 0; c < 12; ++c) b[c] = {T(a[c].re), T(a[c].im)};
+  SpinorIO<P>::store(static_cast<char*>(out.p) + r * out.stride, vh, i, b);
 }
 
-void launch_spinor_convert(int pin, Vec in, int pout, Vec out, long vh, int nrhs, int accumulate, hipStream_t st) {
-  dim3 grid(nblk(vh, 256), nrhs);
-#define QCU_SC(A, B)                                                                                       \
-  if (pin == A && pout == B) {                                                                             \
-    hipLaunchKernelGGL((spinor_convert_kernel<A, B>), grid, dim3(256), 0, st, in, out, vh, accumulate); \
-    return;                                                                                                \
-  }
-  QCU_SC(F64, F64) QCU_SC(F64, F32) QCU_SC(F64, F16)
-  QCU_SC(F32, F64) QCU_SC(F32, F32) QCU_SC(F32, F16)
-  QCU_SC(F16, F64) QCU_SC(F16, F32) QCU_SC(F16, F16)
-#undef QCU_SC
+void launch_spinor_convert(Vec in, int prec, Vec out, long vh, int nrhs, hipStream_t st) {
+  const dim3 grid(nblk(vh, 256), nrhs);
+  if (prec == F64) hipLaunchKernelGGL(spinor_convert_kernel<F64>, grid, dim3(256), 0, st, in, out, vh);
+  else if (prec == F32) hipLaunchKernelGGL(spinor_convert_kernel<F32>, grid, dim3(256), 0, st, in, out, vh);
+  else hipLaunchKernelGGL(spinor_convert_kernel<F16>, grid, dim3(256), 0, st, in, out, vh);
 }
-
 
 }  // namespace qcu

@@ -51,8 +51,8 @@ void launch_gauge_import(const void* aos, void* out, uint64_t* parts, long vh, h
 void launch_shift_storage(int kind, int to_soa, const void* src, void* dst, long vh, hipStream_t st);
 // lexicographic <-> even-odd, nc (12 or 9) complex per site, nfields fields of V sites
 void launch_lex_eo(int to_eo, const void* src, void* dst, const int L[4], int nc, int nfields, hipStream_t st);
-// out = in (accumulate = 0) or out += in (accumulate = 1), any precisions
-void launch_spinor_convert(int pin, Vec in, int pout, Vec out, long vh, int nrhs, int accumulate, hipStream_t st);
+// out, in `prec`, = in, in FP64
+void launch_spinor_convert(Vec in, int prec, Vec out, long vh, int nrhs, hipStream_t st);
 
 // ----------------------------------------------------------------- blas -----
 // per-right-hand-side CG scalars kept in device memory
