@@ -305,19 +305,27 @@ static int eighth_of_t(const Geom& geo) {
 // the LDS kernel does once per batch: 24^3x48 4 RHS 61 / 62, 16^3x32 6 RHS 21 / 20, 12 RHS
 // 33 / 36.
 //
-// A clover epilogue reads the clover once per right-hand side here, where the LDS kernel
-// stages it once: each after the second counts as bytes.  Clover solves, LDS kernel / this
-// (ms): FP64 16^3x32 4 RHS (237 MB with the clover) 29.3 / 25.3, 6 (352) 36.6 / 39.1, 16^4
-// 8 (239) 20.9 / 19.2, 16 (491) 37.1 / 42.1, 20^3x40 2 (246) 48.1 / 38.8; FP32 20^3x40 3 (200)
-// 28.0 / 27.3, 4 (276) 33.6 / 35.6, 16^3x32 6 (176) 20.9 / 18.5, 16 (491) 44.7 / 53.6.  FP16
-// up to 3 RHS (24^3x48 50.9 / 43.5), and beyond them to 80 MB: 16^4 6 (46) 10.0 / 8.6, 12 (94)
-// 13.9 / 14.6, 16^3x32 8 (124) 18.1 / 18.7, 24^3x48 4 (297) 51.2 / 56.5.
+// A clover epilogue's clover is part of a single launch's data: clover solves of one source
+// with hop_kernel / this (ms): FP32 24^3x48 (286 MB with the clover) 8.7 / 8.2, recon-18 (350)
+// 9.9 / 10.5, 24^3x56 (334) 9.6 / 10.5, 28^3x48 (455) 12.9 / 13.4; FP64 recon-12 24^3x40 (477)
+// 13.6 / 13.2, 24^3x48 (573) 15.7 / 15.8, 24^3x56 (668) 17.2 / 18.9, 24^3x64 (764) 19.5 / 20.7;
+// without a clover FP32 28^3x48 (303) 10.1 / 9.9, 24^3x64 recon-18 (339) 9.9 / 10.1, FP64
+// recon-12 26^3x56 (566) 18.0 / 17.8, 28^3x64 (809) 24.5 / 25.7.
+// In a batch the clover is read once per right-hand side here, where the LDS kernel stages it
+// once, and each after the second counts (solves, LDS kernel / this): FP64 16^3x32 4 RHS (237
+// MB with the clover) 29.3 / 25.3, 6 (352) 36.6 / 39.1, 16^4 8 (239) 20.9 / 19.2, 16 (491) 37.1
+// / 42.1, 20^3x40 2 (246) 48.1 / 38.8; FP32 20^3x40 3 (200) 28.0 / 27.3, 4 (276) 33.6 / 35.6,
+// 16^3x32 6 (176) 20.9 / 18.5, 16 (491) 44.7 / 53.6.  FP16 counts none up to 3 RHS (24^3x48 50.9
+// / 43.5, 24^3x64 19.1 / 17.8), and beyond them its line is 80 MB: 16^4 6 (46) 10.0 / 8.6, 12
+// (94) 13.9 / 14.6, 16^3x32 8 (124) 18.1 / 18.7, 24^3x48 4 (297) 51.2 / 56.5.
 static bool split_pays(int prec, int recon, long vh, int nrhs, int epi) {
-  const bool clover = (epi == EPI_CLOV || epi == EPI_CLOV_XPAY) && nrhs > 2;
+  const bool clover = epi == EPI_CLOV || epi == EPI_CLOV_XPAY;
+  const bool few16 = prec == F16 && nrhs <= 3;
+  const int counted = !clover ? 0 : nrhs == 1 ? 1 : few16 ? 0 : nrhs - 2;
   const size_t bytes = gauge_bytes(prec, recon, vh) + 2 * (size_t)nrhs * spinor_bytes(prec, vh) +
-                       (clover ? (size_t)(nrhs - 2) * (clover_bytes(prec, vh) / 2) : 0);
-  if (bytes > ((size_t)(nrhs > 1 ? 256 : prec == F64 && recon == 12 ? 550 : 320) << 20)) return false;
-  if (prec == F16 && clover) return nrhs <= 3 || bytes <= (size_t)80 << 20;
+                       (size_t)counted * (clover_bytes(prec, vh) / 2);
+  if (bytes > ((size_t)(nrhs > 1 ? 256 : prec == F64 && recon == 12 ? 550 : 300) << 20)) return false;
+  if (prec == F16 && clover) return few16 || bytes <= (size_t)80 << 20;
   return prec != F16 || nrhs <= 4 || (vh + 63) / 64 * nrhs <= 6144;
 }
 // t-slices its chunks are taken at a time (ChunkOrder): an eighth of Lt, one tile per XCD

@@ -231,8 +231,7 @@ def test_tuner_times_reducing_hops_as_solves_launch_them(host_hip):
 
 def test_clover_batches_leave_the_split_kernel_in_time(host_hip):
     """The leg-split kernel reads the clover once per right-hand side: points on both sides
-    of where that costs more than it gains, each measured.  Without a clover, or with one
-    or two right-hand sides, the line is where it was."""
+    of where that costs more than it gains, each measured."""
     run(host_hip, textwrap.dedent("""
     f = q.lib()["_ZN3qcu9tuned_hopEiilii"]
     f.restype = None
@@ -292,4 +291,27 @@ def test_layout_streams_what_is_not_read_next(host_hip):
             q.check(f(b.ptr, a.ptr, (ctypes.c_int * 4)(*L), field))
             assert H.host_hip_launches(b"lex_eo_kernelILb%dELi%dELi%dELi%dE" % (to_eo, nc, *nt)) == 1, (L, field, to_eo)
         del a, b
+    """))
+
+
+def test_clover_counts_in_a_single_launch(host_hip):
+    """One right-hand side: the clover a launch reads counts like its links and spinors, on
+    both sides of the line by measured points; without one the line is at 300 MiB (550 for
+    FP64 recon-12)."""
+    run(host_hip, textwrap.dedent("""
+    f = q.lib()["_ZN3qcu9tuned_hopEiilii"]
+    f.restype = None
+    def split(prec, recon, L, epi):
+        t = (ctypes.c_int * 15)()
+        f(t, ctypes.c_int(prec), ctypes.c_int(recon), ctypes.c_long(q.half_volume(L)), ctypes.c_int(1), ctypes.c_int(epi))
+        return t[14] == 1
+    T = lambda t: (24, 24, 24, t)
+    for epi in (2, 3):
+        for prec, recon, L in ((0, 12, T(40)), (0, 12, T(48)), (1, 12, T(48)), (1, 18, T(40)), (2, 18, T(64))):
+            assert split(prec, recon, L, epi), (prec, recon, L)
+        for prec, recon, L in ((0, 12, T(56)), (0, 12, T(64)), (1, 12, T(56)), (1, 12, T(64)), (1, 18, T(48)),
+                               (1, 18, T(56)), (2, 18, (28, 28, 28, 64))):
+            assert not split(prec, recon, L, epi), (prec, recon, L)
+            assert prec == 0 and L == T(64) or split(prec, recon, L, epi - 2), (prec, recon, L)
+    assert split(0, 12, T(64), 0) and not split(1, 18, T(64), 0) and not split(0, 12, (28, 28, 28, 64), 0)
     """))
