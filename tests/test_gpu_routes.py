@@ -145,13 +145,13 @@ def test_scalar_steps_hand_over_mid_solve(q):
         assert np.array_equal(xa.to_numpy((2, vh, 4, 3)), xs[r].to_numpy((2, vh, 4, 3))), r
 
 
-@pytest.mark.parametrize("L", [(24, 20, 20, 40), (20, 18, 22, 46)])
+@pytest.mark.parametrize("L", [(24, 24, 24, 36), (22, 22, 26, 38)])
 def test_dslash_past_the_cache(q, L):
-    """dslashQcu on data beyond the 256 MB Infinity Cache takes its chunks in storage order;
-    half volumes on and off the 64-site chunk, the bits of the hop on packed links."""
+    """dslashQcu on data well beyond the 256 MB Infinity Cache takes its chunks in storage
+    order; half volumes on and off the 64-site chunk, the bits of the hop on packed links."""
     g = q.Gauge.random(L, seed=49, eps=0.25)
     vh = q.half_volume(L)
-    assert vh * (8 * 144 + 2 * 192) > 256 << 20
+    assert vh * (8 * 144 + 2 * 192) > 340 << 20
     prm = q.param(L)
     gd, a = q.DeviceBuffer(8 * vh * 144), q.source_gaussian_device(L, 15)
     q.check(q.lib().qcuGaugeExport(g.handle, gd.ptr))
