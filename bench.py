@@ -60,9 +60,10 @@ def compulsory_bytes(prec, recon, nrhs=1):
     return 8 * LINK_BYTES[(prec, recon)] + nrhs * 2 * SPINOR_BYTES[prec]
 
 
-# sources that fix the hop kernel's code: a PMC traffic figure measured on other
-# sources is stale and is not reported
-HOP_SOURCES = ("k_hop.inc", "k_hop.hip", "qcu_fields.h", "qcu_common.h", "qcu_kernels.h")
+# sources that fix the hop kernels' code and which of them a launch takes (api.cpp): a PMC
+# traffic figure measured on other sources is stale and is not reported
+HOP_SOURCES = ("k_hop.inc", "k_hop.hip", "k_hop_split.inc", "k_hop_split_f64.hip", "qcu_fields.h", "qcu_common.h",
+               "qcu_kernels.h", "api.cpp")
 
 
 def hop_source_hash():
@@ -401,8 +402,8 @@ def config4_section(q):
 def dropin_section(q, g=None):
     """The reference's entry points as a caller sees them, on the 16^3x32 gauge of the
     headline: host-synchronous dslashQcu (one parity, s = +1, periodic, kappa = 1) and
-    fullDslashQcu (A - D with kappa = c_sw = 1, even-first full spinors), each call
-    including the interface <-> internal layout conversions."""
+    fullDslashQcu (A - D with kappa = c_sw = 1, even-first full spinors, with the check of
+    the caller's gauge), one kernel each on the caller's buffers, launch and wait included."""
     import ctypes
 
     import numpy as np
@@ -433,8 +434,8 @@ def dropin_section(q, g=None):
         res[name] = {"us_per_call": round(us, 2), "calls": n}
         log(f"drop-in {name} 16^3x32: {us:.1f} us per call")
     q.check(q.lib().qcuGetLastError())
-    res["note"] = ("host-synchronous calls through the drop-in symbols, including the layout conversions; "
-                   "the hop kernel alone is roofline.avg_launch_us")
+    res["note"] = ("host-synchronous calls through the drop-in symbols on the caller's buffers, launch and wait "
+                   "included; the hop on internal fields alone is roofline.avg_launch_us")
     del np
     return res
 
@@ -681,7 +682,7 @@ def main():
     out["config"] = {"workload": "even-odd Wilson hop D_eo/D_oe, FP64, 18-real links, 16^3x32, antiperiodic t",
                      "lattice": list(L_MAIN), "half_volume": vh, "bytes_per_site": 2880,
                      "flop_per_site": 1320}
-    out["roofline"] = roofline("hop_kernel<F64,18,EPI_PLAIN> 16^3x32", "f64", 18, vh, ms_event, "hop_f64_r18_16x32")
+    out["roofline"] = roofline("hop_split_kernel<F64,18,EPI_PLAIN> 16^3x32", "f64", 18, vh, ms_event, "hop_f64_r18_16x32")
     log(f"hop f64 r18 16^3x32: {ms_event*1e3:.2f} us/launch, {achieved:.0f} GB/s algorithmic, "
         f"{out['roofline']['achieved']:.0f} GB/s compulsory")
     # the same hop as the median of 100 windows of 20 back-to-back launches, each

@@ -124,9 +124,9 @@ int qcuHopBatch(qcuGauge g, int nrhs, void* const* out, const void* const* in, i
                 int t_boundary, int recon, int precision);
 /* qcuHop without device allocation.  No counterpart in the reference: it is for callers
  * that cannot allocate device memory (code under hipGraph capture, tight serving loops,
- * harnesses that forbid hipMalloc).  The same kernels and result as qcuHop, bit for
- * bit, with the two internal staging fields in a static device array of 32 MiB that
- * each device the library runs on holds until the process ends: a half volume whose two
+ * harnesses that forbid hipMalloc).  The result of qcuHop, bit for bit, through two
+ * internal staging fields in a static device array of 32 MiB that each device the
+ * library runs on holds until the process ends: a half volume whose two
  * fields of `precision` exceed it (FP64 above 87,360 half sites; 16^3x32 fits) is
  * rejected with QCU_ERROR_INVALID_VALUE.  It allocates nothing itself, so the gauge's
  * packed links of this precision and recon must exist already (one qcuHop, qcuHopBatch

@@ -1,4 +1,4 @@
-// k_hop_split_f16.hip -- FP16 hops on interface fields (k_hop_split.inc).
+// k_hop_split_f16.hip -- FP16 leg-split hops, on interface and internal fields (k_hop_split.inc).
 #include "k_hop_split.inc"
 
 namespace qcu {

@@ -1,4 +1,4 @@
-// k_hop_split_f32.hip -- FP32 hops on interface fields (k_hop_split.inc).
+// k_hop_split_f32.hip -- FP32 leg-split hops, on interface and internal fields (k_hop_split.inc).
 #include "k_hop_split.inc"
 
 namespace qcu {

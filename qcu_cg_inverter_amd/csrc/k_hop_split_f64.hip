@@ -1,4 +1,5 @@
-// k_hop_split_f64.hip -- FP64 hops on interface fields (k_hop_split.inc).
+// k_hop_split_f64.hip -- FP64 leg-split hops, on interface and internal fields, and dslashQcu
+// (k_hop_split.inc).
 #include "k_hop_split.inc"
 
 namespace qcu {

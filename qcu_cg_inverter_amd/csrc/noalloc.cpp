@@ -1,19 +1,19 @@
 // noalloc.cpp -- qcuHopNoAlloc: qcuHop for callers that cannot allocate device memory
 // (code under hipGraph capture, tight serving loops, harnesses that forbid hipMalloc).
 //
-// qcuHop stages the caller's interface spinor in the internal layout of the requested
-// precision, runs the hop into a second internal field and converts that back; its two
-// staging fields are library allocations that grow on demand.  Here the two fields
-// live in one file-scope device array, `scratch`, of kNoAllocScratchBytes, which every
-// device the library runs on holds until the process ends.  Host code never passes the
-// array's name to a kernel (on the host it is only a stand-in for the symbol): the
-// library's init call looks up the device address once per device with
-// hipGetSymbolAddress, and the launches take that address.
+// qcuHop runs on the caller's buffers and stages nothing unless they overlap.  This entry
+// point converts the caller's interface spinor to the internal layout of the requested
+// precision, runs the hop into a second internal field and converts that back, so that in
+// and out may overlap and a pinned launch shape applies.  The two fields live in one
+// file-scope device array, `scratch`, of kNoAllocScratchBytes, which every device the
+// library runs on holds until the process ends.  Host code never passes the array's name
+// to a kernel (on the host it is only a stand-in for the symbol): the library's init call
+// looks up the device address once per device with hipGetSymbolAddress, and the launches
+// take that address.
 //
-// The kernels of qcuHop run unchanged, so the result is the same bit for bit.  Nothing
-// in the array has to start at zero: the conversion writes every site of the staged
-// input and the hop every site of its output before either is read.  Calls that
-// overlap on one device race on the array.
+// The result is qcuHop's, bit for bit.  Nothing in the array has to start at zero: the
+// conversion writes every site of the staged input and the hop every site of its output
+// before either is read.  Calls that overlap on one device race on the array.
 #include <cstring>
 
 #include "qcu_host.h"
