@@ -59,9 +59,12 @@ CgBatch::CgBatch(GaugeField& g, int prec, int recon, int t_boundary, bool clover
   part_ss_ = pp + 2 * nw_ * cap_;
   scal_.alloc(sizeof(CgScal) * cap_);
   dsc_ = static_cast<CgScal*>(scal_.p);
-  QHIP(hipHostMalloc((void**)&hsc_, sizeof(CgScal) * cap_, 0));
-  QHIP(hipHostMalloc((void**)&hsum_, sizeof(double) * 3 * cap_, 0));
   rebind(g);
+  // last: a constructor that throws has no destructor to free them
+  QHIP(hipHostMalloc((void**)&hsc_, sizeof(CgScal) * cap_, 0));
+  const hipError_t e2 = hipHostMalloc((void**)&hsum_, sizeof(double) * 3 * cap_, 0);
+  if (e2 != hipSuccess) (void)hipHostFree(hsc_);
+  QHIP(e2);
   const char* e = getenv("QCU_DEBUG");
   debug_ = e && e[0] && e[0] != '0';
 }

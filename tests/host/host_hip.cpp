@@ -33,6 +33,7 @@ std::string g_wrong;
 hipError_t g_last = hipSuccess;
 long g_until_fail = -1;  // allocations until the one that fails, -1: none does
 size_t g_live = 0;
+long g_pinned = 0;
 double g_clock = 0.0;
 dim3 g_grid, g_block;
 size_t g_shmem;
@@ -107,6 +108,7 @@ long host_hip_fail_after(long n) {
   return left;
 }
 size_t host_hip_live() { return g_live; }
+long host_hip_pinned() { return g_pinned; }  // live pinned allocations
 void host_hip_clear_log() {
   g_log.clear();
   g_wrong.clear();
@@ -187,9 +189,11 @@ hipError_t hipFree(void* p) {
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   *p = calloc(1, n);
+  ++g_pinned;
   return hipSuccess;
 }
 hipError_t hipHostFree(void* p) {
+  if (p) --g_pinned;
   free(p);
   return hipSuccess;
 }

@@ -315,3 +315,18 @@ def test_clover_counts_in_a_single_launch(host_hip):
             assert prec == 0 and L == T(64) or split(prec, recon, L, epi - 2), (prec, recon, L)
     assert split(0, 12, T(64), 0) and not split(1, 18, T(64), 0) and not split(0, 12, (28, 28, 28, 64), 0)
     """))
+
+
+def test_failed_solves_leave_no_pinned_memory(host_hip):
+    """Whichever device allocation of a first solve fails, the scalars it pins are freed."""
+    run(host_hip, CALLS + textwrap.dedent("""
+    for k in range(100):
+        g = q.Gauge.random(L, seed=1, eps=0.2)
+        H.host_hip_fail_after(k)
+        rc = call(g, "solve1")
+        if H.host_hip_fail_after(-1) >= 0: break
+        assert rc == 3, (k, rc)
+        g.destroy()
+        assert H.host_hip_pinned() == 0, (k, H.host_hip_pinned())
+    assert k > 6, k
+    """))
